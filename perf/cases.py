@@ -314,9 +314,9 @@ def tolerance(case):
     (up to 3e-3 over long sequences)."""
     kind, bf16 = case["kind"], case["dtype"] == "bf16"
     if kind == "block" or (kind == "module" and case["train"]):
-        return {"rel": 3e-2 if bf16 else 1e-2, "max": 1.0}
+        return {"rel": 3e-2 if bf16 else 1e-2, "max": 0.99}
     if kind == "p1" and case["op"] == "relu":
-        return {"rel": 1e-2, "max": 1.0}
+        return {"rel": 1e-2, "max": 0.99}
     if bf16:  # each output and gradient is rounded to 8 bits once: 1.6e-3 - 2.3e-3
         return {"rel": 1e-2}
     if kind == "decode":  # sums over the width, then a step: 1.2e-7 - 5e-7
