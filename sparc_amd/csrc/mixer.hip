@@ -65,8 +65,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 #define SPARC_MIXER_FWD_S 8
 #endif
 constexpr int kS = SPARC_MIXER_FWD_S;  // steps per prefetched block of the forward scan
-constexpr int kCtrlRows = 16;  // rows per workgroup of the controls forward
-constexpr int kCtrlBwdRows = 128;  // rows per workgroup of the controls backward
+constexpr int kCtrlBwdRows = 128;  // most rows per workgroup of the controls backward
 constexpr int kMaxRowBlocks = 65535;  // grid.y limit: more row blocks loop in the workgroups
 // bf16 x: the write is rounded to bf16 before the scan, as the reference
 // stores it in x's dtype (write_r.to(x.dtype), sparc-kernal/forward/
@@ -258,8 +257,11 @@ mixer_prepare_kernel(int M, const float* nu_log, const float* theta_log, const f
 // A workgroup of NW waves takes kCtrlRows rows; each thread 8 consecutive
 // inputs per pass, the direction values it loads serving every row of the
 // workgroup.  One wave for rows of up to 1024 inputs (no idle waves in the
-// reduction), four above.
-template <typename IO, int NW>
+// reduction), four above.  Bound by its reads of x as long as enough
+// workgroups are in flight (7.0 TB/s with 2048 workgroups of 16 rows: B=8,
+// T=4096, width 32768); launch_ctrl_fwd takes fewer rows per workgroup when
+// there are few rows.
+template <typename IO, int NW, int kCtrlRows>
 __global__ void __launch_bounds__(NW * 64)
 ctrl_fwd_kernel(int64_t R, int W, const void* x, const float* pdir, const float* rdir,
                 float* eta, float* delta) {
@@ -295,11 +297,11 @@ ctrl_fwd_kernel(int64_t R, int W, const void* x, const float* pdir, const float*
     }
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  static_assert(2 * kCtrlRows == 32, "two sums per leader lane below");
-  wave_sums_to_leaders<2 * kCtrlRows>(acc);  // lanes 4k: the sums of values 2k, 2k + 1
-  if (lane % 4 == 0) {
-    red[wave][lane / 2] = acc[0];
-    red[wave][lane / 2 + 1] = acc[1];
+  constexpr int N = 2 * kCtrlRows, K = N >= 16 ? N / 16 : 1, G = 64 * K / N;
+  wave_sums_to_leaders<N>(acc);  // lanes l % G == 0: the sums of values l / G * K ...
+  if (lane % G == 0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) red[wave][lane / G * K + k] = acc[k];
   }
   __syncthreads();
   if (threadIdx.x < kCtrlRows) {
@@ -314,14 +316,27 @@ ctrl_fwd_kernel(int64_t R, int W, const void* x, const float* pdir, const float*
   }
 }
 
+template <typename IO, int ROWS>
+void launch_ctrl_fwd_rows(hipStream_t st, int64_t R, int W, const void* x, const float* pdir, const float* rdir,
+                          float* eta, float* delta) {
+  const dim3 g(static_cast<unsigned>((R + ROWS - 1) / ROWS));
+  if (W <= 1024)
+    hipLaunchKernelGGL((ctrl_fwd_kernel<IO, 1, ROWS>), g, dim3(64), 0, st, R, W, x, pdir, rdir, eta, delta);
+  else
+    hipLaunchKernelGGL((ctrl_fwd_kernel<IO, 4, ROWS>), g, dim3(256), 0, st, R, W, x, pdir, rdir, eta, delta);
+}
+// 16 rows per workgroup where that leaves at least kCtrlFwdGroups workgroups
+// (four per CU, one wave per SIMD and workgroup), else 8 or 4: with few rows
+// 16 each left most CUs without work (232 workgroups at 3711 rows of 24576
+// bf16: 98 us, 1.9 TB/s; the no-gradient module forward there 372 -> 310 us
+// with 4 rows each).
+constexpr int64_t kCtrlFwdGroups = 1024;
 template <typename IO>
 void launch_ctrl_fwd(hipStream_t st, int64_t R, int W, const void* x, const float* pdir, const float* rdir,
                      float* eta, float* delta) {
-  const dim3 g(static_cast<unsigned>((R + kCtrlRows - 1) / kCtrlRows));
-  if (W <= 1024)
-    hipLaunchKernelGGL((ctrl_fwd_kernel<IO, 1>), g, dim3(64), 0, st, R, W, x, pdir, rdir, eta, delta);
-  else
-    hipLaunchKernelGGL((ctrl_fwd_kernel<IO, 4>), g, dim3(256), 0, st, R, W, x, pdir, rdir, eta, delta);
+  if (R >= 16 * kCtrlFwdGroups) launch_ctrl_fwd_rows<IO, 16>(st, R, W, x, pdir, rdir, eta, delta);
+  else if (R >= 8 * kCtrlFwdGroups) launch_ctrl_fwd_rows<IO, 8>(st, R, W, x, pdir, rdir, eta, delta);
+  else launch_ctrl_fwd_rows<IO, 4>(st, R, W, x, pdir, rdir, eta, delta);
 }
 
 // ---------------------------------------------------------------------------
@@ -1935,6 +1950,31 @@ void choose_segments(int64_t B, int64_t T, int n_mb, int& n_seg, int& t_seg) {
   t_seg = static_cast<int>(len);
 }
 
+// The controls backward over rows of width W: n_cb column blocks of 2048
+// inputs, row blocks of `rows` rows (a multiple of 4 in [4, 128], chosen so
+// that the grid has about 1024 workgroups), and the partial direction
+// gradients pd [2][n_rb][W] and bias partials pbias [2][n_rb] in the workspace.
+struct ControlsLayout {
+  int n_cb = 0, n_rb = 0, rows = 0;
+  size_t pbias = 0, total = 0;
+};
+
+// (At 512 rows of 2048 fp32, row blocks of 128 left 4 workgroups, each a
+// serial chain of 32 four-row groups: 102 us; with blocks of 4 rows the
+// module's training step there takes 229 us against 306.)
+ControlsLayout controls_layout(int64_t R, int64_t W) {
+  ControlsLayout c;
+  c.n_cb = static_cast<int>((W + 2047) / 2048);
+  int64_t rows = (R * c.n_cb + 1023) / 1024;
+  rows = (rows + 3) / 4 * 4;
+  c.rows = static_cast<int>(rows < 4 ? 4 : (rows > kCtrlBwdRows ? kCtrlBwdRows : rows));
+  c.n_rb = static_cast<int>(std::min<int64_t>((R + c.rows - 1) / c.rows, kMaxRowBlocks));
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  c.pbias = up(static_cast<size_t>(2) * c.n_rb * W * 4);
+  c.total = c.pbias + up(static_cast<size_t>(2) * (c.n_rb > 0 ? c.n_rb : 1) * 4);
+  return c;
+}
+
 // The module backward without time segments runs in time pieces: the
 // controls backward of piece p then runs on a second stream while the mixer
 // backward works on piece p - 1.  The most pieces, up to kPieces, whose
@@ -1949,7 +1989,7 @@ constexpr int kPieces = SPARC_MIXER_BWD_PIECES;
 
 struct Layout {
   bool piped = false;
-  int V = 1, n_mb = 0, n_rb = 0, n_rb_piece = 0, n_seg = 1, t_seg = 1;
+  int V = 1, n_mb = 0, n_rb = 0, rb_rows = 0, n_rb_piece = 0, n_seg = 1, t_seg = 1;
   int64_t R = 0;
   size_t consts = 0, part_tok = 0, tok = 0, part_mode = 0, pd = 0, pbias = 0, seg_sum = 0, seg_state = 0, total = 0;
 };
@@ -1962,13 +2002,16 @@ Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, b
   l.n_mb = static_cast<int>((M + 64 * l.V - 1) / (64 * l.V));
   choose_segments(B, T, l.n_mb, l.n_seg, l.t_seg);
   l.R = B * T;
-  l.n_rb = static_cast<int>(std::min<int64_t>((l.R + kCtrlBwdRows - 1) / kCtrlBwdRows, kMaxRowBlocks));
+  const ControlsLayout cl = controls_layout(l.R, 2 * M);
+  l.n_rb = cl.n_rb;
+  l.rb_rows = cl.rows;
   int np = kPieces;
   while (np > 1 && T % (static_cast<int64_t>(np) * kCtrlBwdRows) != 0) np /= 2;
   if (pieces && np > 1 && T > 0 && direction == 1 && !gw && l.n_seg == 1 && l.V == 1) {
     l.piped = true;
     l.n_seg = np;
     l.t_seg = static_cast<int>(T / np);
+    l.rb_rows = kCtrlBwdRows;
     l.n_rb_piece = static_cast<int>(std::min<int64_t>(B * l.t_seg / kCtrlBwdRows, kMaxRowBlocks));
     l.n_rb = np * l.n_rb_piece;
   }
@@ -2405,28 +2448,6 @@ sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const
 
 }  // namespace sparc
 
-// The controls backward over rows of width W: n_cb column blocks of 2048
-// inputs, row blocks of `rows` rows (a multiple of 4 in [16, 128], chosen so
-// that the grid has about 1024 workgroups), and the partial direction
-// gradients pd [2][n_rb][W] and bias partials pbias [2][n_rb] in the workspace.
-struct ControlsLayout {
-  int n_cb = 0, n_rb = 0, rows = 0;
-  size_t pbias = 0, total = 0;
-};
-
-ControlsLayout controls_layout(int64_t R, int64_t W) {
-  ControlsLayout c;
-  c.n_cb = static_cast<int>((W + 2047) / 2048);
-  int64_t rows = (R * c.n_cb + 1023) / 1024;
-  rows = (rows + 3) / 4 * 4;
-  c.rows = static_cast<int>(rows < 16 ? 16 : (rows > kCtrlBwdRows ? kCtrlBwdRows : rows));
-  c.n_rb = static_cast<int>(std::min<int64_t>((R + c.rows - 1) / c.rows, kMaxRowBlocks));
-  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-  c.pbias = up(static_cast<size_t>(2) * c.n_rb * W * 4);
-  c.total = c.pbias + up(static_cast<size_t>(2) * (c.n_rb > 0 ? c.n_rb : 1) * 4);
-  return c;
-}
-
 sparc_status check_controls(int64_t rows, int64_t width, int32_t io_dtype) {
   if (io_dtype != SPARC_BF16 && io_dtype != SPARC_F32) return fail(SPARC_EINVAL, "controls: io_dtype must be bf16 or f32");
   if (rows < 0 || rows > (int64_t(1) << 40)) return fail(SPARC_EINVAL, "controls: rows out of range");
@@ -2578,11 +2599,11 @@ sparc_status piped_backward(const Layout& l, int64_t batch, int64_t length, int6
     const int64_t t0 = static_cast<int64_t>(p) * L;
     const int rb0 = p * l.n_rb_piece;
     if (io_dtype == SPARC_BF16)
-      hipLaunchKernelGGL(ctrl_bwd_kernel<sparc::bf16>, gb, dim3(256), 0, cs, rows_p, W, kCtrlBwdRows, x,
+      hipLaunchKernelGGL(ctrl_bwd_kernel<sparc::bf16>, gb, dim3(256), 0, cs, rows_p, W, l.rb_rows, x,
                          phase_direction, radial_direction, eta, delta, de, dd, dx, pd, pbias, length, t0, L, rb0,
                          l.n_rb);
     else
-      hipLaunchKernelGGL(ctrl_bwd_kernel<float>, gb, dim3(256), 0, cs, rows_p, W, kCtrlBwdRows, x,
+      hipLaunchKernelGGL(ctrl_bwd_kernel<float>, gb, dim3(256), 0, cs, rows_p, W, l.rb_rows, x,
                          phase_direction, radial_direction, eta, delta, de, dd, dx, pd, pbias, length, t0, L, rb0,
                          l.n_rb);
     if (hipError_t le = hipGetLastError()) {
@@ -2916,10 +2937,10 @@ sparc_status sparc_mixer_backward(int64_t batch, int64_t length, int64_t modes, 
   float* pbias = reinterpret_cast<float*>(ws + l.pbias);
   const dim3 gb(static_cast<unsigned>((W + 2047) / 2048), static_cast<unsigned>(l.n_rb));
   if (io_dtype == SPARC_BF16)
-    hipLaunchKernelGGL(ctrl_bwd_kernel<sparc::bf16>, gb, dim3(256), 0, st, l.R, W, kCtrlBwdRows, x, phase_direction,
+    hipLaunchKernelGGL(ctrl_bwd_kernel<sparc::bf16>, gb, dim3(256), 0, st, l.R, W, l.rb_rows, x, phase_direction,
                        radial_direction, eta, delta, deta, ddelta, dx, pd, pbias, l.R, int64_t(0), l.R, 0, l.n_rb);
   else
-    hipLaunchKernelGGL(ctrl_bwd_kernel<float>, gb, dim3(256), 0, st, l.R, W, kCtrlBwdRows, x, phase_direction,
+    hipLaunchKernelGGL(ctrl_bwd_kernel<float>, gb, dim3(256), 0, st, l.R, W, l.rb_rows, x, phase_direction,
                        radial_direction, eta, delta, deta, ddelta, dx, pd, pbias, l.R, int64_t(0), l.R, 0, l.n_rb);
   // direction gradients: columns 0..W-1 from the row-block partials, the bias from pbias
   if (sparc_status s = direction_sums(l.n_rb, W, pd, pbias, dphase_direction, dradial_direction, stream)) return s;
