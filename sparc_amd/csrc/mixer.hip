@@ -92,6 +92,7 @@ template <typename IO> constexpr bool kRoundWrite = SPARC_MIXER_ROUND_WRITE && s
 //            mixer_bwd_kernel.
 enum : int { kModule = 0, kPlanes = 1, kRelu = 2, kReset = 4, kCoop = 8 };
 constexpr int kStateChunk = 64;  // steps per saved chunk state (sparc_scan_chunk_length)
+constexpr int kSplitWaves = 16;  // most waves per workgroup of the split-chain kernels
 // A lane byte offset past every buffer resource of these kernels (each spans
 // less than 2^31 bytes): the hardware range check drops a store through it.
 // Lanes that must not store (past M) store through it, so that no store
@@ -997,6 +998,234 @@ mixer_fwd_wide_kernel(Args a) {
       a.last_im[static_cast<int64_t>(b) * a.M + m0 + v] = hi[v];
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// forward over split chains: the waves of a workgroup share a chain's time
+// ---------------------------------------------------------------------------
+// A chain is a batch row and 64 V modes; its workgroup of NW waves walks T in
+// rounds of NW * S steps, wave w taking steps [w S, (w + 1) S) of a round.
+// Each wave forms its steps' transitions and writes once, keeps them in
+// registers, and reduces them to its map h -> P h + Q from a zero state; the
+// maps meet in LDS (one barrier per round, double-buffered), each wave
+// composes those before its own onto the state that the last wave left after
+// the round before, and replays its steps from there.  So the time axis is
+// parallel over NW waves at 8 FMAs per mode-step for the map and 4 NW / (2 S)
+// for the composition, where time segments pay for a second pass over the
+// transitions, the writes and their loads.  A wave's next rows are loaded
+// right after its current ones are used, and have its map, the barrier, the
+// replay and the other waves to arrive in.
+template <typename IO, int V, int S, int MODE>
+__global__ void __launch_bounds__(64 * kSplitWaves)
+mixer_fwd_split_kernel(Args a) {
+  using RawT = typename Raw<IO, V>::T;
+  constexpr int ESZ = sizeof(IO);
+  constexpr int MB = 64 * V;
+  constexpr int CM = MODE & 3;             // the chain mode without kReset
+  constexpr bool RST = (MODE & kReset) != 0;
+  constexpr bool GW = CM != kModule;       // the writes are given
+  static_assert(kStateChunk % S == 0, "blocks must tile the saved-state chunks");
+  static_assert(GW || !RST, "resets in the P1 scan only");
+  // [2][NW - 1][V][64] maps (Pr, Pi, Qr, Qi) of the waves but the last, then
+  // [2][V][64] float2 states
+  extern __shared__ float4 split_lds[];
+  const int NW = static_cast<int>(blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  float2* states = reinterpret_cast<float2*>(split_lds + 2 * (NW - 1) * V * 64);
+  const ChainPos cp = chain_pos(a);
+  const int b = cp.b, mb = cp.mb, T = a.T;
+  const int m0 = mb * MB + lane * V;
+  const bool lane_ok = m0 < a.M;  // the host requires M % V == 0
+  ModeConsts<V, false> mc;
+  mc.load(a.consts, m0, lane_ok);
+  const int64_t row0 = static_cast<int64_t>(b) * T;
+  const int64_t mbase = static_cast<int64_t>(mb) * MB;
+  const int64_t W = 2 * static_cast<int64_t>(a.M);
+  const uint32_t lane_bytes = static_cast<uint32_t>(lane * V * ESZ);
+  const uint32_t lane_ld = lane_ok ? lane_bytes : 0u;
+  const uint32_t lane_st = lane_ok ? lane_bytes : kDropOffset;
+  // bytes of one row of x / y (2M) and of h / w (M) (< 2^31: the host limits M to 2^24)
+  const uint32_t row_x = static_cast<uint32_t>(W * ESZ), half_x = static_cast<uint32_t>(a.M * ESZ);
+  if (wave == 0) {  // the state before step 0: the caller's (the P1 scan) or zero
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const bool h0 = GW && lane_ok && a.h0_re != nullptr;
+      states[v * 64 + lane] = make_float2(h0 ? a.h0_re[static_cast<int64_t>(b) * a.M + m0 + v] : 0.0f,
+                                          h0 ? a.h0_im[static_cast<int64_t>(b) * a.M + m0 + v] : 0.0f);
+    }
+  }
+  wait_vm_all();  // the loop-carried constants, before the first prefetch
+
+  RawT xr[S], xi[S];
+  float ev, dv;  // lane s < S: eta, delta of step s
+  int kv;        // RST: lane s < S: whether step s keeps its transition
+  // the rows from t0; rows past T re-read row T-1 (no loads under a branch)
+  auto load_rows = [&](int t0) __attribute__((always_inline)) {
+    const int tb = min(t0, T - 1);
+    if constexpr (GW) {
+      const int64_t off = wave_uniform(((row0 + tb) * a.M + mbase) * ESZ);
+      const __amdgpu_buffer_rsrc_t rwr = make_rsrc(static_cast<const char*>(a.w_re) + off, S * half_x);
+      const __amdgpu_buffer_rsrc_t rwi = make_rsrc(static_cast<const char*>(a.w_im) + off, S * half_x);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const uint32_t o = static_cast<uint32_t>(min(t0 + s, T - 1) - tb) * half_x;
+        xr[s] = buf_load<RawT, CPOL_NT>(rwr, lane_ld, o);
+        xi[s] = buf_load<RawT, CPOL_NT>(rwi, lane_ld, o);
+      }
+    } else {
+      const int64_t off = wave_uniform(((row0 + tb) * W + mbase) * ESZ);
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char*>(a.x) + off, S * row_x);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const uint32_t o = static_cast<uint32_t>(min(t0 + s, T - 1) - tb) * row_x;
+        xr[s] = buf_load<RawT, CPOL_NT>(rx, lane_ld, o);
+        xi[s] = buf_load<RawT, CPOL_NT>(rx, lane_ld, o + half_x);
+      }
+    }
+    const int tl = min(t0 + (lane & (S - 1)), T - 1);
+    ev = a.eta[row0 + tl];
+    dv = a.delta[row0 + tl];
+    if constexpr (RST) kv = p1_keep(a, b, tl);
+  };
+
+  float hr[V], hi[V];
+  // one round; TAIL: the round that holds T, with steps past T (no update, no
+  // store) and waves past T (the identity map)
+  auto round = [&](int k, auto tail_tag) __attribute__((always_inline)) {
+    constexpr bool TAIL = decltype(tail_tag)::value;
+    const int t0 = (k * NW + wave) * S;
+    float ar[S][V], ai[S][V], wr[S][V], wi[S][V];
+    {
+      const float ee = fast_exp(ev);  // lane s: e^eta of step s
+      float Es[S], Ds[S], Rs[S];
+      p1_block_steps<S>(ee, dv, Es, Ds, Rs);
+      if constexpr (GW) {
+        float em[S][V];
+        p1_block_transitions<IO, MODE, S, V>(mc, Es, Ds, Rs, ar, ai, em);
+      }
+      if constexpr (RST) p1_block_resets<S, V>(kv, ar, ai);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        float cr[V], ci[V];
+        unpack<IO, V>(xr[s], cr);
+        unpack<IO, V>(xi[s], ci);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          if constexpr (GW) {
+            wr[s][v] = cr[v];
+            wi[s][v] = ci[v];
+          } else {
+            const float eta = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ev), s));
+            const StepMode q = p1_step<P1Math<IO, MODE>::HW>(mc.nu[v], mc.ct[v], mc.st[v], mc.g2[v], mc.pl[v],
+                                                             mc.rl[v], Es[s], eta, Ds[s], Rs[s]);
+            ar[s][v] = q.ar;
+            ai[s][v] = q.ai;
+            wr[s][v] = q.gain * tanh_fast(cr[v]);
+            wi[s][v] = q.gain * tanh_fast(ci[v]);
+            if constexpr (kRoundWrite<IO>) round_bf16x2(wr[s][v], wi[s][v]);
+          }
+        }
+      }
+    }
+    if constexpr (!TAIL) load_rows(t0 + NW * S);
+    if (wave < NW - 1) {  // this wave's map (nobody reads the last wave's)
+      float Pr[V], Pi[V], Qr[V], Qi[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) { Pr[v] = 1.0f; Pi[v] = 0.0f; Qr[v] = 0.0f; Qi[v] = 0.0f; }
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if (TAIL && t0 + s >= T) break;  // wave-uniform
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const float qr = fmaf(ar[s][v], Qr[v], fmaf(-ai[s][v], Qi[v], wr[s][v]));
+          Qi[v] = fmaf(ai[s][v], Qr[v], fmaf(ar[s][v], Qi[v], wi[s][v]));
+          Qr[v] = qr;
+          const float pr = fmaf(ar[s][v], Pr[v], -ai[s][v] * Pi[v]);
+          Pi[v] = fmaf(ai[s][v], Pr[v], ar[s][v] * Pi[v]);
+          Pr[v] = pr;
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+        split_lds[(((k & 1) * (NW - 1) + wave) * V + v) * 64 + lane] = make_float4(Pr[v], Pi[v], Qr[v], Qi[v]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < V; ++v) {  // the state before this round, as its last wave left it
+      const float2 h = states[((k & 1) * V + v) * 64 + lane];
+      hr[v] = h.x;
+      hi[v] = h.y;
+    }
+    for (int j = 0; j < wave; ++j) {  // the maps before this wave's
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const float4 e = split_lds[(((k & 1) * (NW - 1) + j) * V + v) * 64 + lane];
+        const float nr = fmaf(e.x, hr[v], fmaf(-e.y, hi[v], e.z));
+        hi[v] = fmaf(e.x, hi[v], fmaf(e.y, hr[v], e.w));
+        hr[v] = nr;
+      }
+    }
+    // the replay and the stores
+    const int ts = TAIL ? min(t0, T - 1) : t0;
+    const int64_t yoff = wave_uniform(((row0 + ts) * W + mbase) * ESZ);
+    const int64_t hoff = wave_uniform(((row0 + ts) * a.M + mbase) * ESZ);
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc(static_cast<char*>(a.y) + yoff, S * row_x);
+    const __amdgpu_buffer_rsrc_t rhr = make_rsrc(static_cast<char*>(a.h_re) + hoff, S * half_x);
+    const __amdgpu_buffer_rsrc_t rhi = make_rsrc(static_cast<char*>(a.h_im) + hoff, S * half_x);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if (TAIL && t0 + s >= T) break;  // wave-uniform
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const float nr = fmaf(ar[s][v], hr[v], fmaf(-ai[s][v], hi[v], wr[s][v]));
+        const float ni = fmaf(ai[s][v], hr[v], fmaf(ar[s][v], hi[v], wi[s][v]));
+        hr[v] = nr;
+        hi[v] = ni;
+      }
+      if constexpr (CM != kPlanes) {  // y = relu(cat(h_re, h_im))
+        float rr[V], ri[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) { rr[v] = fmaxf(hr[v], 0.0f); ri[v] = fmaxf(hi[v], 0.0f); }
+        const uint32_t yo = static_cast<uint32_t>(s) * row_x;
+        buf_store<RawT, CPOL_NT>(pack<IO, V>(rr), ry, lane_st, yo);
+        buf_store<RawT, CPOL_NT>(pack<IO, V>(ri), ry, lane_st, yo + half_x);
+      }
+      if constexpr (CM != kRelu) {  // the states
+        const uint32_t ho = static_cast<uint32_t>(s) * half_x;
+        buf_store<RawT, CPOL_NT>(pack<IO, V>(hr), rhr, lane_st, ho);
+        buf_store<RawT, CPOL_NT>(pack<IO, V>(hi), rhi, lane_st, ho);
+      }
+    }
+    if (wave == NW - 1) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) states[((1 - (k & 1)) * V + v) * 64 + lane] = make_float2(hr[v], hi[v]);
+    }
+    if constexpr (GW) {
+      // the state after the last step of every 64-step chunk and after T-1
+      const int t_last = (TAIL ? min(t0 + S, T) : t0 + S) - 1;
+      if (t_last >= t0 && ((t_last + 1) % kStateChunk == 0 || t_last == T - 1)) {  // wave-uniform
+        const int64_t n_chunks = (T + kStateChunk - 1) / kStateChunk;
+        const int64_t off = wave_uniform(((static_cast<int64_t>(b) * n_chunks + t_last / kStateChunk) * a.M + mbase) * 8);
+        const __amdgpu_buffer_rsrc_t rc = make_rsrc(reinterpret_cast<char*>(a.chunk_state) + off, MB * 8u);
+        float o[2 * V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) { o[2 * v] = hr[v]; o[2 * v + 1] = hi[v]; }
+        buffer_store_f32<2 * V, CPOL_DEFAULT>(rc, lane_ok ? static_cast<uint32_t>(lane * V * 8) : kDropOffset, o);
+      }
+    }
+    if (a.last_re && lane_ok && t0 < T && t0 + S >= T) {  // this wave holds step T-1
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        a.last_re[static_cast<int64_t>(b) * a.M + m0 + v] = hr[v];
+        a.last_im[static_cast<int64_t>(b) * a.M + m0 + v] = hi[v];
+      }
+    }
+  };
+  const int n_full = T / (NW * S);
+  load_rows(wave * S);
+  for (int k = 0; k < n_full; ++k) round(k, std::false_type{});
+  if (n_full * NW * S < T) round(n_full, std::true_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1987,20 +2216,56 @@ ControlsLayout controls_layout(int64_t R, int64_t W) {
 #endif
 constexpr int kPieces = SPARC_MIXER_BWD_PIECES;
 
+// Split chains.  The forward gives each chain (batch row x 128 modes) the
+// waves of one workgroup (mixer_fwd_split_kernel), 8 steps of a round per
+// wave (fp32: 4, which hold the same registers).  Waves per chain so that
+// about two to four run per SIMD; measured (us, forward without gradients,
+// one wave per chain or time segments against split):
+//   module bf16: 128 modes x 1024 chains, T=4096 1775 -> 1694 (the wide
+//     kernel before); 512 chains 1070 -> 897-919; 384 chains, T=2048 594 ->
+//     411; 256 chains, T=1024 222 -> 136; fp32, 128 chains 345 -> 273
+//   P1 bf16: 512 chains, T=4096 630 -> 448; 256 chains, T=2048 188 -> 107;
+//     128 chains, T=4096 174 -> 165; fp32, 192 chains, T=1024 150 -> 97
+// Fewer chains than that leave CUs idle (module, 96 chains, T=4000: 310 in
+// segments, 391 split; 16 chains, T=4096: 96 and 321), except where T is
+// short: segments have at least 128 steps and two passes (module, 8 chains,
+// T=700: 93 -> 66; 16 chains, T=256, fp32: 85 -> 45; T=1500: 97 against 128).
+// The wide kernel stays ahead with many chains for the P1 scan (754 against
+// 822-918 at 1024 chains, T=4096) and the fp32 module (1475 against 1724,
+// T=2048), and below kSplitMinSteps with many chains nothing is split.
+constexpr int kSplitV = 2;
+template <typename IO> constexpr int kSplitFwdS = sizeof(IO) == 2 ? 8 : 4;
+constexpr int64_t kSplitChains = 128, kSplitMinSteps = 2 * kMinSegSteps, kSplitFewSteps = 768;
+// waves per chain of the split forward, 0: not split
+int split_waves(int64_t B, int64_t T, int64_t M) {
+  const int64_t chains = B * ((M + 64 * kSplitV - 1) / (64 * kSplitV));
+  if (chains < kSplitChains) {
+    if (T < 16 || T > kSplitFewSteps) return 0;
+    return static_cast<int>(std::min<int64_t>(kSplitWaves, (T + 3) / 4));
+  }
+  if (T < kSplitMinSteps) return 0;
+  return chains >= 512 ? 4 : chains >= 192 ? 8 : kSplitWaves;
+}
 struct Layout {
   bool piped = false;
+  int split = 0;  // waves per chain of the split-chain kernels (0: not taken)
   int V = 1, n_mb = 0, n_rb = 0, rb_rows = 0, n_rb_piece = 0, n_seg = 1, t_seg = 1;
   int64_t R = 0;
   size_t consts = 0, part_tok = 0, tok = 0, part_mode = 0, pd = 0, pbias = 0, seg_sum = 0, seg_state = 0, total = 0;
 };
 
 // gw: the P1 scan with the writes given (no controls, two per-mode gradients);
-// pieces: the module backward in time pieces where the shape allows
-Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, bool pieces = false) {
+// pieces: the module backward in time pieces where the shape allows;
+// allow_split: the split-chain kernels where the shape takes them
+Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, bool pieces = false,
+              bool allow_split = true) {
   Layout l;
   l.V = mixer_v(B, T, M, direction, gw);
+  l.split = allow_split && direction == 0 ? split_waves(B, T, M) : 0;
+  if (l.split) l.V = kSplitV;
   l.n_mb = static_cast<int>((M + 64 * l.V - 1) / (64 * l.V));
-  choose_segments(B, T, l.n_mb, l.n_seg, l.t_seg);
+  if (l.split) l.t_seg = static_cast<int>(T);
+  else choose_segments(B, T, l.n_mb, l.n_seg, l.t_seg);
   l.R = B * T;
   const ControlsLayout cl = controls_layout(l.R, 2 * M);
   l.n_rb = cl.n_rb;
@@ -2162,8 +2427,24 @@ constexpr int64_t kWideChains = SPARC_MIXER_WIDE_CHAINS;
 constexpr int64_t kWideChainsMaxModule = 1024;
 bool fwd_wide(const Layout& l, int64_t batch, int64_t modes, bool module = false) {
   const int64_t chains = batch * ((modes + 255) / 256);
-  return SPARC_MIXER_WIDE && l.n_seg == 1 && modes % 4 == 0 && chains >= kWideChains &&
+  return SPARC_MIXER_WIDE && l.n_seg == 1 && !l.split && modes % 4 == 0 && chains >= kWideChains &&
          (!module || chains <= kWideChainsMaxModule);
+}
+// The forward's layout: split chains unless the wide kernel is the faster one
+// there (the P1 scan and the fp32 module with many chains, see split_waves).
+Layout forward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, bool gw) {
+  const Layout l = layout(batch, length, modes, 0, gw, false, false);
+  if ((gw || io_dtype == SPARC_F32) && fwd_wide(l, batch, modes, !gw)) return l;
+  return layout(batch, length, modes, 0, gw);
+}
+
+// the split forward: l.split waves per chain
+template <int MODE>
+void run_fwd_split(const Args& a, int nw, bool bf, hipStream_t st) {
+  const dim3 g(static_cast<unsigned>(a.B) * static_cast<unsigned>(a.n_mb)), blk(64 * static_cast<unsigned>(nw));
+  const size_t lds = static_cast<size_t>(2) * (nw - 1) * kSplitV * 64 * 16 + 2 * kSplitV * 64 * 8;
+  if (bf) hipLaunchKernelGGL((mixer_fwd_split_kernel<sparc::bf16, kSplitV, kSplitFwdS<sparc::bf16>, MODE>), g, blk, lds, st, a);
+  else hipLaunchKernelGGL((mixer_fwd_split_kernel<float, kSplitV, kSplitFwdS<float>, MODE>), g, blk, lds, st, a);
 }
 
 // the wide forward (a.n_mb: blocks of 256 modes)
@@ -2204,7 +2485,9 @@ sparc_status scan_forward_impl(const Layout& l, int64_t batch, int64_t length, i
     a.n_seg = l.n_seg; a.t_seg = l.t_seg; a.seg_lo = 0;
     a.seg_sum = reinterpret_cast<float*>(ws + l.seg_sum);
     a.seg_state = reinterpret_cast<float*>(ws + l.seg_state);
-    if (fwd_wide(l, batch, modes, true)) {
+    if (l.split) {
+      run_fwd_split<kModule>(a, l.split, io_dtype == SPARC_BF16, st);
+    } else if (fwd_wide(l, batch, modes, true)) {
       a.n_mb = static_cast<int>((modes + 255) / 256);
       run_fwd_wide<kModule>(a, io_dtype == SPARC_BF16, st);
     } else if (io_dtype == SPARC_BF16) {
@@ -2321,6 +2604,7 @@ bool p1_fused_shape(const sparc_scan_desc* d) {
 
 size_t p1_fused_workspace_bytes(const sparc_scan_desc* d, int direction) {
   if (!p1_fused_shape(d)) return 0;
+  if (direction == 0) return forward_layout(d->batch, d->length, d->modes, d->io_dtype, true).total;
   return layout(d->batch, d->length, d->modes, direction, true).total;
 }
 
@@ -2348,7 +2632,7 @@ sparc_status p1_fused_forward(const sparc_scan_desc* d, const float* eta, const 
                               void* y_im, float* chunk_state, void* workspace, size_t workspace_bytes,
                               sparc_stream_t stream) {
   if (!p1_fused_shape(d) || d->length <= 0) return fail(SPARC_EINVAL, "p1 fused forward: shape");
-  const Layout l = layout(d->batch, d->length, d->modes, 0, true);
+  const Layout l = forward_layout(d->batch, d->length, d->modes, d->io_dtype, true);
   if (workspace_bytes < l.total) return fail(SPARC_EWORKSPACE, "workspace too small: %zu < %zu", workspace_bytes, l.total);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
@@ -2377,7 +2661,12 @@ sparc_status p1_fused_forward(const sparc_scan_desc* d, const float* eta, const 
   a.seg_sum = reinterpret_cast<float*>(ws + l.seg_sum);
   a.seg_state = reinterpret_cast<float*>(ws + l.seg_state);
   const bool bf = d->io_dtype == SPARC_BF16;
-  if (fwd_wide(l, d->batch, d->modes)) {
+  if (l.split) {
+    if (relu && reset) run_fwd_split<kRelu | kReset>(a, l.split, bf, st);
+    else if (relu) run_fwd_split<kRelu>(a, l.split, bf, st);
+    else if (reset) run_fwd_split<kPlanes | kReset>(a, l.split, bf, st);
+    else run_fwd_split<kPlanes>(a, l.split, bf, st);
+  } else if (fwd_wide(l, d->batch, d->modes)) {
     a.n_mb = static_cast<int>((d->modes + 255) / 256);
     if (relu && reset) run_fwd_wide<kRelu | kReset>(a, bf, st);
     else if (relu) run_fwd_wide<kRelu>(a, bf, st);
@@ -2777,8 +3066,10 @@ extern "C" {
 
 size_t sparc_mixer_workspace_bytes(int64_t batch, int64_t length, int64_t modes, int direction) {
   if (batch <= 0 || length < 0 || modes <= 0 || modes % 4 || (direction != 0 && direction != 1)) return 0;
-  // the module backward may run in time pieces or in one launch (larger workspaces)
+  // every form either I/O type may take: chains split or not, and the module
+  // backward in time pieces or in one launch
   size_t n = std::max(layout(batch, length, modes, direction).total, layout(batch, length, modes, direction, false, true).total);
+  n = std::max(n, layout(batch, length, modes, direction, false, false, false).total);
   if (direction == 1) n = std::max(n, coop_layout(batch, length, modes, kCoopS).total);
   return n;
 }
@@ -2807,7 +3098,7 @@ sparc_status sparc_mixer_scan_forward(int64_t batch, int64_t length, int64_t mod
       !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
     return fail(SPARC_EINVAL, "mixer scan forward: NULL pointer");
   if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer scan forward: last_re/last_im");
-  const Layout l = layout(batch, length, modes, 0);
+  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer scan forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
   const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
@@ -2831,7 +3122,7 @@ sparc_status sparc_mixer_forward(int64_t batch, int64_t length, int64_t modes, i
       !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
     return fail(SPARC_EINVAL, "mixer forward: NULL pointer");
   if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer forward: last_re/last_im");
-  const Layout l = layout(batch, length, modes, 0);
+  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
   const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;

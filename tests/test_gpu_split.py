@@ -1,0 +1,102 @@
+"""The split-chain kernels (a chain's time shared by the waves of a workgroup)
+at the sizes where they can go wrong: one round and its remainders, rounds
+that end on and off the 64-step chunks, lanes past M, every number of waves
+per chain, and the chain modes (states or relu out, an initial state, resets,
+a gradient through the last state).
+
+Few chains are held against the float64 oracle; the shapes with enough chains
+for 16, 8 and 4 waves each against the general chain kernels, whose per-step
+recurrence is the same: both are fp32 recurrences with relative error about
+2^-24 per remembered step, so 1e-5 of max |reference| over 300 steps (bf16
+I/O: one rounding to 8 bits, 2^-8)."""
+import pytest
+import torch
+
+import sparc_amd
+from sparc_amd import ops
+from test_gpu_scan import BF16, F32, check_case, make_case, rel_err
+
+pytestmark = pytest.mark.gpu
+
+FEW = [  # few chains: T from 16 to 768 steps is split
+    ("one_round_f32", 2, 16, 256, F32, {}),
+    ("one_past_f32", 2, 17, 132, F32, dict(h0=True, dlast=True)),
+    ("chunk_less_one_bf16", 1, 63, 256, BF16, dict(h0=True)),
+    ("chunk_plus_one_f32", 1, 65, 128, F32, dict(h0=True, dlast=True, seg=True)),
+    ("round_plus_one_bf16", 2, 129, 260, BF16, dict(dlast=True)),
+    ("resets_bf16", 2, 200, 128, BF16, dict(h0=True, dlast=True, seg=True, reset_first=True)),
+    ("relu_f32", 2, 257, 132, F32, dict(relu=True, h0=True, dlast=True)),
+    ("relu_resets_bf16", 2, 150, 256, BF16, dict(relu=True, seg=True)),
+    ("longest_f32", 1, 768, 64, F32, dict(h0=True, dlast=True)),
+]
+
+
+@pytest.mark.parametrize("cid,B,T,M,dtype,extra", FEW, ids=[c[0] for c in FEW])
+def test_split_few_chains(cid, B, T, M, dtype, extra):
+    print(f"[case] split {cid} B={B} T={T} M={M} {dtype}", flush=True)
+    ops.set_algorithm("auto")
+    check_case(make_case("p1", B, T, M, 1, dtype, seed=sum(map(ord, cid)) % 1000, **extra))
+
+
+def _run(case, algorithm, want_grads):
+    ops.set_algorithm(algorithm)
+    try:
+        names = ("g0", "g1", "nu_log", "theta_log", "w_re", "w_im")
+        leaves = [case[n].cuda().requires_grad_(want_grads) for n in names]
+        init = None if case["init"] is None else tuple(t.cuda().requires_grad_(want_grads) for t in case["init"])
+        segpos = None if case["segpos"] is None else case["segpos"].cuda()
+        y, last = ops.chunk_scan("p1", *leaves[:2], *leaves[4:], *leaves[2:4], initial_state=init, segment_pos=segpos,
+                                 reset_first=case["reset_first"], relu_output=case["relu"])
+        outs = [*([y] if case["relu"] else y), *last]
+        if not want_grads:
+            return outs
+        dys = [case["dy_re"].cuda()] + ([] if case["relu"] else [case["dy_im"].cuda()]) + [d.cuda() for d in case["dlast"]]
+        return outs + list(torch.autograd.grad(outs, leaves + list(init or ()), dys))
+    finally:
+        ops.set_algorithm("auto")
+
+
+@pytest.mark.parametrize("B,M,dtype,extra", [
+    (2, 8188, F32, dict(h0=True, dlast=True)),                            # 128 chains: 16 waves each
+    (3, 8192, BF16, dict(dlast=True, relu=True)),                         # 192 chains: 8 waves
+    (3, 8192, F32, dict(h0=True, dlast=True, seg=True)),
+    (8, 8188, BF16, dict(h0=True, dlast=True, reset_first=True)),         # 512 chains: 4 waves
+    (8, 8192, F32, dict(dlast=True, relu=True, h0=True)),
+], ids=["waves16_f32", "waves8_relu_bf16", "waves8_resets_f32", "waves4_bf16", "waves4_relu_f32"])
+@pytest.mark.parametrize("T", [256, 300])
+def test_split_many_chains(B, M, dtype, extra, T):
+    print(f"[case] split B={B} T={T} M={M} {dtype} {extra}", flush=True)
+    case = make_case("p1", B, T, M, 1, dtype, seed=B + T, **extra)
+    tol = 1e-5 if dtype == F32 else 2.0 ** -8
+    for k, (a, b) in enumerate(zip(_run(case, "auto", False), _run(case, "chain", False))):
+        assert rel_err(a, b) <= tol, f"output {k}: {rel_err(a, b):.3g}"
+
+
+@pytest.mark.parametrize("B,L,width,dtype", [
+    (2, 20, 264, torch.float32), (1, 129, 2048, torch.bfloat16), (2, 300, 16376, torch.float32),
+    (3, 256, 16384, torch.bfloat16), (8, 259, 16384, torch.bfloat16),
+])
+def test_split_module_forward(B, L, width, dtype):
+    """The module's forward (few chains; 16, 8 and 4 waves per chain) against
+    the composed path, whose scan runs the general kernels."""
+    print(f"[case] split module B={B} L={L} width={width} {dtype}", flush=True)
+    torch.manual_seed(L)
+    m = sparc_amd.SPARCMixer(width).cuda()
+    with torch.no_grad():
+        for p in (m.phase_direction, m.radial_direction):
+            p.copy_(torch.randn_like(p) * 0.5 / width ** 0.5)
+        for p in (m.write_phase_response, m.write_radial_response):
+            p.copy_(torch.randn_like(p) * 0.3)
+        x = torch.randn(B, L, width, device="cuda").to(dtype)
+        got = {}
+        for path in ("fused", "composed"):
+            sparc_amd.set_mixer_path(path)
+            try:
+                y, last = m(x, return_cache=True)
+            finally:
+                sparc_amd.set_mixer_path("auto")
+            got[path] = [y, *last]
+    # bf16: the write's rounding meets the states at other places when its last fp32 bit differs
+    tol = 2e-5 if dtype == torch.float32 else 2.0 ** -7
+    for a, b in zip(got["fused"], got["composed"]):
+        assert rel_err(a, b) <= tol, rel_err(a, b)
