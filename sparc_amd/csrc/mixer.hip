@@ -2180,7 +2180,7 @@ void choose_segments(int64_t B, int64_t T, int n_mb, int& n_seg, int& t_seg) {
 }
 
 // The controls backward over rows of width W: n_cb column blocks of 2048
-// inputs, row blocks of `rows` rows (a multiple of 4 in [4, 128], chosen so
+// inputs, row blocks of `rows` rows (a multiple of 4 in [min_rows, 128], chosen so
 // that the grid has about 1024 workgroups), and the partial direction
 // gradients pd [2][n_rb][W] and bias partials pbias [2][n_rb] in the workspace.
 struct ControlsLayout {
@@ -2190,13 +2190,14 @@ struct ControlsLayout {
 
 // (At 512 rows of 2048 fp32, row blocks of 128 left 4 workgroups, each a
 // serial chain of 32 four-row groups: 102 us; with blocks of 4 rows the
-// module's training step there takes 229 us against 306.)
-ControlsLayout controls_layout(int64_t R, int64_t W) {
+// module's training step there takes 229 us against 306.  The generic entry
+// point keeps blocks of at least 16 rows: its workspace size is its callers'.)
+ControlsLayout controls_layout(int64_t R, int64_t W, int min_rows = 16) {
   ControlsLayout c;
   c.n_cb = static_cast<int>((W + 2047) / 2048);
   int64_t rows = (R * c.n_cb + 1023) / 1024;
   rows = (rows + 3) / 4 * 4;
-  c.rows = static_cast<int>(rows < 4 ? 4 : (rows > kCtrlBwdRows ? kCtrlBwdRows : rows));
+  c.rows = static_cast<int>(rows < min_rows ? min_rows : (rows > kCtrlBwdRows ? kCtrlBwdRows : rows));
   c.n_rb = static_cast<int>(std::min<int64_t>((R + c.rows - 1) / c.rows, kMaxRowBlocks));
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   c.pbias = up(static_cast<size_t>(2) * c.n_rb * W * 4);
@@ -2267,7 +2268,7 @@ Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, b
   if (l.split) l.t_seg = static_cast<int>(T);
   else choose_segments(B, T, l.n_mb, l.n_seg, l.t_seg);
   l.R = B * T;
-  const ControlsLayout cl = controls_layout(l.R, 2 * M);
+  const ControlsLayout cl = controls_layout(l.R, 2 * M, 4);
   l.n_rb = cl.n_rb;
   l.rb_rows = cl.rows;
   int np = kPieces;
