@@ -359,7 +359,7 @@ const char* sparc_version(void);
  * h_re, h_im, eta, delta, dy, dx, deta, ddelta) are neither read nor written
  * and may be NULL; the last state is zero and every gradient is zero.
  * ------------------------------------------------------------------------- */
-/* Workspace bytes of sparc_mixer_forward (direction 0) or _backward (1); 0 if
+/* Workspace bytes of sparc_mixer_forward / _infer (direction 0) or _backward (1); 0 if
  * the shape is invalid. */
 size_t sparc_mixer_workspace_bytes(int64_t batch, int64_t length, int64_t modes, int direction);
 
@@ -391,6 +391,24 @@ sparc_status sparc_mixer_scan_forward(int64_t batch, int64_t length, int64_t mod
                                       const float* write_phase_response, const float* write_radial_response,
                                       void* y, void* h_re, void* h_im, float* last_re, float* last_im,
                                       void* workspace, size_t workspace_bytes, sparc_stream_t stream);
+
+/* sparc_mixer_forward and sparc_mixer_scan_forward for a caller that keeps
+ * nothing for a backward: the same y and last state, without the saved
+ * states h_re, h_im (a third of what the forward writes).  Replaces the same
+ * reference path under torch.no_grad (sparc-kernal/backward/scan.py:1839-1877
+ * for its own inference scans). */
+sparc_status sparc_mixer_infer(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
+                               const void* x, const float* phase_direction, const float* radial_direction,
+                               const float* nu_log, const float* theta_log, const float* write_log_gain,
+                               const float* write_phase_response, const float* write_radial_response,
+                               float* eta, float* delta, void* y, float* last_re, float* last_im,
+                               void* workspace, size_t workspace_bytes, sparc_stream_t stream);
+sparc_status sparc_mixer_scan_infer(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
+                                    const void* x, const float* eta, const float* delta, const float* nu_log,
+                                    const float* theta_log, const float* write_log_gain,
+                                    const float* write_phase_response, const float* write_radial_response,
+                                    void* y, float* last_re, float* last_im, void* workspace,
+                                    size_t workspace_bytes, sparc_stream_t stream);
 
 /* The backward of sparc_mixer_scan_forward: dx [B,T,2M] (io_dtype) through
  * the write only, deta, ddelta [B*T] fp32 (the gradients of the controls)

@@ -45,10 +45,12 @@ EXPORTED_SYMBOLS = (
     "sparc_column_sum",
     "sparc_mixer_workspace_bytes",
     "sparc_mixer_forward",
+    "sparc_mixer_infer",
     "sparc_mixer_backward",
     "sparc_mixer_backward_form",
     "sparc_mixer_backward_plan",
     "sparc_mixer_scan_forward",
+    "sparc_mixer_scan_infer",
     "sparc_mixer_scan_backward",
     "sparc_controls_forward",
     "sparc_controls_workspace_bytes",
@@ -144,6 +146,10 @@ def load() -> ctypes.CDLL:
         lib.sparc_mixer_backward_plan.restype = ctypes.c_int
         lib.sparc_mixer_scan_forward.argtypes = [_I64, _I64, _I64, _I32] + [_P] * 14 + [_SZ, _P]
         lib.sparc_mixer_scan_forward.restype = ctypes.c_int
+        lib.sparc_mixer_infer.argtypes = [_I64, _I64, _I64, _I32] + [_P] * 14 + [_SZ, _P]
+        lib.sparc_mixer_infer.restype = ctypes.c_int
+        lib.sparc_mixer_scan_infer.argtypes = [_I64, _I64, _I64, _I32] + [_P] * 12 + [_SZ, _P]
+        lib.sparc_mixer_scan_infer.restype = ctypes.c_int
         lib.sparc_mixer_scan_backward.argtypes = [_I64, _I64, _I64, _I32] + [_P] * 22 + [_SZ, _P]
         lib.sparc_mixer_scan_backward.restype = ctypes.c_int
         lib.sparc_controls_forward.argtypes = [_I64, _I64, _I32] + [_P] * 6

@@ -87,10 +87,12 @@ template <typename IO> constexpr bool kRoundWrite = SPARC_MIXER_ROUND_WRITE && s
 //            states (forward only).
 //   | kReset: kPlanes or kRelu with reset steps (segment_pos[b, t] == 0, or
 //            step 0 with reset_first): the transition there is 0.
+//   | kNoSave: kModule without the saved states (forward of a caller that
+//            keeps no gradients: two of its six planes less to write).
 //   | kCoop: the module backward in one launch that also runs the controls'
 //            backward (dx completed, direction gradients): see
 //            mixer_bwd_kernel.
-enum : int { kModule = 0, kPlanes = 1, kRelu = 2, kReset = 4, kCoop = 8 };
+enum : int { kModule = 0, kPlanes = 1, kRelu = 2, kReset = 4, kCoop = 8, kNoSave = 16 };
 constexpr int kStateChunk = 64;  // steps per saved chunk state (sparc_scan_chunk_length)
 constexpr int kSplitWaves = 16;  // most waves per workgroup of the split-chain kernels
 // A lane byte offset past every buffer resource of these kernels (each spans
@@ -505,6 +507,7 @@ mixer_fwd_kernel(Args a) {
   constexpr int CM = MODE & 3;             // the chain mode without kReset
   constexpr bool RST = (MODE & kReset) != 0;
   constexpr bool GW = CM != kModule;  // the writes are given
+  constexpr bool SAVE = CM != kRelu && (MODE & kNoSave) == 0;  // the states out
   static_assert(kStateChunk % kS == 0, "blocks must tile the saved-state chunks");
   static_assert(GW || !RST, "resets in the P1 scan only");
   // a summary's loads keep their lines in the caches (the replay that follows
@@ -684,7 +687,7 @@ mixer_fwd_kernel(Args a) {
         buf_store<RawT, CPOL_NT>(pack<IO, V>(rr), ry, lane_st, yo);
         buf_store<RawT, CPOL_NT>(pack<IO, V>(ri), ry, lane_st, yo + half_x);
       }
-      if constexpr (CM != kRelu) {  // the states
+      if constexpr (SAVE) {  // the states
         const uint32_t ho = static_cast<uint32_t>(s) * half_x;
         buf_store<RawT, CPOL_NT>(pack<IO, V>(hr), rhr, lane_st, ho);
         buf_store<RawT, CPOL_NT>(pack<IO, V>(hi), rhi, lane_st, ho);
@@ -763,6 +766,7 @@ mixer_fwd_wide_kernel(Args a) {
   constexpr int CM = MODE & 3;             // the chain mode without kReset
   constexpr bool RST = (MODE & kReset) != 0;
   constexpr bool GW = CM != kModule;       // the writes are given
+  constexpr bool SAVE = CM != kRelu && (MODE & kNoSave) == 0;  // the states out
   static_assert(GW || !RST, "resets in the P1 scan only");
   constexpr bool PACKW = sizeof(IO) == 2;  // bf16 writes: one dword (re | im << 16) per mode
   static_assert(GW || PACKW == kRoundWrite<IO>, "the module's bf16 writes are rounded to bf16");
@@ -913,8 +917,8 @@ mixer_fwd_wide_kernel(Args a) {
     const int64_t yoff = wave_uniform(((row0 + t0) * W + mbase) * ESZ);
     const int64_t hoff = wave_uniform(((row0 + t0) * a.M + mbase) * ESZ);
     const __amdgpu_buffer_rsrc_t ry = make_rsrc(static_cast<char*>(a.y) + yoff, CM != kPlanes ? S * row_x : 0u);
-    const __amdgpu_buffer_rsrc_t rhr = make_rsrc(static_cast<char*>(a.h_re) + hoff, CM != kRelu ? S * half_x : 0u);
-    const __amdgpu_buffer_rsrc_t rhi = make_rsrc(static_cast<char*>(a.h_im) + hoff, CM != kRelu ? S * half_x : 0u);
+    const __amdgpu_buffer_rsrc_t rhr = make_rsrc(static_cast<char*>(a.h_re) + hoff, SAVE ? S * half_x : 0u);
+    const __amdgpu_buffer_rsrc_t rhi = make_rsrc(static_cast<char*>(a.h_im) + hoff, SAVE ? S * half_x : 0u);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       if (t0 + s >= T) break;  // wave-uniform
@@ -949,7 +953,7 @@ mixer_fwd_wide_kernel(Args a) {
         buf_store<RawT, CPOL_NT>(pack<IO, V>(rr), ry, lane_st, yo);
         buf_store<RawT, CPOL_NT>(pack<IO, V>(ri), ry, lane_st, yo + half_x);
       }
-      if constexpr (CM != kRelu) {  // the states
+      if constexpr (SAVE) {  // the states
         const uint32_t ho = static_cast<uint32_t>(s) * half_x;
         buf_store<RawT, CPOL_NT>(pack<IO, V>(hr), rhr, lane_st, ho);
         buf_store<RawT, CPOL_NT>(pack<IO, V>(hi), rhi, lane_st, ho);
@@ -1024,6 +1028,7 @@ mixer_fwd_split_kernel(Args a) {
   constexpr int CM = MODE & 3;             // the chain mode without kReset
   constexpr bool RST = (MODE & kReset) != 0;
   constexpr bool GW = CM != kModule;       // the writes are given
+  constexpr bool SAVE = CM != kRelu && (MODE & kNoSave) == 0;  // the states out
   static_assert(kStateChunk % S == 0, "blocks must tile the saved-state chunks");
   static_assert(GW || !RST, "resets in the P1 scan only");
   // [2][NW - 1][V][64] maps (Pr, Pi, Qr, Qi) of the waves but the last, then
@@ -1191,7 +1196,7 @@ mixer_fwd_split_kernel(Args a) {
         buf_store<RawT, CPOL_NT>(pack<IO, V>(rr), ry, lane_st, yo);
         buf_store<RawT, CPOL_NT>(pack<IO, V>(ri), ry, lane_st, yo + half_x);
       }
-      if constexpr (CM != kRelu) {  // the states
+      if constexpr (SAVE) {  // the states
         const uint32_t ho = static_cast<uint32_t>(s) * half_x;
         buf_store<RawT, CPOL_NT>(pack<IO, V>(hr), rhr, lane_st, ho);
         buf_store<RawT, CPOL_NT>(pack<IO, V>(hi), rhi, lane_st, ho);
@@ -2456,9 +2461,24 @@ void run_fwd_wide(const Args& a, bool bf, hipStream_t st) {
   else hipLaunchKernelGGL((mixer_fwd_wide_kernel<float, kWideHelpers, kWideS, MODE>), g, blk, 0, st, a);
 }
 
+// the module's forward in the form its layout chose
+template <int MODE>
+void run_fwd_module(const Layout& l, Args a, bool bf, hipStream_t st) {
+  if (l.split) {
+    run_fwd_split<MODE>(a, l.split, bf, st);
+  } else if (fwd_wide(l, a.B, a.M, true)) {
+    a.n_mb = (a.M + 255) / 256;
+    run_fwd_wide<MODE>(a, bf, st);
+  } else if (bf) {
+    if (l.V == 2) run_fwd<sparc::bf16, 2, MODE>(a, st); else run_fwd<sparc::bf16, 1, MODE>(a, st);
+  } else {
+    if (l.V == 2) run_fwd<float, 2, MODE>(a, st); else run_fwd<float, 1, MODE>(a, st);
+  }
+}
+
 // The scan and its backward with the controls given; the per-mode constants
 // are built in the workspace first.  Shapes, pointers and the workspace are
-// checked by the callers.
+// checked by the callers.  h_re, h_im NULL: the states are not kept.
 sparc_status scan_forward_impl(const Layout& l, int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
                                const void* x, const float* eta, const float* delta, const float* nu_log,
                                const float* theta_log, const float* write_log_gain,
@@ -2486,16 +2506,9 @@ sparc_status scan_forward_impl(const Layout& l, int64_t batch, int64_t length, i
     a.n_seg = l.n_seg; a.t_seg = l.t_seg; a.seg_lo = 0;
     a.seg_sum = reinterpret_cast<float*>(ws + l.seg_sum);
     a.seg_state = reinterpret_cast<float*>(ws + l.seg_state);
-    if (l.split) {
-      run_fwd_split<kModule>(a, l.split, io_dtype == SPARC_BF16, st);
-    } else if (fwd_wide(l, batch, modes, true)) {
-      a.n_mb = static_cast<int>((modes + 255) / 256);
-      run_fwd_wide<kModule>(a, io_dtype == SPARC_BF16, st);
-    } else if (io_dtype == SPARC_BF16) {
-      if (l.V == 2) run_fwd<sparc::bf16, 2>(a, st); else run_fwd<sparc::bf16, 1>(a, st);
-    } else {
-      if (l.V == 2) run_fwd<float, 2>(a, st); else run_fwd<float, 1>(a, st);
-    }
+    const bool bf = io_dtype == SPARC_BF16;
+    if (h_re) run_fwd_module<kModule>(l, a, bf, st);
+    else run_fwd_module<kModule | kNoSave>(l, a, bf, st);
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? SPARC_OK : fail(SPARC_EHIP, "mixer scan forward: %s", hipGetErrorString(e));
@@ -3063,6 +3076,65 @@ sparc_status coop_backward(int kS, int64_t batch, int64_t length, int64_t modes,
   return e == hipSuccess ? SPARC_OK : fail(SPARC_EHIP, "mixer backward: %s", hipGetErrorString(e));
 }
 
+// sparc_mixer_scan_forward (save) and sparc_mixer_scan_infer (h_re, h_im NULL)
+static sparc_status scan_forward_call(bool save, int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
+                                      const void* x, const float* eta, const float* delta, const float* nu_log,
+                                      const float* theta_log, const float* write_log_gain,
+                                      const float* write_phase_response, const float* write_radial_response,
+                                      void* y, void* h_re, void* h_im, float* last_re, float* last_im,
+                                      void* workspace, size_t workspace_bytes, sparc_stream_t stream) {
+  if (sparc_status s = check_shape(batch, length, modes, io_dtype)) return s;
+  // per-token tensors may be NULL when length is 0 (nothing is read or written)
+  const bool rows = length > 0;
+  if ((rows && (!x || !eta || !delta || !y || (save && (!h_re || !h_im)))) ||
+      !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
+    return fail(SPARC_EINVAL, "mixer scan forward: NULL pointer");
+  if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer scan forward: last_re/last_im");
+  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
+  if (!workspace || workspace_bytes < l.total)
+    return fail(SPARC_EWORKSPACE, "mixer scan forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
+  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
+  if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(workspace, 256))
+    return fail(SPARC_EINVAL, "mixer scan forward: misaligned tensor");
+  return scan_forward_impl(l, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
+                           write_phase_response, write_radial_response, y, h_re, h_im, last_re, last_im,
+                           static_cast<char*>(workspace), reinterpret_cast<hipStream_t>(stream));
+}
+
+// sparc_mixer_forward (save) and sparc_mixer_infer (h_re, h_im NULL)
+static sparc_status mixer_forward_call(bool save, int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
+                                       const void* x, const float* phase_direction, const float* radial_direction,
+                                       const float* nu_log, const float* theta_log, const float* write_log_gain,
+                                       const float* write_phase_response, const float* write_radial_response,
+                                       float* eta, float* delta, void* y, void* h_re, void* h_im,
+                                       float* last_re, float* last_im, void* workspace, size_t workspace_bytes,
+                                       sparc_stream_t stream) {
+  if (sparc_status s = check_shape(batch, length, modes, io_dtype)) return s;
+  const bool rows = length > 0;  // per-token tensors may be NULL when length is 0
+  if ((rows && (!x || !eta || !delta || !y || (save && (!h_re || !h_im)))) || !phase_direction || !radial_direction ||
+      !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
+    return fail(SPARC_EINVAL, "mixer forward: NULL pointer");
+  if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer forward: last_re/last_im");
+  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
+  if (!workspace || workspace_bytes < l.total)
+    return fail(SPARC_EWORKSPACE, "mixer forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
+  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
+  if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(phase_direction, 16) ||
+      !al(radial_direction, 16) || !al(workspace, 256))
+    return fail(SPARC_EINVAL, "mixer forward: misaligned tensor");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int W = 2 * static_cast<int>(modes);
+  if (length > 0) {
+    if (io_dtype == SPARC_BF16)
+      launch_ctrl_fwd<sparc::bf16>(st, l.R, W, x, phase_direction, radial_direction, eta, delta);
+    else
+      launch_ctrl_fwd<float>(st, l.R, W, x, phase_direction, radial_direction, eta, delta);
+  }
+  return scan_forward_impl(l, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
+                           write_phase_response, write_radial_response, y, h_re, h_im, last_re, last_im,
+                           static_cast<char*>(workspace), st);
+}
+
 extern "C" {
 
 size_t sparc_mixer_workspace_bytes(int64_t batch, int64_t length, int64_t modes, int direction) {
@@ -3092,22 +3164,20 @@ sparc_status sparc_mixer_scan_forward(int64_t batch, int64_t length, int64_t mod
                                       const float* write_phase_response, const float* write_radial_response,
                                       void* y, void* h_re, void* h_im, float* last_re, float* last_im,
                                       void* workspace, size_t workspace_bytes, sparc_stream_t stream) {
-  if (sparc_status s = check_shape(batch, length, modes, io_dtype)) return s;
-  // per-token tensors may be NULL when length is 0 (nothing is read or written)
-  const bool rows = length > 0;
-  if ((rows && (!x || !eta || !delta || !y || !h_re || !h_im)) ||
-      !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
-    return fail(SPARC_EINVAL, "mixer scan forward: NULL pointer");
-  if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer scan forward: last_re/last_im");
-  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
-  if (!workspace || workspace_bytes < l.total)
-    return fail(SPARC_EWORKSPACE, "mixer scan forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
-  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
-  if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(workspace, 256))
-    return fail(SPARC_EINVAL, "mixer scan forward: misaligned tensor");
-  return scan_forward_impl(l, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
-                           write_phase_response, write_radial_response, y, h_re, h_im, last_re, last_im,
-                           static_cast<char*>(workspace), reinterpret_cast<hipStream_t>(stream));
+  return scan_forward_call(true, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
+                           write_phase_response, write_radial_response, y, h_re, h_im, last_re, last_im, workspace,
+                           workspace_bytes, stream);
+}
+
+sparc_status sparc_mixer_scan_infer(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
+                                    const void* x, const float* eta, const float* delta, const float* nu_log,
+                                    const float* theta_log, const float* write_log_gain,
+                                    const float* write_phase_response, const float* write_radial_response,
+                                    void* y, float* last_re, float* last_im, void* workspace,
+                                    size_t workspace_bytes, sparc_stream_t stream) {
+  return scan_forward_call(false, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
+                           write_phase_response, write_radial_response, y, nullptr, nullptr, last_re, last_im,
+                           workspace, workspace_bytes, stream);
 }
 
 sparc_status sparc_mixer_forward(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
@@ -3117,30 +3187,20 @@ sparc_status sparc_mixer_forward(int64_t batch, int64_t length, int64_t modes, i
                                  float* eta, float* delta, void* y, void* h_re, void* h_im,
                                  float* last_re, float* last_im, void* workspace, size_t workspace_bytes,
                                  sparc_stream_t stream) {
-  if (sparc_status s = check_shape(batch, length, modes, io_dtype)) return s;
-  const bool rows = length > 0;  // per-token tensors may be NULL when length is 0
-  if ((rows && (!x || !eta || !delta || !y || !h_re || !h_im)) || !phase_direction || !radial_direction ||
-      !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
-    return fail(SPARC_EINVAL, "mixer forward: NULL pointer");
-  if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer forward: last_re/last_im");
-  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
-  if (!workspace || workspace_bytes < l.total)
-    return fail(SPARC_EWORKSPACE, "mixer forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
-  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
-  if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(phase_direction, 16) ||
-      !al(radial_direction, 16) || !al(workspace, 256))
-    return fail(SPARC_EINVAL, "mixer forward: misaligned tensor");
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int W = 2 * static_cast<int>(modes);
-  if (length > 0) {
-    if (io_dtype == SPARC_BF16)
-      launch_ctrl_fwd<sparc::bf16>(st, l.R, W, x, phase_direction, radial_direction, eta, delta);
-    else
-      launch_ctrl_fwd<float>(st, l.R, W, x, phase_direction, radial_direction, eta, delta);
-  }
-  return scan_forward_impl(l, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
-                           write_phase_response, write_radial_response, y, h_re, h_im, last_re, last_im,
-                           static_cast<char*>(workspace), st);
+  return mixer_forward_call(true, batch, length, modes, io_dtype, x, phase_direction, radial_direction, nu_log,
+                            theta_log, write_log_gain, write_phase_response, write_radial_response, eta, delta, y,
+                            h_re, h_im, last_re, last_im, workspace, workspace_bytes, stream);
+}
+
+sparc_status sparc_mixer_infer(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
+                               const void* x, const float* phase_direction, const float* radial_direction,
+                               const float* nu_log, const float* theta_log, const float* write_log_gain,
+                               const float* write_phase_response, const float* write_radial_response,
+                               float* eta, float* delta, void* y, float* last_re, float* last_im,
+                               void* workspace, size_t workspace_bytes, sparc_stream_t stream) {
+  return mixer_forward_call(false, batch, length, modes, io_dtype, x, phase_direction, radial_direction, nu_log,
+                            theta_log, write_log_gain, write_phase_response, write_radial_response, eta, delta, y,
+                            nullptr, nullptr, last_re, last_im, workspace, workspace_bytes, stream);
 }
 
 sparc_status sparc_mixer_scan_backward(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,

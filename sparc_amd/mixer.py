@@ -94,13 +94,20 @@ _PARAMS = ("phase_direction", "radial_direction", "nu_log", "theta_log", "write_
            "write_phase_response", "write_radial_response")
 
 
+def _keeps_gradients(*tensors) -> bool:
+    """Whether a call on these tensors will be differentiated: only then does
+    the forward keep its states."""
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+
+
 class _FusedMixer(torch.autograd.Function):
     """Outputs y = relu(cat(h_re, h_im)) [B, L, 2M] (x's dtype) and the last
-    state (last_re, last_im) fp32 [B, M]."""
+    state (last_re, last_im) fp32 [B, M].  ``save``: keep the states for the
+    backward (False: there will be none)."""
 
     @staticmethod
     def forward(ctx, x, phase_direction, radial_direction, nu_log, theta_log, write_log_gain,
-                write_phase_response, write_radial_response, energy_response):
+                write_phase_response, write_radial_response, energy_response, save=True):
         lib = _lib.load()
         _lib.check_params(x.shape[-1], phase_direction=phase_direction, radial_direction=radial_direction,
                           nu_log=nu_log, theta_log=theta_log, write_log_gain=write_log_gain,
@@ -116,8 +123,6 @@ class _FusedMixer(torch.autograd.Function):
         eta = torch.empty(B, T, dtype=torch.float32, device=dev)
         delta = torch.empty_like(eta)
         y = torch.empty_like(x)
-        h_re = torch.empty(B, T, M, dtype=x.dtype, device=dev)
-        h_im = torch.empty_like(h_re)
         last_re = torch.empty(B, M, dtype=torch.float32, device=dev)
         last_im = torch.empty_like(last_re)
         ws_bytes = lib.sparc_mixer_workspace_bytes(B, T, M, 0)
@@ -125,6 +130,13 @@ class _FusedMixer(torch.autograd.Function):
             raise ValueError("invalid shape for the fused mixer")
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         P = _lib.ptr
+        if not save:
+            _lib.check(lib.sparc_mixer_infer(
+                B, T, M, io, P(x), *[P(p) for p in params], P(eta), P(delta), P(y), P(last_re), P(last_im), P(ws),
+                ws.numel(), _lib.stream_of(dev)), "sparc_mixer_infer")
+            return y, last_re, last_im
+        h_re = torch.empty(B, T, M, dtype=x.dtype, device=dev)
+        h_im = torch.empty_like(h_re)
         _lib.check(lib.sparc_mixer_forward(
             B, T, M, io, P(x), *[P(p) for p in params], P(eta), P(delta), P(y), P(h_re), P(h_im),
             P(last_re), P(last_im), P(ws), ws.numel(), _lib.stream_of(dev)), "sparc_mixer_forward")
@@ -161,13 +173,13 @@ class _FusedMixer(torch.autograd.Function):
         grads = [g.to(dt) for g, dt in zip(grads, ctx.dtypes)]
         shape, dt = ctx.energy
         # energy_response is an inactive parameter (0 * sum in make_controls): gradient 0
-        return (dx, *grads, torch.zeros(shape, dtype=dt, device=dev))
+        return (dx, *grads, torch.zeros(shape, dtype=dt, device=dev), None)
 
 
 def fused_sequence(module, x: torch.Tensor):
     """(y, (last_re, last_im)) of the module on x through the fused path."""
-    y, last_re, last_im = _FusedMixer.apply(
-        x, *[getattr(module, n) for n in _PARAMS], module.energy_response)
+    args = (x, *[getattr(module, n) for n in _PARAMS], module.energy_response)
+    y, last_re, last_im = _FusedMixer.apply(*args, _keeps_gradients(*args))
     return y, (last_re, last_im)
 
 
@@ -186,11 +198,11 @@ class _ProjectedMixer(torch.autograd.Function):
     rank-2 term that the projection's own gradients absorb as
     d xn += dp (u W) and dW += u^T (dp^T xn); the direction gradient is
     (dp^T xn) W^T.  The scan, the write and the epilogue run as
-    sparc_mixer_scan_forward / _backward."""
+    sparc_mixer_scan_forward / _backward.  ``save`` as in _FusedMixer."""
 
     @staticmethod
     def forward(ctx, xn, weight, phase_direction, radial_direction, nu_log, theta_log, write_log_gain,
-                write_phase_response, write_radial_response, energy_response):
+                write_phase_response, write_radial_response, energy_response, save=True):
         lib = _lib.load()
         B, T, D = xn.shape
         W = weight.shape[0]
@@ -234,14 +246,19 @@ class _ProjectedMixer(torch.autograd.Function):
                                               P(delta), _lib.stream_of(dev)), "sparc_controls_forward")
         io = _lib.io_code(x.dtype)
         y = torch.empty_like(x)
-        h_re = torch.empty(B, T, M, dtype=x.dtype, device=dev)
-        h_im = torch.empty_like(h_re)
         last_re = torch.empty(B, M, dtype=torch.float32, device=dev)
         last_im = torch.empty_like(last_re)
         ws_bytes = lib.sparc_mixer_workspace_bytes(B, T, M, 0)
         if ws_bytes == 0:
             raise ValueError("invalid shape for the fused mixer")
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        if not save:
+            _lib.check(lib.sparc_mixer_scan_infer(
+                B, T, M, io, P(x), P(eta), P(delta), *[P(t) for t in params], P(y), P(last_re), P(last_im), P(ws),
+                ws.numel(), _lib.stream_of(dev)), "sparc_mixer_scan_infer")
+            return y, last_re, last_im
+        h_re = torch.empty(B, T, M, dtype=x.dtype, device=dev)
+        h_im = torch.empty_like(h_re)
         _lib.check(lib.sparc_mixer_scan_forward(
             B, T, M, io, P(x), P(eta), P(delta), *[P(t) for t in params], P(y), P(h_re), P(h_im),
             P(last_re), P(last_im), P(ws), ws.numel(), _lib.stream_of(dev)), "sparc_mixer_scan_forward")
@@ -310,7 +327,7 @@ class _ProjectedMixer(torch.autograd.Function):
         else:
             out = [g.to(dt) for g, dt in zip([g_dirs[0], g_dirs[1], *grads], ctx.dtypes)]
         shape, dt = ctx.energy
-        return (g_xn, g_w.to(weight.dtype), *out, torch.zeros(shape, dtype=dt, device=dev))
+        return (g_xn, g_w.to(weight.dtype), *out, torch.zeros(shape, dtype=dt, device=dev), None)
 
 
 def projected_fused_supported(xn: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -322,6 +339,6 @@ def projected_fused_supported(xn: torch.Tensor, weight: torch.Tensor) -> bool:
 def projected_sequence(module, xn: torch.Tensor, weight: torch.Tensor):
     """(y, (last_re, last_im)) of ``module`` on ``xn @ weight^T`` with the
     controls folded into the projection."""
-    y, last_re, last_im = _ProjectedMixer.apply(
-        xn, weight, *[getattr(module, n) for n in _PARAMS], module.energy_response)
+    args = (xn, weight, *[getattr(module, n) for n in _PARAMS], module.energy_response)
+    y, last_re, last_im = _ProjectedMixer.apply(*args, _keeps_gradients(*args))
     return y, (last_re, last_im)

@@ -1,5 +1,5 @@
 """The controls kernels over every number of rows per workgroup that their
-launches choose (forward 4, 8 or 16; backward 4 to 128 rows per row block),
+launches choose (forward 4, 8 or 16; backward 16 to 128 rows per row block, 4 to 128 inside the module),
 at the first and last row counts of each and with partial last blocks,
 against float64.
 

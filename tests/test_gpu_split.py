@@ -100,3 +100,26 @@ def test_split_module_forward(B, L, width, dtype):
     tol = 2e-5 if dtype == torch.float32 else 2.0 ** -7
     for a, b in zip(got["fused"], got["composed"]):
         assert rel_err(a, b) <= tol, rel_err(a, b)
+
+
+@pytest.mark.parametrize("B,L,width,dtype", [
+    (1, 1500, 256, torch.float32),          # time segments
+    (2, 40, 512, torch.bfloat16),           # split chains
+    (8, 70, 32768, torch.bfloat16),         # the wide kernel
+    (1, 100, 32768, torch.float32),         # one wave per chain
+])
+def test_forward_without_gradients_matches(B, L, width, dtype):
+    """The forward that keeps no states gives the same bits as the one that
+    does, with gradients switched off and with nothing that requires them."""
+    print(f"[case] no-gradient forward B={B} L={L} width={width} {dtype}", flush=True)
+    torch.manual_seed(L)
+    m = sparc_amd.SPARCMixer(width).cuda()
+    x = torch.randn(B, L, width, device="cuda").to(dtype)
+    y, last = m(x, return_cache=True)
+    assert y.requires_grad
+    with torch.no_grad():
+        y1, last1 = m(x, return_cache=True)
+    m.requires_grad_(False)
+    y2, last2 = m(x, return_cache=True)
+    for a, b, c in zip((y, *last), (y1, *last1), (y2, *last2)):
+        assert torch.equal(a, b) and torch.equal(a, c) and not b.requires_grad
