@@ -94,7 +94,8 @@ template <typename IO> constexpr bool kRoundWrite = SPARC_MIXER_ROUND_WRITE && s
 //            mixer_bwd_kernel.
 enum : int { kModule = 0, kPlanes = 1, kRelu = 2, kReset = 4, kCoop = 8, kNoSave = 16 };
 constexpr int kStateChunk = 64;  // steps per saved chunk state (sparc_scan_chunk_length)
-constexpr int kSplitWaves = 16;  // most waves per workgroup of the split-chain kernels
+constexpr int kSplitWaves = 16;  // most waves per workgroup of the split-chain forward
+constexpr int kSplitBwdWaves = 8;  // and of its backward
 // A lane byte offset past every buffer resource of these kernels (each spans
 // less than 2^31 bytes): the hardware range check drops a store through it.
 // Lanes that must not store (past M) store through it, so that no store
@@ -1918,6 +1919,450 @@ mixer_bwd_kernel(Args a) {
 }
 
 // ---------------------------------------------------------------------------
+// backward over split chains (mixer_fwd_split_kernel's decomposition)
+// ---------------------------------------------------------------------------
+// Rounds of NW * S steps in reverse time; wave w of a round holds steps [w S,
+// (w + 1) S): its transitions, its map of the adjoint X -> P X + Q over them
+// (P the product of conj(a), Q from the relu-masked dy), one exchange of the
+// maps in LDS, and from the adjoint entering its steps the gradients, as
+// mixer_bwd_kernel forms them.  The adjoint crosses rounds as the first wave
+// left it.  Where the one-wave kernel splits time into segments it pays for a
+// summary pass over the transitions and dy instead.
+//   kModule, kPlanes: the states are read back (h_re, h_im).
+//   kRelu: the relu output's backward, whose states nobody saved: each round
+//     starts from its chunk state and recomputes them in fp32 from the writes
+//     (the forward's map, exchange and replay in front of the adjoint's), so
+//     NW * S must be a multiple of kStateChunk.
+template <typename IO, int V, int S, int MODE>
+__global__ void __launch_bounds__(64 * kSplitBwdWaves)
+mixer_bwd_split_kernel(Args a) {
+  using RawT = typename Raw<IO, V>::T;
+  constexpr int ESZ = sizeof(IO);
+  constexpr int MB = 64 * V;
+  constexpr int CM = MODE & 3;             // the chain mode without kReset
+  constexpr bool RST = (MODE & kReset) != 0;
+  constexpr bool MOD = CM == kModule;      // x, the write's backward, the relu mask from h
+  constexpr bool REC = CM == kRelu;        // recomputed states, the relu mask from them
+  constexpr int HS = MOD ? S + 1 : S;      // rows of h: steps t0-1 .. (the module's mask: up to t0+S-1)
+  constexpr int NP = MOD ? 5 : 2;          // per-mode sums
+  static_assert(!MOD || !RST, "resets in the P1 scan only");
+  // the adjoint's maps [2][NW - 1][V][64] (kRelu, with its two barriers per
+  // round: one buffer of them and one of the states' maps); [2][V][64] float2
+  // adjoints entering a round; at the end the per-mode sums [NW][NP][V][64]
+  extern __shared__ float4 split_lds[];
+  __shared__ float4 tok[kSplitBwdWaves][S];  // a wave's per-step values
+  const int NW = static_cast<int>(blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int n_map = (NW - 1) * V * 64;
+  float2* adj = reinterpret_cast<float2*>(split_lds + 2 * n_map);
+  const ChainPos cp = chain_pos(a);
+  const int b = cp.b, mb = cp.mb, T = a.T;
+  const int m0 = mb * MB + lane * V;
+  const bool lane_ok = m0 < a.M;  // the host requires M % V == 0
+  const int64_t R = static_cast<int64_t>(a.B) * T;
+  const int64_t row0 = static_cast<int64_t>(b) * T;
+  const int64_t mbase = static_cast<int64_t>(mb) * MB;
+  const int64_t bm0 = static_cast<int64_t>(b) * a.M + m0;
+  const int64_t W = 2 * static_cast<int64_t>(a.M);
+  const uint32_t lane_bytes = static_cast<uint32_t>(lane * V * ESZ);
+  const uint32_t lane_ld = lane_ok ? lane_bytes : 0u;
+  const uint32_t lane_st = lane_ok ? lane_bytes : kDropOffset;
+  // bytes of one row of x / dy / dx (2M) and of h / w (M) (< 2^31: the host limits M to 2^24)
+  const uint32_t row_x = static_cast<uint32_t>(W * ESZ), half_x = static_cast<uint32_t>(a.M * ESZ);
+  const int64_t n_chunks = (T + kStateChunk - 1) / kStateChunk;
+  ModeConsts<V, true> mc;
+  mc.load(a.consts, m0, lane_ok);
+  float acc[NP][V];      // nu_log, theta_log and (module) wlg, wpr, wrr
+  float h0r[V], h0i[V];  // the state before step 0 (the P1 scan's caller's, else zero)
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) acc[p][v] = 0.0f;
+    const bool h0 = !MOD && lane_ok && a.h0_re != nullptr;
+    h0r[v] = h0 ? a.h0_re[bm0 + v] : 0.0f;
+    h0i[v] = h0 ? a.h0_im[bm0 + v] : 0.0f;
+    if (wave == 0)  // the adjoint entering the last round
+      adj[v * 64 + lane] = make_float2(lane_ok && a.dlast_re ? a.dlast_re[bm0 + v] : 0.0f,
+                                       lane_ok && a.dlast_im ? a.dlast_im[bm0 + v] : 0.0f);
+  }
+  wait_vm_all();  // the loop-carried values above, before the first prefetch
+
+  RawT dr[2][S], di[2][S];                              // dy
+  RawT xr[2][REC || MOD ? S : 1], xi[2][REC || MOD ? S : 1];  // module: x; kRelu: the writes
+  RawT pr[2][REC ? 1 : HS], pi[2][REC ? 1 : HS];        // the states from step t0-1
+  float cs[2][REC ? 2 * V : 1];                         // kRelu: the state entering the round
+  float ev[2], dv[2];
+  int kv[2];  // RST: lane s < S: whether step s keeps its transition
+  // this wave's rows of round k; rows outside [0, T) read the nearest one
+  // inside (no loads under a branch)
+  auto load_rows = [&](auto h_tag, int k) __attribute__((always_inline)) {
+    constexpr int h = decltype(h_tag)::value;
+    const int t0 = (k * NW + wave) * S;
+    const int tb = min(t0, T - 1), hb = min(max(t0 - 1, 0), T - 1);
+    const int64_t xoff = wave_uniform(((row0 + tb) * W + mbase) * ESZ);
+    const int64_t woff = wave_uniform(((row0 + tb) * a.M + mbase) * ESZ);
+    const int64_t poff = wave_uniform(((row0 + hb) * a.M + mbase) * ESZ);
+    // dy: [B,T,2M] (the module, the relu output) or the planes dy_re, dy_im
+    constexpr bool CAT = MOD || REC;
+    const uint32_t row_d = CAT ? row_x : half_x;
+    const __amdgpu_buffer_rsrc_t rdr = make_rsrc(static_cast<const char*>(a.dy) + (CAT ? xoff : woff), S * row_d);
+    const __amdgpu_buffer_rsrc_t rdi =
+        CAT ? rdr : make_rsrc(static_cast<const char*>(a.dy_im) + woff, S * row_d);
+    const __amdgpu_buffer_rsrc_t rxr = MOD ? make_rsrc(static_cast<const char*>(a.x) + xoff, S * row_x)
+                                           : make_rsrc(static_cast<const char*>(a.w_re) + woff, S * half_x);
+    const __amdgpu_buffer_rsrc_t rxi =
+        MOD ? rxr : make_rsrc(static_cast<const char*>(a.w_im) + woff, S * half_x);
+    const __amdgpu_buffer_rsrc_t rpr = make_rsrc(static_cast<const char*>(a.h_re) + poff, HS * half_x);
+    const __amdgpu_buffer_rsrc_t rpi = make_rsrc(static_cast<const char*>(a.h_im) + poff, HS * half_x);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t rel = static_cast<uint32_t>(min(t0 + s, T - 1) - tb);
+      dr[h][s] = buf_load<RawT, CPOL_NT>(rdr, lane_ld, rel * row_d);
+      di[h][s] = buf_load<RawT, CPOL_NT>(rdi, lane_ld, rel * row_d + (CAT ? half_x : 0u));
+      if constexpr (MOD || REC) {
+        const uint32_t o = rel * (MOD ? row_x : half_x);
+        xr[h][s] = buf_load<RawT, CPOL_NT>(rxr, lane_ld, o);
+        xi[h][s] = buf_load<RawT, CPOL_NT>(rxi, lane_ld, o + (MOD ? half_x : 0u));
+      }
+    }
+    if constexpr (!REC) {
+#pragma unroll
+      for (int j = 0; j < HS; ++j) {
+        const uint32_t o = static_cast<uint32_t>(min(max(t0 - 1 + j, 0), T - 1) - hb) * half_x;
+        pr[h][j] = buf_load<RawT, CPOL_NT>(rpr, lane_ld, o);
+        pi[h][j] = buf_load<RawT, CPOL_NT>(rpi, lane_ld, o);
+      }
+    } else {
+      // the state before the round: the chunk state that ends there, or
+      // nothing for the first round (an empty range reads zeros; h0 is added)
+      const int c = k * NW * S / kStateChunk - 1;
+      const int64_t off = wave_uniform(((static_cast<int64_t>(b) * n_chunks + max(c, 0)) * a.M + mbase) * 8);
+      const __amdgpu_buffer_rsrc_t rc =
+          make_rsrc(reinterpret_cast<const char*>(a.chunk_state) + off, c >= 0 ? MB * 8u : 0u);
+      buffer_load_f32<2 * V, CPOL_DEFAULT>(rc, lane_ok ? static_cast<uint32_t>(lane * V * 8) : 0u, cs[h]);
+    }
+    const int tl = min(t0 + (lane & (S - 1)), T - 1);
+    ev[h] = a.eta[row0 + tl];
+    dv[h] = a.delta[row0 + tl];
+    if constexpr (RST) kv[h] = p1_keep(a, b, tl);
+  };
+
+  // round k, the (n+1)-th processed (n & 1: the LDS buffers); TAIL: the round
+  // that holds T, with steps past T (nothing) and waves past T (the identity)
+  auto round = [&](auto h_tag, int k, int n, auto tail_tag) __attribute__((always_inline)) {
+    constexpr int h = decltype(h_tag)::value;
+    constexpr bool TAIL = decltype(tail_tag)::value;
+    const int t0 = (k * NW + wave) * S;
+    float4* maps = split_lds + (REC ? 0 : n & 1) * n_map;
+    load_rows(std::integral_constant<int, 1 - h>{}, max(k - 1, 0));
+    wave_lds_fence();
+    tok[wave][lane & (S - 1)] = make_float4(fast_exp(ev[h]), dv[h], dv[h] * kNegInv2Pi, ev[h]);
+    wave_lds_fence();
+    float Es[S], Ds[S], Rs[S], Hs[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const float4 t4 = tok[wave][s];
+      Es[s] = t4.x;
+      Ds[s] = t4.y;
+      Rs[s] = t4.z;
+      Hs[s] = t4.w;
+    }
+    float qar[S][V], qai[S][V], qem[S][V];
+    p1_block_transitions<IO, MODE, S, V>(mc, Es, Ds, Rs, qar, qai, qem);
+    if constexpr (RST) p1_block_resets<S, V>(kv[h], qar, qai);
+    float Pr[V], Pi[V];  // the product of this wave's conj(a)
+#pragma unroll
+    for (int v = 0; v < V; ++v) { Pr[v] = 1.0f; Pi[v] = 0.0f; }
+    // kRelu: the states before each step, and whether each output passed the relu
+    float hpr[REC ? S : 1][V], hpi[REC ? S : 1][V];
+    uint32_t up = 0;  // bit 2 (s V + v): re of step s, mode v; the next bit: im
+    if constexpr (REC) {
+      float4* fm = split_lds + n_map;
+      float Qr[V], Qi[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) { Qr[v] = 0.0f; Qi[v] = 0.0f; }
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if (TAIL && t0 + s >= T) break;  // wave-uniform
+        float wr[V], wi[V];
+        unpack<IO, V>(xr[h][s], wr);
+        unpack<IO, V>(xi[h][s], wi);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const float qr = fmaf(qar[s][v], Qr[v], fmaf(-qai[s][v], Qi[v], wr[v]));
+          Qi[v] = fmaf(qai[s][v], Qr[v], fmaf(qar[s][v], Qi[v], wi[v]));
+          Qr[v] = qr;
+          const float p2 = fmaf(qar[s][v], Pr[v], qai[s][v] * Pi[v]);
+          Pi[v] = fmaf(qar[s][v], Pi[v], -qai[s][v] * Pr[v]);
+          Pr[v] = p2;
+        }
+      }
+      if (wave < NW - 1) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) fm[(wave * V + v) * 64 + lane] = make_float4(Pr[v], -Pi[v], Qr[v], Qi[v]);
+      }
+      __syncthreads();
+      float hr[V], hi[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        hr[v] = cs[h][2 * v] + (k == 0 ? h0r[v] : 0.0f);
+        hi[v] = cs[h][2 * v + 1] + (k == 0 ? h0i[v] : 0.0f);
+      }
+      for (int j = 0; j < wave; ++j) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const float4 e = fm[(j * V + v) * 64 + lane];
+          const float nr = fmaf(e.x, hr[v], fmaf(-e.y, hi[v], e.z));
+          hi[v] = fmaf(e.x, hi[v], fmaf(e.y, hr[v], e.w));
+          hr[v] = nr;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        float wr[V], wi[V];
+        unpack<IO, V>(xr[h][s], wr);
+        unpack<IO, V>(xi[h][s], wi);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          hpr[s][v] = hr[v];
+          hpi[s][v] = hi[v];
+          const float nr = fmaf(qar[s][v], hr[v], fmaf(-qai[s][v], hi[v], wr[v]));
+          const float ni = fmaf(qai[s][v], hr[v], fmaf(qar[s][v], hi[v], wi[v]));
+          hr[v] = nr;
+          hi[v] = ni;
+          up |= (nr > 0.0f ? 1u : 0u) << (2 * (s * V + v));
+          up |= (ni > 0.0f ? 1u : 0u) << (2 * (s * V + v) + 1);
+        }
+      }
+    }
+    // dy of step s behind the relu
+    auto masked_dy = [&](int s, float (&gyr)[V], float (&gyi)[V]) __attribute__((always_inline)) {
+      unpack<IO, V>(dr[h][s], gyr);
+      unpack<IO, V>(di[h][s], gyi);
+      if constexpr (MOD) {  // h_t > 0: the row after the step's own
+        float mr[V], mi[V];
+        unpack<IO, V>(pr[h][s + 1], mr);
+        unpack<IO, V>(pi[h][s + 1], mi);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          gyr[v] = mr[v] > 0.0f ? gyr[v] : 0.0f;
+          gyi[v] = mi[v] > 0.0f ? gyi[v] : 0.0f;
+        }
+      } else if constexpr (REC) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          gyr[v] = (up >> (2 * (s * V + v))) & 1u ? gyr[v] : 0.0f;
+          gyi[v] = (up >> (2 * (s * V + v) + 1)) & 1u ? gyi[v] : 0.0f;
+        }
+      }
+    };
+    if (wave > 0) {  // the adjoint's map (nobody reads the first wave's)
+      float Qr[V], Qi[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) { Qr[v] = 0.0f; Qi[v] = 0.0f; }
+#pragma unroll
+      for (int s = S - 1; s >= 0; --s) {
+        if (TAIL && t0 + s >= T) continue;  // wave-uniform
+        float gyr[V], gyi[V];
+        masked_dy(s, gyr, gyi);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const float l_r = gyr[v] + Qr[v], l_i = gyi[v] + Qi[v];
+          Qr[v] = fmaf(qar[s][v], l_r, qai[s][v] * l_i);
+          Qi[v] = fmaf(qar[s][v], l_i, -qai[s][v] * l_r);
+          if constexpr (!REC) {
+            const float p2 = fmaf(qar[s][v], Pr[v], qai[s][v] * Pi[v]);
+            Pi[v] = fmaf(qar[s][v], Pi[v], -qai[s][v] * Pr[v]);
+            Pr[v] = p2;
+          }
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+        maps[((wave - 1) * V + v) * 64 + lane] = make_float4(Pr[v], Pi[v], Qr[v], Qi[v]);
+    }
+    __syncthreads();
+    float Xr[V], Xi[V];  // conj(a_{t+1}) lambda_{t+1}
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const float2 x0 = adj[((n & 1) * V + v) * 64 + lane];
+      Xr[v] = x0.x;
+      Xi[v] = x0.y;
+    }
+    for (int j = NW - 1; j > wave; --j) {  // the maps of the waves after this one in time
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const float4 e = maps[((j - 1) * V + v) * 64 + lane];
+        const float nr = fmaf(e.x, Xr[v], fmaf(-e.y, Xi[v], e.z));
+        Xi[v] = fmaf(e.x, Xi[v], fmaf(e.y, Xr[v], e.w));
+        Xr[v] = nr;
+      }
+    }
+    // the gradients (mixer_bwd_kernel's, with the same names)
+    RawT dwr[S], dwi[S];  // dw, or the module's dx
+    float e[2 * S];
+#pragma unroll
+    for (int s = S - 1; s >= 0; --s) {
+      if (TAIL && t0 + s >= T) {  // wave-uniform: no such step
+        e[2 * s] = 0.0f;
+        e[2 * s + 1] = 0.0f;
+        continue;
+      }
+      float gyr[V], gyi[V], hr[V], hi[V], outr[V], outi[V];
+      masked_dy(s, gyr, gyi);
+      if constexpr (REC) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) { hr[v] = hpr[s][v]; hi[v] = hpi[s][v]; }
+      } else {
+        unpack<IO, V>(pr[h][s], hr);
+        unpack<IO, V>(pi[h][s], hi);
+        if (s == 0) {  // the state before step 0: selects, not a branch
+          const bool first = t0 == 0;
+#pragma unroll
+          for (int v = 0; v < V; ++v) {
+            hr[v] = first ? h0r[v] : hr[v];
+            hi[v] = first ? h0i[v] : hi[v];
+          }
+        }
+      }
+      const float E = Es[s], delta = Ds[s];
+      float se = 0.0f, sd = 0.0f, cxr[V], cxi[V];
+      if constexpr (MOD) {
+        unpack<IO, V>(xr[h][s], cxr);
+        unpack<IO, V>(xi[h][s], cxi);
+      }
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const float l_r = gyr[v] + Xr[v], l_i = gyi[v] + Xi[v];
+        const float xr1 = fmaf(qar[s][v], l_r, qai[s][v] * l_i);
+        const float xi1 = fmaf(qar[s][v], l_i, -qai[s][v] * l_r);
+        Xr[v] = xr1;
+        Xi[v] = xi1;
+        const float zr = fmaf(xr1, hr[v], xi1 * hi[v]);   // Re Z
+        const float zi = fmaf(xi1, hr[v], -xr1 * hi[v]);  // Im Z = dphi
+        const float em = qem[s][v];
+        const float tt = fmaf(fmaf(em, delta, delta), zi, -zr);  // rho delta dphi - Re Z
+        if constexpr (!MOD) {
+          outr[v] = l_r;
+          outi[v] = l_i;
+          const float u = mc.nu[v] * tt;  // radial / E
+          se += u;
+          sd = fmaf(-em, zi, sd);
+          acc[0][v] = fmaf(E, u, acc[0][v]);
+          acc[1][v] += zi;
+        } else {
+          const float e2 = fmaf(em, em, em + em);
+          const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(fmaf(delta, mc.pl[v], Hs[s] * mc.rl[v])));
+          const float Y = mc.g2[v] * e2, r = __builtin_amdgcn_rsqf(fmaxf(Y, 1e-30f));
+          const float gain = Y * r * sg;
+          const float tr = tanh_fast(cxr[v]), ti = tanh_fast(cxi[v]);
+          float w_r = l_r, w_i = l_i;
+          if constexpr (kRoundWrite<IO>) round_bf16x2(w_r, w_i);
+          const float wgr = w_r * gain, wgi = w_i * gain;
+          outr[v] = wgr * fmaf(-tr, tr, 1.0f);
+          outi[v] = wgi * fmaf(-ti, ti, 1.0f);
+          const float g = fmaf(wgr, tr, wgi * ti);
+          const float ue = (mc.nu[v] * E) * fmaf(-g, fmaf(mc.g2[v], r * r, 1.0f), tt);
+          const float gs = g * (1.0f - sg);
+          se = fmaf(gs, mc.wrr_s[v], se + ue);
+          sd = fmaf(-em, zi, fmaf(gs, mc.wpr_s[v], sd));
+          acc[0][v] += ue;
+          acc[1][v] += zi;
+          acc[2][v] += g;
+          acc[3][v] = fmaf(gs, delta, acc[3][v]);
+          acc[4][v] = fmaf(gs, Hs[s], acc[4][v]);
+        }
+      }
+      dwr[s] = pack<IO, V>(outr);
+      dwi[s] = pack<IO, V>(outi);
+      // lanes past M: finite zeros from their zero constants, kept exact in the module
+      e[2 * s] = MOD ? (lane_ok ? se : 0.0f) : se * E;
+      e[2 * s + 1] = !MOD || lane_ok ? sd : 0.0f;
+    }
+    if (wave == 0) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) adj[((1 - (n & 1)) * V + v) * 64 + lane] = make_float2(Xr[v], Xi[v]);
+    }
+    {
+      const int ts = TAIL ? min(t0, T - 1) : t0;
+      const int64_t xoff = wave_uniform(((row0 + ts) * W + mbase) * ESZ);
+      const int64_t woff = wave_uniform(((row0 + ts) * a.M + mbase) * ESZ);
+      const uint32_t row_o = MOD ? row_x : half_x;
+      const __amdgpu_buffer_rsrc_t ror = make_rsrc(static_cast<char*>(a.dx) + (MOD ? xoff : woff), S * row_o);
+      const __amdgpu_buffer_rsrc_t roi = MOD ? ror : make_rsrc(static_cast<char*>(a.dw_im) + woff, S * row_o);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if (TAIL && t0 + s >= T) break;  // wave-uniform
+        buf_store<RawT, CPOL_NT>(dwr[s], ror, lane_st, static_cast<uint32_t>(s) * row_o);
+        buf_store<RawT, CPOL_NT>(dwi[s], roi, lane_st, static_cast<uint32_t>(s) * row_o + (MOD ? half_x : 0u));
+      }
+    }
+    // the wave sums of the per-token values, as mixer_bwd_kernel stores them
+    wave_sums_to_leaders<2 * S>(e);
+    constexpr int K = 2 * S >= 16 ? 2 * S / 16 : 1, G = 64 * K / (2 * S);
+    const uint32_t nb = static_cast<uint32_t>(TAIL ? max(min(S, T - t0), 0) : S) * 4u;
+    const int tc = TAIL ? min(t0, T - 1) : t0;
+    const int64_t o0 = wave_uniform((static_cast<int64_t>(mb) * R + row0 + tc) * 4);
+    const int64_t o1 = wave_uniform(((static_cast<int64_t>(a.n_mb) + mb) * R + row0 + tc) * 4);
+    const __amdgpu_buffer_rsrc_t rt0 = make_rsrc(reinterpret_cast<char*>(a.part_tok) + o0, nb);
+    const __amdgpu_buffer_rsrc_t rt1 = make_rsrc(reinterpret_cast<char*>(a.part_tok) + o1, nb);
+    const bool lead = lane % G == 0;
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+      const int i = lane / G * K + q;
+      const uint32_t off = static_cast<uint32_t>(i >> 1) * 4u;
+      const float v[1] = {e[q]};
+      buffer_store_f32<1, CPOL_DEFAULT>(rt0, lead && !(i & 1) ? off : kDropOffset, v);
+      buffer_store_f32<1, CPOL_DEFAULT>(rt1, lead && (i & 1) ? off : kDropOffset, v);
+    }
+    if constexpr (!MOD) {  // the gradient of the initial state: conj(a_0) lambda_0
+      if (t0 == 0 && a.dh0_re && lane_ok) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          a.dh0_re[bm0 + v] = Xr[v];
+          a.dh0_im[bm0 + v] = Xi[v];
+        }
+      }
+    }
+  };
+  const int n_full = T / (NW * S);
+  int k = n_full - 1, n = 0;
+  if (n_full * NW * S < T) {
+    load_rows(std::integral_constant<int, 1>{}, n_full);
+    round(std::integral_constant<int, 1>{}, n_full, n++, std::true_type{});
+  } else {
+    load_rows(std::integral_constant<int, 0>{}, k);
+  }
+  // registers [0] hold round k here; rounds in pairs, so that every buffer
+  // index is a compile-time constant
+  for (; k >= 0; k -= 2) {
+    round(std::integral_constant<int, 0>{}, k, n++, std::false_type{});
+    if (k >= 1) round(std::integral_constant<int, 1>{}, k - 1, n++, std::false_type{});
+  }
+  // the per-mode sums over the waves, in wave order
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(split_lds);
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    acc[1][v] *= mc.th[v];  // d theta_log = theta sum dphi
+    if constexpr (MOD) {    // the module's constant factors (mixer_bwd_kernel)
+      acc[0][v] = fmaf(-mc.kappa[v], acc[2][v], acc[0][v]);
+      acc[3][v] *= kTwoOverPi;
+      acc[4][v] *= kInvLog16;
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) red[((wave * NP + p) * V + v) * 64 + lane] = acc[p][v];
+  }
+  __syncthreads();
+  for (int q = wave; q < NP * V; q += NW) {  // sum p = q / V, mode v = q % V of every lane
+    float sum = 0.0f;
+    for (int j = 0; j < NW; ++j) sum += red[(j * NP * V + q) * 64 + lane];
+    if (lane_ok) a.part_mode[(static_cast<int64_t>(q / V) * a.B + b) * a.M + m0 + q % V] = sum;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // carries across time segments
 // ---------------------------------------------------------------------------
 // Each segment maps the state entering it to the state leaving it, h -> P h + Q
@@ -2252,6 +2697,56 @@ int split_waves(int64_t B, int64_t T, int64_t M) {
   if (T < kSplitMinSteps) return 0;
   return chains >= 512 ? 4 : chains >= 192 ? 8 : kSplitWaves;
 }
+// The split backward: waves per chain and modes per lane, or waves 0 (the
+// other forms).  Steps of a round per wave: 4 in the module (bf16 2 modes per
+// lane 186 VGPRs, two workgroups of 4 waves per CU; 1 mode 133, three), 8 in
+// the P1 scan.  Measured (us per training step, bf16 unless said, n chains of
+// 128 modes, before -> split):
+//   module, T=2048: n = 128 497 -> 558, 192 653 -> 634, 256 780 -> 687, 384
+//     1255 -> 1182 (1 mode per lane: 1117), 448 1385 -> 1233, 512 1862 ->
+//     1301, 640 2032 -> 1790 (1 mode: 1716), 768 2090 -> 1986; 1024 2350 ->
+//     2567 (the one-launch form stays).  One mode per lane where the
+//     workgroups of 2 would leave a CU's second place empty on most CUs.
+//     fp32: 128 727 -> 678, 384 2090 -> 1848; 512 2065 -> 2304
+//   P1 scan, T=2048: 128 230 -> 251, 192 304 -> 293, 384 557 -> 495, 512 668
+//     -> 556, 1024 1248 -> 1129, 2048 (T=1024) 1250 -> 1181; fp32: 128 347 ->
+//     316, 512 1150 -> 1016, 768 1736 -> 1520, 1024 2034 -> 2069
+//   relu output (recomputing, against the general kernels): T=2048: 96 345 ->
+//     279 or less (the host's time), 128 421 -> 278, 384 1100 -> 556, 2048
+//     (T=1024) 4200 -> 1460; 16 chains, T=4096 185 -> 298
+// As in the forward, with few chains only short sequences are split, and with
+// many nothing below kSplitMinSteps is.
+struct SplitBwd {
+  int waves = 0, V = 1;
+};
+// controls: the whole module backward, which from 512 chains on has the
+// one-launch form; up to this many steps it keeps that form there, as
+// sparc_mixer_backward_form has always reported for such shapes.
+constexpr int64_t kCoopKeepSteps = 1024;
+constexpr int kReluBwdWaves = 8;  // 8 steps each: a round is a saved-state chunk
+SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int cm, bool controls = false) {
+  const int64_t n = B * ((M + 127) / 128);
+  const bool bf = io == SPARC_BF16, few = T >= 16 && T <= kSplitFewSteps;
+  SplitBwd r;
+  if (cm == kRelu) {
+    if (n >= 64 || few) r.waves = kReluBwdWaves;
+    return r;
+  }
+  r.V = bf ? 2 : 1;
+  if (n < kSplitChains) {
+    if (few) r.waves = static_cast<int>(std::min<int64_t>(kSplitBwdWaves, (T + 3) / 4));
+    return r;
+  }
+  if (T < kSplitMinSteps || (bf && n < 192)) return r;
+  if (cm == kModule) {
+    if (n > (bf ? 768 : 511) || (controls && n >= 512 && T <= kCoopKeepSteps)) return r;
+    if (bf && n > 256 && (n - 1) % 256 < 128) r.V = 1;
+    r.waves = !bf || n <= 256 ? 8 : 4;
+  } else if (bf || n < 1024) {
+    r.waves = n >= 1024 ? 4 : 8;
+  }
+  return r;
+}
 struct Layout {
   bool piped = false;
   int split = 0;  // waves per chain of the split-chain kernels (0: not taken)
@@ -2261,14 +2756,14 @@ struct Layout {
 };
 
 // gw: the P1 scan with the writes given (no controls, two per-mode gradients);
-// pieces: the module backward in time pieces where the shape allows;
-// allow_split: the split-chain kernels where the shape takes them
-Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, bool pieces = false,
-              bool allow_split = true) {
+// pieces: the module backward in time pieces where the shape allows; split:
+// waves per chain of the split-chain kernels, of split_v modes per lane
+Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, bool pieces = false, int split = 0,
+              int split_v = kSplitV) {
   Layout l;
   l.V = mixer_v(B, T, M, direction, gw);
-  l.split = allow_split && direction == 0 ? split_waves(B, T, M) : 0;
-  if (l.split) l.V = kSplitV;
+  l.split = split;
+  if (l.split) l.V = split_v;
   l.n_mb = static_cast<int>((M + 64 * l.V - 1) / (64 * l.V));
   if (l.split) l.t_seg = static_cast<int>(T);
   else choose_segments(B, T, l.n_mb, l.n_seg, l.t_seg);
@@ -2278,7 +2773,7 @@ Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, b
   l.rb_rows = cl.rows;
   int np = kPieces;
   while (np > 1 && T % (static_cast<int64_t>(np) * kCtrlBwdRows) != 0) np /= 2;
-  if (pieces && np > 1 && T > 0 && direction == 1 && !gw && l.n_seg == 1 && l.V == 1) {
+  if (pieces && !split && np > 1 && T > 0 && direction == 1 && !gw && l.n_seg == 1 && l.V == 1) {
     l.piped = true;
     l.n_seg = np;
     l.t_seg = static_cast<int>(T / np);
@@ -2439,9 +2934,18 @@ bool fwd_wide(const Layout& l, int64_t batch, int64_t modes, bool module = false
 // The forward's layout: split chains unless the wide kernel is the faster one
 // there (the P1 scan and the fp32 module with many chains, see split_waves).
 Layout forward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, bool gw) {
-  const Layout l = layout(batch, length, modes, 0, gw, false, false);
+  const Layout l = layout(batch, length, modes, 0, gw);
   if ((gw || io_dtype == SPARC_F32) && fwd_wide(l, batch, modes, !gw)) return l;
-  return layout(batch, length, modes, 0, gw);
+  const int nw = split_waves(batch, length, modes);
+  return nw ? layout(batch, length, modes, 0, gw, false, nw) : l;
+}
+// The backward's, for chain mode cm (kRelu: split, or not there at all);
+// controls: the whole module backward (its time pieces, split_bwd).
+Layout backward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, int cm,
+                       bool controls = false) {
+  const SplitBwd sp = split_bwd(batch, length, modes, io_dtype, cm, controls);
+  if (!sp.waves) return layout(batch, length, modes, 1, cm != kModule, controls);
+  return layout(batch, length, modes, 1, cm != kModule, false, sp.waves, sp.V);
 }
 
 // the split forward: l.split waves per chain
@@ -2473,6 +2977,27 @@ void run_fwd_module(const Layout& l, Args a, bool bf, hipStream_t st) {
     if (l.V == 2) run_fwd<sparc::bf16, 2, MODE>(a, st); else run_fwd<sparc::bf16, 1, MODE>(a, st);
   } else {
     if (l.V == 2) run_fwd<float, 2, MODE>(a, st); else run_fwd<float, 1, MODE>(a, st);
+  }
+}
+
+// the split backward: l.split waves per chain, l.V modes per lane
+template <typename IO, int V, int MODE>
+void launch_bwd_split(const Args& a, int nw, hipStream_t st) {
+  constexpr int S = (MODE & 3) == kModule ? 4 : 8;
+  static_assert((MODE & 3) != kRelu || S * kReluBwdWaves % kStateChunk == 0, "rounds start on saved states");
+  const dim3 g(static_cast<unsigned>(a.B) * static_cast<unsigned>(a.n_mb)), blk(64 * static_cast<unsigned>(nw));
+  const size_t lds = static_cast<size_t>(2) * (nw - 1) * V * 64 * 16 + 2 * V * 64 * 8;
+  hipLaunchKernelGGL((mixer_bwd_split_kernel<IO, V, S, MODE>), g, blk, lds, st, a);
+}
+template <int MODE>
+void run_bwd_split(const Args& a, const Layout& l, bool bf, hipStream_t st) {
+  if (!bf) {
+    launch_bwd_split<float, 1, MODE>(a, l.split, st);
+  } else if constexpr ((MODE & 3) == kModule) {
+    if (l.V == 2) launch_bwd_split<sparc::bf16, 2, MODE>(a, l.split, st);
+    else launch_bwd_split<sparc::bf16, 1, MODE>(a, l.split, st);
+  } else {
+    launch_bwd_split<sparc::bf16, (MODE & 3) == kRelu ? 1 : 2, MODE>(a, l.split, st);
   }
 }
 
@@ -2548,7 +3073,9 @@ sparc_status scan_backward_impl(const Layout& l, int64_t batch, int64_t length, 
   a.n_seg = l.n_seg; a.t_seg = l.t_seg; a.seg_lo = 0;
   a.seg_sum = reinterpret_cast<float*>(ws + l.seg_sum);
   a.seg_state = reinterpret_cast<float*>(ws + l.seg_state);
-  if (io_dtype == SPARC_BF16) {
+  if (l.split) {
+    run_bwd_split<kModule>(a, l, io_dtype == SPARC_BF16, st);
+  } else if (io_dtype == SPARC_BF16) {
     if (l.V == 2) run_bwd<sparc::bf16, 2>(a, st); else run_bwd<sparc::bf16, 1>(a, st);
   } else {
     if (l.V == 2) run_bwd<float, 2>(a, st); else run_bwd<float, 1>(a, st);
@@ -2616,10 +3143,18 @@ bool p1_fused_shape(const sparc_scan_desc* d) {
   return check_shape(d->batch, d->length, d->modes, d->io_dtype) == SPARC_OK;
 }
 
+bool p1_fused_relu_backward(const sparc_scan_desc* d) {
+  return p1_fused_shape(d) && split_bwd(d->batch, d->length, d->modes, d->io_dtype, kRelu).waves != 0;
+}
+
 size_t p1_fused_workspace_bytes(const sparc_scan_desc* d, int direction) {
   if (!p1_fused_shape(d)) return 0;
   if (direction == 0) return forward_layout(d->batch, d->length, d->modes, d->io_dtype, true).total;
-  return layout(d->batch, d->length, d->modes, direction, true).total;
+  // the relu output's backward is the general kernels' where it is not split
+  size_t n = backward_layout(d->batch, d->length, d->modes, d->io_dtype, kPlanes).total;
+  if (p1_fused_relu_backward(d))
+    n = std::max(n, backward_layout(d->batch, d->length, d->modes, d->io_dtype, kRelu).total);
+  return n;
 }
 
 // the launches of one chain mode for the I/O type and modes per lane
@@ -2695,15 +3230,17 @@ sparc_status p1_fused_forward(const sparc_scan_desc* d, const float* eta, const 
 }
 
 sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const float* delta,
-                               const float* nu_log, const float* theta_log, const void* y_re, const void* y_im,
+                               const float* nu_log, const float* theta_log, const void* w_re, const void* w_im,
+                               const void* y_re, const void* y_im, const float* chunk_state,
                                const float* h0_re, const float* h0_im, const int32_t* segment_pos,
                                const void* dy_re, const void* dy_im, const float* dlast_re, const float* dlast_im,
                                void* dw_re, void* dw_im, float* deta, float* ddelta, float* dnu_log,
                                float* dtheta_log, float* dh0_re, float* dh0_im, void* workspace,
                                size_t workspace_bytes, sparc_stream_t stream) {
-  if (!p1_fused_shape(d) || d->length <= 0 || (d->flags & SPARC_FLAG_RELU_OUTPUT))
+  const bool relu = d && (d->flags & SPARC_FLAG_RELU_OUTPUT) != 0;
+  if (!p1_fused_shape(d) || d->length <= 0 || (relu && !p1_fused_relu_backward(d)))
     return fail(SPARC_EINVAL, "p1 fused backward: shape");
-  const Layout l = layout(d->batch, d->length, d->modes, 1, true);
+  const Layout l = backward_layout(d->batch, d->length, d->modes, d->io_dtype, relu ? kRelu : kPlanes);
   if (workspace_bytes < l.total) return fail(SPARC_EWORKSPACE, "workspace too small: %zu < %zu", workspace_bytes, l.total);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
@@ -2719,7 +3256,11 @@ sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const
   a.M = M;
   a.n_mb = l.n_mb;
   a.consts = consts; a.eta = eta; a.delta = delta;
-  a.h_re = const_cast<void*>(y_re); a.h_im = const_cast<void*>(y_im);
+  if (relu) {
+    a.w_re = w_re; a.w_im = w_im; a.chunk_state = const_cast<float*>(chunk_state);
+  } else {
+    a.h_re = const_cast<void*>(y_re); a.h_im = const_cast<void*>(y_im);
+  }
   a.dy = dy_re; a.dy_im = dy_im; a.dlast_re = dlast_re; a.dlast_im = dlast_im;
   a.dx = dw_re; a.dw_im = dw_im;
   a.h0_re = h0_re; a.h0_im = h0_im; a.dh0_re = dh0_re; a.dh0_im = dh0_im;
@@ -2730,7 +3271,12 @@ sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const
   a.segpos = segment_pos;
   a.reset_first = (d->flags & SPARC_FLAG_RESET_FIRST) != 0;
   const bool bf = d->io_dtype == SPARC_BF16;
-  if (segment_pos || a.reset_first) run_bwd_mode<kPlanes | kReset>(a, bf, l.V, st);
+  const bool reset = segment_pos || a.reset_first;
+  if (relu && reset) run_bwd_split<kRelu | kReset>(a, l, bf, st);
+  else if (relu) run_bwd_split<kRelu>(a, l, bf, st);
+  else if (l.split && reset) run_bwd_split<kPlanes | kReset>(a, l, bf, st);
+  else if (l.split) run_bwd_split<kPlanes>(a, l, bf, st);
+  else if (reset) run_bwd_mode<kPlanes | kReset>(a, bf, l.V, st);
   else run_bwd_mode<kPlanes>(a, bf, l.V, st);
   // d eta, d delta per token over the mode blocks; d nu_log, d theta_log per
   // mode over the (batch row, segment) partial rows
@@ -3090,10 +3636,12 @@ static sparc_status scan_forward_call(bool save, int64_t batch, int64_t length, 
       !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
     return fail(SPARC_EINVAL, "mixer scan forward: NULL pointer");
   if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer scan forward: last_re/last_im");
-  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
+  Layout l = forward_layout(batch, length, modes, io_dtype, false);
+  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
+  // states aligned for one mode only: the forms that store one mode per lane
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 0);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer scan forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
-  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
   if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(workspace, 256))
     return fail(SPARC_EINVAL, "mixer scan forward: misaligned tensor");
   return scan_forward_impl(l, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
@@ -3115,10 +3663,12 @@ static sparc_status mixer_forward_call(bool save, int64_t batch, int64_t length,
       !params_ok(nu_log, theta_log, write_log_gain, write_phase_response, write_radial_response))
     return fail(SPARC_EINVAL, "mixer forward: NULL pointer");
   if ((last_re == nullptr) != (last_im == nullptr)) return fail(SPARC_EINVAL, "mixer forward: last_re/last_im");
-  const Layout l = forward_layout(batch, length, modes, io_dtype, false);
+  Layout l = forward_layout(batch, length, modes, io_dtype, false);
+  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
+  // states aligned for one mode only: the forms that store one mode per lane
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 0);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
-  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
   if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(phase_direction, 16) ||
       !al(radial_direction, 16) || !al(workspace, 256))
     return fail(SPARC_EINVAL, "mixer forward: misaligned tensor");
@@ -3141,9 +3691,12 @@ size_t sparc_mixer_workspace_bytes(int64_t batch, int64_t length, int64_t modes,
   if (batch <= 0 || length < 0 || modes <= 0 || modes % 4 || (direction != 0 && direction != 1)) return 0;
   // every form either I/O type may take: chains split or not, and the module
   // backward in time pieces or in one launch
-  size_t n = std::max(layout(batch, length, modes, direction).total, layout(batch, length, modes, direction, false, true).total);
-  n = std::max(n, layout(batch, length, modes, direction, false, false, false).total);
-  if (direction == 1) n = std::max(n, coop_layout(batch, length, modes, kCoopS).total);
+  size_t n = layout(batch, length, modes, direction).total;
+  for (const int32_t io : {SPARC_F32, SPARC_BF16})
+    n = std::max(n, direction == 0 ? forward_layout(batch, length, modes, io, false).total
+                                   : backward_layout(batch, length, modes, io, kModule, true).total);
+  if (direction == 1)
+    n = std::max({n, layout(batch, length, modes, 1, false, true).total, coop_layout(batch, length, modes, kCoopS).total});
   return n;
 }
 
@@ -3154,8 +3707,9 @@ int sparc_mixer_backward_plan(int plan) {
 
 int sparc_mixer_backward_form(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype) {
   if (check_shape(batch, length, modes, io_dtype)) return -1;
-  if (coop_steps(batch, length, modes, io_dtype)) return 2;
-  return layout(batch, length, modes, 1, false, true).piped ? 1 : 0;
+  const Layout l = backward_layout(batch, length, modes, io_dtype, kModule, true);
+  if (!l.split && coop_steps(batch, length, modes, io_dtype)) return 2;
+  return l.piped ? 1 : 0;
 }
 
 sparc_status sparc_mixer_scan_forward(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype,
@@ -3219,10 +3773,11 @@ sparc_status sparc_mixer_scan_backward(int64_t batch, int64_t length, int64_t mo
       !params_ok(dnu_log, dtheta_log, dwrite_log_gain, dwrite_phase_response, dwrite_radial_response))
     return fail(SPARC_EINVAL, "mixer scan backward: NULL pointer");
   if ((dlast_re == nullptr) != (dlast_im == nullptr)) return fail(SPARC_EINVAL, "mixer scan backward: dlast_re/dlast_im");
-  const Layout l = layout(batch, length, modes, 1);
+  Layout l = backward_layout(batch, length, modes, io_dtype, kModule);
+  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 1);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer scan backward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
-  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
   if (!al(x, 16) || !al(dy, 16) || !al(dx, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(workspace, 256))
     return fail(SPARC_EINVAL, "mixer scan backward: misaligned tensor");
   return scan_backward_impl(l, batch, length, modes, io_dtype, x, eta, delta, nu_log, theta_log, write_log_gain,
@@ -3249,12 +3804,13 @@ sparc_status sparc_mixer_backward(int64_t batch, int64_t length, int64_t modes, 
       !params_ok(dnu_log, dtheta_log, dwrite_log_gain, dwrite_phase_response, dwrite_radial_response))
     return fail(SPARC_EINVAL, "mixer backward: NULL pointer");
   if ((dlast_re == nullptr) != (dlast_im == nullptr)) return fail(SPARC_EINVAL, "mixer backward: dlast_re/dlast_im");
-  const Layout l = layout(batch, length, modes, 1, false, true);
-  const int cs = coop_steps(batch, length, modes, io_dtype);
+  Layout l = backward_layout(batch, length, modes, io_dtype, kModule, true);
+  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 1, false, true);
+  const int cs = l.split ? 0 : coop_steps(batch, length, modes, io_dtype);
   const size_t need = cs ? coop_layout(batch, length, modes, cs).total : l.total;
   if (!workspace || workspace_bytes < need)
     return fail(SPARC_EWORKSPACE, "mixer backward: workspace too small (%zu < %zu)", workspace_bytes, need);
-  const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
   if (!al(x, 16) || !al(dy, 16) || !al(dx, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) ||
       !al(phase_direction, 16) || !al(radial_direction, 16) || !al(workspace, 256))
     return fail(SPARC_EINVAL, "mixer backward: misaligned tensor");

@@ -31,9 +31,17 @@ sparc_status p1_fused_forward(const sparc_scan_desc* d, const float* eta, const 
                               void* y_im, float* chunk_state, void* workspace, size_t workspace_bytes,
                               sparc_stream_t stream);
 
-// Backward from the forward's states y_re, y_im (no relu output).  T > 0.
+// Whether the relu output's backward runs here (p1_fused_backward with
+// SPARC_FLAG_RELU_OUTPUT) rather than on the general kernels.
+bool p1_fused_relu_backward(const sparc_scan_desc* d);
+
+// Backward.  Without the relu output from the forward's states y_re, y_im
+// (w_re, w_im and chunk_state unused); with it dy_re is [B,T,2M], dy_im NULL,
+// and the states are recomputed from the writes and the chunk states (y_re,
+// y_im unused).  T > 0.
 sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const float* delta,
-                               const float* nu_log, const float* theta_log, const void* y_re, const void* y_im,
+                               const float* nu_log, const float* theta_log, const void* w_re, const void* w_im,
+                               const void* y_re, const void* y_im, const float* chunk_state,
                                const float* h0_re, const float* h0_im, const int32_t* segment_pos,
                                const void* dy_re, const void* dy_im, const float* dlast_re, const float* dlast_im,
                                void* dw_re, void* dw_im, float* deta, float* ddelta, float* dnu_log,

@@ -4105,11 +4105,14 @@ sparc_status sparc_scan_backward(const sparc_scan_desc* d, const void* gate0, co
     const void* gp[] = {gate0, gate1, dgate0, dgate1};
     if (sparc_status s = check_gate_ptrs(d, pl, gp, 4)) return s;
   }
-  if (saved) {  // P1 from the saved states: the fused kernels, when they apply
-    const void* fp[] = {y_re, y_im, dy_re, dy_im, dw_re, dw_im, h0_re, h0_im, dh0_re, dh0_im};
+  // P1 from the saved states, or behind the relu from the chunk states and the
+  // writes: the fused kernels, when they apply
+  if (saved || (relu && sparc::p1_fused_relu_backward(d))) {
+    const void* fp[] = {saved ? y_re : w_re, saved ? y_im : w_im, dy_re, relu ? nullptr : dy_im, dw_re, dw_im,
+                        h0_re, h0_im, dh0_re, dh0_im};
     if (p1_fused_route(d, 1, fp, 10, chunk_state, workspace_bytes))
       return sparc::p1_fused_backward(d, static_cast<const float*>(gate0), static_cast<const float*>(gate1), nu_log,
-                                      theta_log, y_re, y_im, h0_re, h0_im, segment_pos, dy_re, dy_im, dlast_re,
+                                      theta_log, w_re, w_im, y_re, y_im, chunk_state, h0_re, h0_im, segment_pos, dy_re, dy_im, dlast_re,
                                       dlast_im, dw_re, dw_im, static_cast<float*>(dgate0),
                                       static_cast<float*>(dgate1), dnu_log, dtheta_log, dh0_re, dh0_im, workspace,
                                       workspace_bytes, stream);

@@ -68,8 +68,20 @@ def test_split_many_chains(B, M, dtype, extra, T):
     print(f"[case] split B={B} T={T} M={M} {dtype} {extra}", flush=True)
     case = make_case("p1", B, T, M, 1, dtype, seed=B + T, **extra)
     tol = 1e-5 if dtype == F32 else 2.0 ** -8
-    for k, (a, b) in enumerate(zip(_run(case, "auto", False), _run(case, "chain", False))):
-        assert rel_err(a, b) <= tol, f"output {k}: {rel_err(a, b):.3g}"
+    n_out = 3 if extra.get("relu") else 4
+    for k, (a, b) in enumerate(zip(_run(case, "auto", True), _run(case, "chain", True))):
+        if k < n_out:
+            assert rel_err(a, b) <= tol, f"output {k}: {rel_err(a, b):.3g}"
+        elif extra.get("relu"):
+            # a state within its rounding of zero may pass the relu in one form
+            # and not in the other; its dy (of order 1) then moves the gradients
+            # of the steps before it: in the 2-norm a few such states of some
+            # millions
+            e = ((a.float() - b.float()).norm() / b.float().norm().clamp_min(1e-30)).item()
+            assert e <= (2e-3 if dtype == F32 else 1e-2), f"gradient {k - n_out}: {e:.3g}"
+        else:
+            # the transition gradients sum over the modes and steps
+            assert rel_err(a, b) <= max(4 * tol, 5e-5), f"gradient {k - n_out}: {rel_err(a, b):.3g}"
 
 
 @pytest.mark.parametrize("B,L,width,dtype", [
@@ -123,3 +135,44 @@ def test_forward_without_gradients_matches(B, L, width, dtype):
     y2, last2 = m(x, return_cache=True)
     for a, b, c in zip((y, *last), (y1, *last1), (y2, *last2)):
         assert torch.equal(a, b) and torch.equal(a, c) and not b.requires_grad
+
+
+@pytest.mark.parametrize("B,L,width,dtype", [
+    (1, 33, 264, torch.float32), (2, 257, 2048, torch.bfloat16),   # few chains
+    (3, 259, 16384, torch.bfloat16),   # 192 chains of 128: 8 waves, 2 modes per lane
+    (5, 260, 16376, torch.bfloat16),   # 320: 4 waves, 1 mode per lane
+    (7, 256, 16384, torch.bfloat16),   # 448: 4 waves, 2 modes per lane
+    (2, 300, 16376, torch.float32),    # 128, fp32
+])
+def test_split_module_backward(B, L, width, dtype):
+    """Every gradient of the module's split backward against the composed path
+    (separate operators on the general kernels), the incoming gradient masked
+    where the state is near the relu's edge."""
+    print(f"[case] split module backward B={B} L={L} width={width} {dtype}", flush=True)
+    torch.manual_seed(L + B)
+    m = sparc_amd.SPARCMixer(width).cuda()
+    with torch.no_grad():
+        for p in (m.phase_direction, m.radial_direction):
+            p.copy_(torch.randn_like(p) * 0.5 / width ** 0.5)
+        for p in (m.write_phase_response, m.write_radial_response):
+            p.copy_(torch.randn_like(p) * 0.3)
+    x = torch.randn(B, L, width, device="cuda").to(dtype)
+    dy = torch.randn(B, L, width, device="cuda").to(dtype)
+    dl = torch.randn(B, width // 2, device="cuda")
+    params = [m.phase_direction, m.radial_direction, m.nu_log, m.theta_log, m.write_log_gain,
+              m.write_phase_response, m.write_radial_response]
+    got, band = {}, None
+    for path in ("composed", "fused"):
+        sparc_amd.set_mixer_path(path)
+        try:
+            xx = x.clone().requires_grad_()
+            y, last = m(xx, return_cache=True)
+            if band is None:  # positive outputs within the band and every zero next to one
+                edge = y.detach().float() < (1e-3 if dtype == torch.float32 else 5e-2)
+                band = (edge & (y.detach() > 0)) | (y.detach() == 0)
+            got[path] = torch.autograd.grad([y, last[0]], [xx, *params], [dy.masked_fill(band, 0.0), dl])
+        finally:
+            sparc_amd.set_mixer_path("auto")
+    tol = 1e-4 if dtype == torch.float32 else 2e-2
+    for k, (a, b) in enumerate(zip(got["fused"], got["composed"])):
+        assert rel_err(a, b) <= tol, f"gradient {k}: {rel_err(a, b):.3g}"
