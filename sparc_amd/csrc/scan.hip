@@ -1891,6 +1891,9 @@ chain_bwd_kernel(ScanArgs p) {
 constexpr int kFastMaxGpw = 16;  // gate groups per wave handled by the fast kernels
 
 
+// the gates' type: fp32 beside bf16 I/O with TR_G32, else the I/O type
+template <int TR, typename IO> using GateT = std::conditional_t<tr_g32(TR), float, IO>;
+
 constexpr int fast_rounds(int S) { return (S * kFastMaxGpw + 63) / 64; }
 
 // Raw gate bits (and segment positions) of the (step, group) pairs of one
@@ -1918,7 +1921,7 @@ __device__ __forceinline__ float bits_to_float(uint32_t bits) {
 // Every lane loads: pairs outside the tensors (steps past T, groups past G in
 // the last mode block, rounds past S * gpw) read element 0, and fill_tab
 // discards them.
-template <int TR, typename IO, int S>
+template <int TR, typename GT, int S>
 __device__ __forceinline__ void load_gate_pairs(const ScanArgs& p, int b, int t0, int g_base, int gpw, int lane,
                                                 GateBlock<S>& gb) {
 #pragma unroll
@@ -1930,8 +1933,8 @@ __device__ __forceinline__ void load_gate_pairs(const ScanArgs& p, int b, int t0
     const bool in_t = idx < S * gpw && t < p.T;
     const int64_t row = static_cast<int64_t>(b) * p.T + t;
     const int64_t gi = (in_t && g < p.G) ? row * p.G + g : 0;
-    gb.g0[r] = load_bits<IO>(p.g0, gi);
-    if constexpr (TR != TR_REAL) gb.g1[r] = load_bits<IO>(p.g1, gi);
+    gb.g0[r] = load_bits<GT>(p.g0, gi);
+    if constexpr (tr_kind(TR) != TR_REAL) gb.g1[r] = load_bits<GT>(p.g1, gi);
     if (p.segpos) gb.pos[r] = p.segpos[in_t ? row : 0];
   }
 }
@@ -1939,7 +1942,7 @@ __device__ __forceinline__ void load_gate_pairs(const ScanArgs& p, int b, int t0
 // tab[pair] = (ar, ai[, cos phi, sin phi]); identity past T, zero at resets
 // and for groups past G.  Returns the lane's reset pairs as a bit mask (bit r:
 // pair r * 64 + lane).
-template <int TR, typename IO, int S, int TW>
+template <int TR, typename GT, int S, int TW>
 __device__ __forceinline__ uint32_t fill_tab(const ScanArgs& p, int t0, int g_base, int gpw, int lane,
                                              bool reset_first, const GateBlock<S>& gb, float* tab) {
   uint32_t rmask = 0u;
@@ -1952,13 +1955,13 @@ __device__ __forceinline__ uint32_t fill_tab(const ScanArgs& p, int t0, int g_ba
       const bool g_ok = g_base + idx - step * gpw < p.G;
       float ar = 1.0f, ai = 0.0f, cp = 1.0f, sp = 0.0f;
       if (t < p.T) {
-        const float v0 = g_ok ? bits_to_float<IO>(gb.g0[r]) : 0.0f;
-        const float v1 = (TR != TR_REAL && g_ok) ? bits_to_float<IO>(gb.g1[r]) : 0.0f;
-        if constexpr (TR == TR_POLAR) {
+        const float v0 = g_ok ? bits_to_float<GT>(gb.g0[r]) : 0.0f;
+        const float v1 = (tr_kind(TR) != TR_REAL && g_ok) ? bits_to_float<GT>(gb.g1[r]) : 0.0f;
+        if constexpr (tr_kind(TR) == TR_POLAR) {
           sincos_moderate(v1, sp, cp);
           ar = v0 * cp;
           ai = v0 * sp;
-        } else if constexpr (TR == TR_CART) {
+        } else if constexpr (tr_kind(TR) == TR_CART) {
           ar = v0;
           ai = v1;
         } else {
@@ -1983,9 +1986,8 @@ __device__ __forceinline__ uint32_t fill_tab(const ScanArgs& p, int t0, int g_ba
 template <int TR, typename IO, int V, int S, int NW, bool RELU>
 __global__ void __launch_bounds__(NW * 64, 4)
 chain_fwd_fast_kernel(ScanArgs p) {
-  static_assert(!tr_g32(TR), "lane-shared kernels read gates in the I/O dtype");
   if (blockIdx.x == 0 && threadIdx.x == 0) *p.error = 0u;  // no waits here: never an error
-  constexpr bool CPLX = TR != TR_REAL;
+  constexpr bool CPLX = tr_kind(TR) != TR_REAL;
   constexpr int C = S * NW;
   constexpr int MB = 64 * V;
   constexpr int NH = CPLX ? 2 : 1;
@@ -2041,7 +2043,7 @@ chain_fwd_fast_kernel(ScanArgs p) {
         wi[hb][s] = wr[hb][s];
       }
     }
-    load_gate_pairs<TR, IO, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
+    load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
   };
 
   load_chunk(0, 0);
@@ -2052,7 +2054,7 @@ chain_fwd_fast_kernel(ScanArgs p) {
       if (c >= p.n_chunks) break;
       const int t0 = c * C + wave * S;
       if (c + 1 < p.n_chunks) load_chunk(1 - h, c + 1);
-      fill_tab<TR, IO, S, TW>(p, t0, g_base, gpw, lane, reset_first, gb[h], tab);
+      fill_tab<TR, GateT<TR, IO>, S, TW>(p, t0, g_base, gpw, lane, reset_first, gb[h], tab);
       __builtin_amdgcn_wave_barrier();
       float ar[S], ai[S];
 #pragma unroll
@@ -2183,14 +2185,13 @@ chain_fwd_fast_kernel(ScanArgs p) {
 template <int TR, typename IO, int V, int S, int NW, bool RELU>
 __global__ void __launch_bounds__(NW * 64, 2)
 chain_bwd_fast_kernel(ScanArgs p) {
-  static_assert(!tr_g32(TR), "lane-shared kernels read gates in the I/O dtype");
   if (blockIdx.x == 0 && threadIdx.x == 0) *p.error = 0u;  // no waits here: never an error
-  constexpr bool CPLX = TR != TR_REAL;
+  constexpr bool CPLX = tr_kind(TR) != TR_REAL;
   constexpr int C = S * NW;
   constexpr int MB = 64 * V;
   constexpr int NH = CPLX ? 2 : 1;
   constexpr int R = fast_rounds(S);
-  constexpr int TW = (TR == TR_POLAR) ? 4 : (CPLX ? 2 : 1);
+  constexpr int TW = (tr_kind(TR) == TR_POLAR) ? 4 : (CPLX ? 2 : 1);
   constexpr int ESZ = sizeof(IO);
   constexpr int NG = CPLX ? 2 : 1;    // gate gradients per (step, group)
   constexpr int RED = S * NG + 1;     // padded LDS row of one lane's partial gate gradients
@@ -2266,7 +2267,7 @@ chain_bwd_fast_kernel(ScanArgs p) {
         di[hb][s] = wr[hb][s];
       }
     }
-    load_gate_pairs<TR, IO, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
+    load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       float h_r = 0.0f, h_i = 0.0f;
@@ -2294,7 +2295,7 @@ chain_bwd_fast_kernel(ScanArgs p) {
       const int t0 = c * C + wave * S;
       const int xb = c & 1;  // s_xi buffer holding the adjoint entering this chunk
       if (c - 1 >= 0) load_chunk(1 - h, c - 1);
-      const uint32_t rmask = fill_tab<TR, IO, S, TW>(p, t0, g_base, gpw, lane, reset_first, gb[h], tab);
+      const uint32_t rmask = fill_tab<TR, GateT<TR, IO>, S, TW>(p, t0, g_base, gpw, lane, reset_first, gb[h], tab);
       __builtin_amdgcn_wave_barrier();
       float ar[S], ai[S];
 #pragma unroll
@@ -2507,7 +2508,7 @@ chain_bwd_fast_kernel(ScanArgs p) {
         }
         float e0 = 0.0f, e1 = 0.0f;
         float cp = 1.0f, sp = 0.0f;
-        if constexpr (TR == TR_POLAR) {
+        if constexpr (tr_kind(TR) == TR_POLAR) {
           cp = tab[(s * gpw + my_g) * TW + 2];
           sp = tab[(s * gpw + my_g) * TW + 3];
         }
@@ -2516,7 +2517,7 @@ chain_bwd_fast_kernel(ScanArgs p) {
           if constexpr (CPLX) {
             const float gar = fmaf(lr[v], hpr[s][v], li[v] * hpi[s][v]);
             const float gai = fmaf(li[v], hpr[s][v], -lr[v] * hpi[s][v]);
-            if constexpr (TR == TR_POLAR) {
+            if constexpr (tr_kind(TR) == TR_POLAR) {
               e0 += fmaf(gar, cp, gai * sp);
               e1 += fmaf(gai, ar[s], -gar * ai[s]);
             } else {
@@ -2560,8 +2561,8 @@ chain_bwd_fast_kernel(ScanArgs p) {
             // a reset step's transition is the constant 0: no gradient
             const bool reset = (rmask >> r) & 1u;
             const int64_t gi = (row0 + t) * p.G + g_base + g;
-            store1<IO>(p.dg0, gi, reset ? 0.0f : a0);
-            if constexpr (CPLX) store1<IO>(p.dg1, gi, reset ? 0.0f : a1);
+            store1<GateT<TR, IO>>(p.dg0, gi, reset ? 0.0f : a0);
+            if constexpr (CPLX) store1<GateT<TR, IO>>(p.dg1, gi, reset ? 0.0f : a1);
           }
         }
       }
@@ -2580,14 +2581,13 @@ chain_bwd_fast_kernel(ScanArgs p) {
 template <int TR, typename IO, int V, int S, int NW>
 __global__ void __launch_bounds__(NW * 64, 2)
 chain_bwd_saved_kernel(ScanArgs p) {
-  static_assert(!tr_g32(TR), "lane-shared kernels read gates in the I/O dtype");
   if (blockIdx.x == 0 && threadIdx.x == 0) *p.error = 0u;  // no waits here: never an error
-  constexpr bool CPLX = TR != TR_REAL;
+  constexpr bool CPLX = tr_kind(TR) != TR_REAL;
   constexpr int C = S * NW;
   constexpr int MB = 64 * V;
   constexpr int NH = CPLX ? 2 : 1;
   constexpr int R = fast_rounds(S);
-  constexpr int TW = (TR == TR_POLAR) ? 4 : (CPLX ? 2 : 1);
+  constexpr int TW = (tr_kind(TR) == TR_POLAR) ? 4 : (CPLX ? 2 : 1);
   constexpr int ESZ = sizeof(IO);
   constexpr int NG = CPLX ? 2 : 1;    // gate gradients per (step, group)
   constexpr int RED = S * NG + 1;     // padded LDS row of one lane's partial gate gradients
@@ -2660,7 +2660,7 @@ chain_bwd_saved_kernel(ScanArgs p) {
         }
       }
     }
-    load_gate_pairs<TR, IO, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
+    load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
   };
 
   load_chunk(0, p.n_chunks - 1);
@@ -2672,7 +2672,7 @@ chain_bwd_saved_kernel(ScanArgs p) {
       const int t0 = c * C + wave * S;
       const int xb = c & 1;  // buffers of this chunk (maps, entering adjoint)
       if (c - 1 >= 0) load_chunk(1 - h, c - 1);
-      const uint32_t rmask = fill_tab<TR, IO, S, TW>(p, t0, g_base, gpw, lane, reset_first, gb[h], tab);
+      const uint32_t rmask = fill_tab<TR, GateT<TR, IO>, S, TW>(p, t0, g_base, gpw, lane, reset_first, gb[h], tab);
       __builtin_amdgcn_wave_barrier();
       float ar[S], ai[S];
 #pragma unroll
@@ -2795,7 +2795,7 @@ chain_bwd_saved_kernel(ScanArgs p) {
         }
         float e0 = 0.0f, e1 = 0.0f;
         float cp = 1.0f, sp = 0.0f;
-        if constexpr (TR == TR_POLAR) {
+        if constexpr (tr_kind(TR) == TR_POLAR) {
           cp = tab[(s * gpw + my_g) * TW + 2];
           sp = tab[(s * gpw + my_g) * TW + 3];
         }
@@ -2804,7 +2804,7 @@ chain_bwd_saved_kernel(ScanArgs p) {
           if constexpr (CPLX) {
             const float gar = fmaf(lr[v], hr[v], li[v] * hi[v]);
             const float gai = fmaf(li[v], hr[v], -lr[v] * hi[v]);
-            if constexpr (TR == TR_POLAR) {
+            if constexpr (tr_kind(TR) == TR_POLAR) {
               e0 += fmaf(gar, cp, gai * sp);
               e1 += fmaf(gai, ar[s], -gar * ai[s]);
             } else {
@@ -2841,8 +2841,8 @@ chain_bwd_saved_kernel(ScanArgs p) {
             // a reset step's transition is the constant 0: no gradient
             const bool reset = (rmask >> r) & 1u;
             const int64_t gi = (row0 + t) * p.G + g_base + g;
-            store1<IO>(p.dg0, gi, reset ? 0.0f : a0);
-            if constexpr (CPLX) store1<IO>(p.dg1, gi, reset ? 0.0f : a1);
+            store1<GateT<TR, IO>>(p.dg0, gi, reset ? 0.0f : a0);
+            if constexpr (CPLX) store1<GateT<TR, IO>>(p.dg1, gi, reset ? 0.0f : a1);
           }
         }
       }
@@ -2913,10 +2913,9 @@ __device__ __forceinline__ SerialPos serial_pos(const ScanArgs& p) {
 template <int TR, typename IO, int V, int S, bool RELU, bool SUMMARY = false>
 __global__ void __launch_bounds__(128, 1)
 chain_fwd_serial_kernel(ScanArgs p) {
-  static_assert(!tr_g32(TR), "lane-shared kernels read gates in the I/O dtype");
   static_assert(kStateChunk % S == 0, "blocks must tile the saved-state chunks");
   if (blockIdx.x == 0 && threadIdx.x == 0) *p.error = 0u;  // no waits here: never an error
-  constexpr bool CPLX = TR != TR_REAL;
+  constexpr bool CPLX = tr_kind(TR) != TR_REAL;
   constexpr int MB = 64 * V;
   constexpr int NH = CPLX ? 2 : 1;
   constexpr int TW = CPLX ? 2 : 1;
@@ -3045,8 +3044,8 @@ chain_fwd_serial_kernel(ScanArgs p) {
   } else {
 #pragma unroll
     for (int d = 0; d < kGateDepth - 1; ++d)
-      if (d < n_blocks) load_gate_pairs<TR, IO, S>(p, b, t_begin + d * S, g_base, gpw, lane, gb[d]);
-    fill_tab<TR, IO, S, TW>(p, t_begin, g_base, gpw, lane, reset_first, gb[0], tab[0]);
+      if (d < n_blocks) load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t_begin + d * S, g_base, gpw, lane, gb[d]);
+    fill_tab<TR, GateT<TR, IO>, S, TW>(p, t_begin, g_base, gpw, lane, reset_first, gb[0], tab[0]);
   }
   __syncthreads();
   // block k = k0 + h: planes and table in buffers k & 1 = h & 1, gates in
@@ -3076,9 +3075,9 @@ chain_fwd_serial_kernel(ScanArgs p) {
           }
         }
       } else if (k + 1 < n_blocks) {
-        fill_tab<TR, IO, S, TW>(p, t0 + S, g_base, gpw, lane, reset_first, gb[(h + 1) % kGateDepth], tab[1 - x]);
+        fill_tab<TR, GateT<TR, IO>, S, TW>(p, t0 + S, g_base, gpw, lane, reset_first, gb[(h + 1) % kGateDepth], tab[1 - x]);
         if (k + kGateDepth - 1 < n_blocks)
-          load_gate_pairs<TR, IO, S>(p, b, t0 + (kGateDepth - 1) * S, g_base, gpw, lane,
+          load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t0 + (kGateDepth - 1) * S, g_base, gpw, lane,
                                      gb[(h + kGateDepth - 1) % kGateDepth]);
       }
       __syncthreads();
@@ -3108,12 +3107,11 @@ chain_fwd_serial_kernel(ScanArgs p) {
 template <int TR, typename IO, int V, int S, bool SUMMARY = false>
 __global__ void __launch_bounds__(128, 1)
 chain_bwd_serial_kernel(ScanArgs p) {
-  static_assert(!tr_g32(TR), "lane-shared kernels read gates in the I/O dtype");
   if (blockIdx.x == 0 && threadIdx.x == 0) *p.error = 0u;  // no waits here: never an error
-  constexpr bool CPLX = TR != TR_REAL;
+  constexpr bool CPLX = tr_kind(TR) != TR_REAL;
   constexpr int MB = 64 * V;
   constexpr int R = fast_rounds(S);
-  constexpr int TW = (TR == TR_POLAR) ? 4 : (CPLX ? 2 : 1);
+  constexpr int TW = (tr_kind(TR) == TR_POLAR) ? 4 : (CPLX ? 2 : 1);
   constexpr int ESZ = sizeof(IO);
   constexpr int NG = CPLX ? 2 : 1;    // transition gradients per (step, group)
   constexpr int RED = S * NG + 1;     // padded LDS row of one lane's partials
@@ -3284,7 +3282,7 @@ chain_bwd_serial_kernel(ScanArgs p) {
         const int t = t0 + step;
         if (t < p.T && g_base + g < p.G) {  // the last mode block may hold fewer groups
           float d0 = sr, d1 = si;
-          if constexpr (TR == TR_POLAR) {
+          if constexpr (tr_kind(TR) == TR_POLAR) {
             const float* e = tb + idx * TW;   // (ar, ai, cos phi, sin phi) of this pair
             d0 = fmaf(sr, e[2], si * e[3]);
             d1 = fmaf(si, e[0], -sr * e[1]);
@@ -3292,8 +3290,8 @@ chain_bwd_serial_kernel(ScanArgs p) {
           // a reset step's transition is the constant 0: no gradient
           const bool reset = (rm >> r) & 1u;
           const int64_t gi = (row0 + t) * p.G + g_base + g;
-          store1<IO>(p.dg0, gi, reset ? 0.0f : d0);
-          if constexpr (CPLX) store1<IO>(p.dg1, gi, reset ? 0.0f : d1);
+          store1<GateT<TR, IO>>(p.dg0, gi, reset ? 0.0f : d0);
+          if constexpr (CPLX) store1<GateT<TR, IO>>(p.dg1, gi, reset ? 0.0f : d1);
         }
       }
     }
@@ -3311,8 +3309,8 @@ chain_bwd_serial_kernel(ScanArgs p) {
 #pragma unroll
     for (int d = 0; d < kGateDepth - 1; ++d)
       if (d < n_blocks)
-        load_gate_pairs<TR, IO, S>(p, b, t_begin + (n_blocks - 1 - d) * S, g_base, gpw, lane, gb[d]);
-    rm_mid = fill_tab<TR, IO, S, TW>(p, t_begin + (n_blocks - 1) * S, g_base, gpw, lane, reset_first, gb[0], tab[0]);
+        load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t_begin + (n_blocks - 1 - d) * S, g_base, gpw, lane, gb[d]);
+    rm_mid = fill_tab<TR, GateT<TR, IO>, S, TW>(p, t_begin + (n_blocks - 1) * S, g_base, gpw, lane, reset_first, gb[0], tab[0]);
   }
   __syncthreads();
   for (int j0 = 0; j0 < n_blocks; j0 += kGateDepth) {
@@ -3331,10 +3329,10 @@ chain_bwd_serial_kernel(ScanArgs p) {
         rm_old = rm_mid;
         rm_mid = 0u;
         if (k >= 1) {
-          rm_mid = fill_tab<TR, IO, S, TW>(p, t0 - S, g_base, gpw, lane, reset_first,
+          rm_mid = fill_tab<TR, GateT<TR, IO>, S, TW>(p, t0 - S, g_base, gpw, lane, reset_first,
                                            gb[(h + 1) % kGateDepth], tab[1 - x]);
           if (k >= kGateDepth - 1)
-            load_gate_pairs<TR, IO, S>(p, b, t0 - (kGateDepth - 1) * S, g_base, gpw, lane,
+            load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t0 - (kGateDepth - 1) * S, g_base, gpw, lane,
                                        gb[(h + kGateDepth - 1) % kGateDepth]);
         }
       }
@@ -3426,7 +3424,7 @@ struct Plan {
   bool chain = false;
   bool fast = false;  // chain kernels specialised for lane-shared gates
   bool serial = false;  // one wave per chain (lane-shared gates, many chains)
-  bool g32 = false;  // fp32 gates beside bf16 I/O (general kernels only)
+  bool g32 = false;  // fp32 gates beside bf16 I/O
   int n_chunks = 0, n_mblocks = 0, n_chains = 0;
   int n_seg = 1, t_seg = 0;  // time segments of the serial kernels (n_seg > 1: few chains)
   int64_t n_tiles = 0;
@@ -3487,7 +3485,7 @@ struct Kernels {
   static constexpr int CS_F = 8, CNW_F = kChunk / CS_F;
   static constexpr int CS_B = 4, CNW_B = kChunk / CS_B;
   static void run(int dir, bool chain, const Plan& pl, hipStream_t st, const sparc::ScanArgs& a) {
-    if constexpr (sparc::tr_kind(TR) != sparc::TR_P1 && GM == sparc::GATE_LANE && !sparc::tr_g32(TR)) {
+    if constexpr (sparc::tr_kind(TR) != sparc::TR_P1 && GM == sparc::GATE_LANE) {
       if (pl.serial && dir == 0) {
         serial_fwd<TR, IO, V>(pl, st, a);
         return;
@@ -3519,7 +3517,7 @@ struct Kernels {
       hipLaunchKernelGGL((sparc::scan_bwd_kernel<TR, IO, V, GM, S, NW, true>), g, dim3(NW * 64), 0, st, a);
       return true;
     }
-    if constexpr (sparc::tr_kind(TR) != sparc::TR_P1 && GM == sparc::GATE_LANE && !sparc::tr_g32(TR)) {
+    if constexpr (sparc::tr_kind(TR) != sparc::TR_P1 && GM == sparc::GATE_LANE) {
       if (pl.serial) {
         serial_bwd<TR, IO, V>(pl, st, a);
         return true;
@@ -3562,7 +3560,7 @@ bool launch_v(int dir, const Plan& pl, hipStream_t st, const sparc::ScanArgs& a)
     return true;                                                                        \
   }
   if constexpr ((sparc::tr_kind(TR) == sparc::TR_POLAR || sparc::tr_kind(TR) == sparc::TR_CART) &&
-                sparc::IsBf16<IO>::value && !sparc::tr_g32(TR)) {
+                sparc::IsBf16<IO>::value) {
     if (V == kWideV) {
       if (!pl.serial || gm != sparc::GATE_LANE) return false;
       if (dir == 1) return false;  // no recomputing kernel: wide plans need the saved output
@@ -3759,7 +3757,6 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   const bool p1 = d->transition == SPARC_TRANSITION_P1;
   if (d->gate_dtype != SPARC_F32 && d->gate_dtype != SPARC_BF16) return "unknown gate_dtype";
   if (p1 && d->gate_dtype != SPARC_F32) return "P1 gates (eta, delta) must be fp32";
-  // fp32 gates beside bf16 I/O: the general (per-lane transition) kernels
   const bool g32 = !p1 && d->gate_dtype == SPARC_F32 && d->io_dtype == SPARC_BF16;
   if (!p1 && d->gate_dtype != d->io_dtype && !g32) return "bf16 gates need bf16 I/O";
   if ((d->flags & SPARC_FLAG_RELU_OUTPUT) && d->transition == SPARC_TRANSITION_REAL)
@@ -3792,7 +3789,7 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   // per lane and plane (4 modes) when that still leaves enough chains, or
   // over time segments when the chains are few.
   bool wide = false;
-  if (!p1 && !g32 && cplx_tr && bf16_io && M % kWideV == 0 &&
+  if (!p1 && cplx_tr && bf16_io && M % kWideV == 0 &&
       gs % kWideV == 0 && (64 * kWideV) % gs == 0 && is_pow2(gs / kWideV) &&
       (64 * kWideV) / gs <= sparc::kFastMaxGpw && !force_l && !force_c && allow_wide) {
     const int64_t chains = d->batch * ((M + 64 * kWideV - 1) / (64 * kWideV));
@@ -3811,7 +3808,7 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   pl->n_mblocks = static_cast<int>((M + 64 * V - 1) / (64 * V));
   pl->n_chains = static_cast<int>(d->batch * pl->n_mblocks);
   pl->n_tiles = static_cast<int64_t>(pl->n_chains) * pl->n_chunks;
-  const bool lane_shared = !p1 && !g32 && gm == sparc::GATE_LANE && (64 * V) / gs <= sparc::kFastMaxGpw;
+  const bool lane_shared = !p1 && gm == sparc::GATE_LANE && (64 * V) / gs <= sparc::kFastMaxGpw;
   // The automatic plan for lane-shared gates, by I/O dtype and transition
   // (MI355X, fwd+bwd at B*T*M = 2^28, G = M/16; `plan_lane_shared` below):
   // bf16 streams half the bytes per tile, so the look-back's per-tile cost

@@ -320,9 +320,8 @@ def test_real_scan_with_last_is_no_grad():
 
 @pytest.mark.parametrize("transition", ["polar", "cartesian", "real"])
 def test_grouped_fp32_gates_bf16_writes_every_algorithm(transition):
-    """fp32 gates shared by groups of modes beside bf16 writes (the general
-    kernels; lane-shared fast paths read gates in the I/O dtype and are not
-    used for this case) under each algorithm, forward and backward."""
+    """fp32 gates shared by groups of modes beside bf16 writes under each
+    algorithm, forward and backward."""
     M, G = 256, 16
     for algo in ("lookback", "chain", "serial"):
         print(f"[case] grouped fp32 gates {transition} B=2 T=300 M={M} G={G} bf16 writes algo={algo}",

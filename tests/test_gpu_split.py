@@ -8,7 +8,8 @@ Few chains are held against the float64 oracle; the shapes with enough chains
 for 16, 8 and 4 waves each against the general chain kernels, whose per-step
 recurrence is the same: both are fp32 recurrences with relative error about
 2^-24 per remembered step, so 1e-5 of max |reference| over 300 steps (bf16
-I/O: one rounding to 8 bits, 2^-8)."""
+I/O: values that differ in their last fp32 bits may round to neighbouring bf16
+values, at most 2^-7 apart)."""
 import pytest
 import torch
 
@@ -67,7 +68,7 @@ def _run(case, algorithm, want_grads):
 def test_split_many_chains(B, M, dtype, extra, T):
     print(f"[case] split B={B} T={T} M={M} {dtype} {extra}", flush=True)
     case = make_case("p1", B, T, M, 1, dtype, seed=B + T, **extra)
-    tol = 1e-5 if dtype == F32 else 2.0 ** -8
+    tol = 1e-5 if dtype == F32 else 2.0 ** -7
     n_out = 3 if extra.get("relu") else 4
     for k, (a, b) in enumerate(zip(_run(case, "auto", True), _run(case, "chain", True))):
         if k < n_out:
