@@ -248,17 +248,20 @@ class _ChunkScan(torch.autograd.Function):
     """Differentiable chunked scan for every transition.
 
     Outputs (y_re, y_im, last_re, last_im); y_re is the visible relu(cat)
-    output with ``relu_output``; unused outputs are empty tensors."""
+    output with ``relu_output``; unused outputs (the last state of an operator
+    that does not return it, without ``want_last``) are empty tensors."""
 
     @staticmethod
     def forward(ctx, transition, relu_output, reset_first, g0, g1, nu_log, theta_log,
-                w_re, w_im, h0_re, h0_im, segment_pos):
+                w_re, w_im, h0_re, h0_im, segment_pos, want_last=True):
         y_re, y_im, cs = scan_forward_raw(
             transition, g0, g1, w_re, w_im, nu_log, theta_log, h0_re, h0_im,
             segment_pos, reset_first, relu_output)
         cplx = transition != "real"
         B, T, M = w_re.shape
-        if T > 0:
+        if not want_last:
+            last_re, last_im = (w_re.new_empty(0, dtype=torch.float32) for _ in range(2))
+        elif T > 0:
             last_re = cs[:, -1, :, 0].contiguous() if cplx else cs[:, -1].contiguous()
             last_im = cs[:, -1, :, 1].contiguous() if cplx else w_re.new_empty(0, dtype=torch.float32)
         else:
@@ -272,9 +275,11 @@ class _ChunkScan(torch.autograd.Function):
         ctx.save_for_backward(g0, g1, nu_log, theta_log, w_re, w_im, h0_re, h0_im, segment_pos, cs,
                               *saved_y)
         ctx.cfg = (transition, relu_output, reset_first)
+        ctx.set_materialize_grads(False)  # unused outputs: no gradient, not zero tensors to fill and read
         if y_im is None:
             y_im = w_re.new_empty(0)
-        ctx.mark_non_differentiable(y_im) if y_im.numel() == 0 else None
+        if y_im.numel() == 0:
+            ctx.mark_non_differentiable(y_im)
         return y_re, y_im, last_re, last_im
 
     @staticmethod
@@ -303,7 +308,7 @@ class _ChunkScan(torch.autograd.Function):
             nu_log, theta_log, h0_re, h0_im, segment_pos, reset_first, relu_output,
             dlast_re, dlast_im, want_dh0=h0_re is not None, y_re=ys_re, y_im=ys_im)
         return (None, None, None, g["dg0"], g["dg1"], g["dnu"], g["dth"],
-                g["dw_re"], g["dw_im"], g["dh0_re"], g["dh0_im"], None)
+                g["dw_re"], g["dw_im"], g["dh0_re"], g["dh0_im"], None, None)
 
 
 def chunk_scan(transition: str, g0, g1, w_re, w_im=None, nu_log=None, theta_log=None,
@@ -319,6 +324,14 @@ def chunk_scan(transition: str, g0, g1, w_re, w_im=None, nu_log=None, theta_log=
     Returns (y, last): y = (h_re, h_im) [B,T,M] each, or relu(cat) [B,T,2M]
     with relu_output, or h [B,T,M] for "real"; last = (last_re, last_im) fp32
     [B,M] (a single tensor for "real")."""
+    return _scan(transition, g0, g1, w_re, w_im, nu_log, theta_log, initial_state, segment_pos, reset_first,
+                 relu_output)
+
+
+def _scan(transition, g0, g1, w_re, w_im=None, nu_log=None, theta_log=None, initial_state=None,
+          segment_pos=None, reset_first=False, relu_output=False, want_last=True):
+    """``chunk_scan``; without ``want_last`` (the operators that return the
+    sequence alone) last is empty."""
     if transition not in TRANSITIONS:
         raise ValueError(f"unknown transition {transition!r}")
     cplx = transition != "real"
@@ -359,7 +372,7 @@ def chunk_scan(transition: str, g0, g1, w_re, w_im=None, nu_log=None, theta_log=
         segment_pos = segment_pos.to(torch.int32)
     y_re, y_im, last_re, last_im = _ChunkScan.apply(
         transition, bool(relu_output), bool(reset_first), _c(g0), _c(g1), _c(nu_log), _c(theta_log),
-        _c(w_re), _c(w_im), _c(h0_re), _c(h0_im), _c(segment_pos))
+        _c(w_re), _c(w_im), _c(h0_re), _c(h0_im), _c(segment_pos), want_last)
     if not cplx:
         return y_re, last_re
     if relu_output:
@@ -384,7 +397,7 @@ def sparc_scan(eta, delta, nu_log, theta_log, br, bi):
     _check_sparc_shapes(eta, delta, br, bi)
     if nu_log.shape != (br.shape[2],) or theta_log.shape != (br.shape[2],):
         raise ValueError("SPARC control, spectrum and write shapes disagree")
-    (out_r, out_i), _ = chunk_scan("p1", eta, delta, br, bi, nu_log, theta_log)
+    (out_r, out_i), _ = _scan("p1", eta, delta, br, bi, nu_log, theta_log, want_last=False)
     return out_r, out_i
 
 
@@ -457,8 +470,7 @@ def sparc_chunk_scan(eta, delta, nu_log, theta_log, br, bi, chunk_size: int = 32
         raise ValueError("prefix group size must be 0, 32, 64 or 128")
     if prefix_group_size and not hierarchical_prefix:
         raise ValueError("a grouped prefix requires hierarchical_prefix")
-    y, _ = chunk_scan("p1", eta, delta, br, bi, nu_log, theta_log,
-                      relu_output=fused_output_relu)
+    y, _ = _scan("p1", eta, delta, br, bi, nu_log, theta_log, relu_output=fused_output_relu, want_last=False)
     return y
 
 
@@ -503,7 +515,7 @@ def complex_scan(ar, ai, br, bi):
     shape = ar.shape
     if any(t.shape != shape for t in (ai, br, bi)) or ar.ndim != 3:
         raise ValueError("complex scan expects matching [B, L, M] tensors")
-    (out_r, out_i), _ = chunk_scan("cartesian", ar, ai, br, bi)
+    (out_r, out_i), _ = _scan("cartesian", ar, ai, br, bi, want_last=False)
     return out_r, out_i
 
 
@@ -521,7 +533,7 @@ def real_scan(a, b):
     """``real_scan`` (backward/scan.py:1643-1644, _RealScan :793-822)."""
     if a.shape != b.shape or a.ndim != 3:
         raise ValueError("real scan expects matching [B, L, D] tensors")
-    out, _ = chunk_scan("real", a, None, b)
+    out, _ = _scan("real", a, None, b, want_last=False)
     return out
 
 
@@ -531,7 +543,7 @@ def real_chunk_scan(a, b, chunk_size: int = 16):
         raise ValueError("real chunk scan expects matching [B, L, D] tensors")
     if chunk_size not in (16, 32, 64) or a.shape[1] % chunk_size:
         raise ValueError("chunk size must be 16, 32 or 64 and divide length")
-    out, _ = chunk_scan("real", a, None, b)
+    out, _ = _scan("real", a, None, b, want_last=False)
     return out
 
 
