@@ -91,6 +91,8 @@ _SZ = ctypes.c_size_t
 def load() -> ctypes.CDLL:
     """Loads the library (once) and declares the argument types."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -216,7 +218,17 @@ def check_params(width: int, **named: torch.Tensor) -> None:
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The device's current stream, without building a Stream object."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def as_f32(t: torch.Tensor) -> torch.Tensor:
+    """``t`` in float32 and contiguous: itself where it already is (a call
+    passes up to nine parameters, mostly such)."""
+    if t.dtype == torch.float32 and t.is_contiguous():
+        return t.detach()
+    return t.detach().float().contiguous()
 
 
 def io_code(dtype: torch.dtype) -> int:

@@ -100,6 +100,12 @@ def _keeps_gradients(*tensors) -> bool:
     return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
 
 
+def _planes(t: torch.Tensor) -> tuple[int, int]:
+    """Addresses of the two halves of a [2, ...] tensor (NULL where empty)."""
+    base = t.data_ptr()
+    return base, base + t.numel() // 2 * t.element_size()
+
+
 class _FusedMixer(torch.autograd.Function):
     """Outputs y = relu(cat(h_re, h_im)) [B, L, 2M] (x's dtype) and the last
     state (last_re, last_im) fp32 [B, M].  ``save``: keep the states for the
@@ -114,33 +120,34 @@ class _FusedMixer(torch.autograd.Function):
                           write_phase_response=write_phase_response, write_radial_response=write_radial_response)
         dev = _lib.require_gpu(x, phase_direction, nu_log)
         x = x.contiguous()
-        params = [p.detach().float().contiguous() for p in (
+        params = [_lib.as_f32(p) for p in (
             phase_direction, radial_direction, nu_log, theta_log, write_log_gain,
             write_phase_response, write_radial_response)]
         B, T, W = x.shape
         M = W // 2
         io = _lib.io_code(x.dtype)
-        eta = torch.empty(B, T, dtype=torch.float32, device=dev)
-        delta = torch.empty_like(eta)
+        # eta and delta, the states' planes, and (backward) the gradients share
+        # one allocation each: the library takes addresses, so no views either
+        controls = torch.empty(2, B, T, dtype=torch.float32, device=dev)
         y = torch.empty_like(x)
         last_re = torch.empty(B, M, dtype=torch.float32, device=dev)
-        last_im = torch.empty_like(last_re)
+        last_im = torch.empty(B, M, dtype=torch.float32, device=dev)
         ws_bytes = lib.sparc_mixer_workspace_bytes(B, T, M, 0)
         if ws_bytes == 0:
             raise ValueError("invalid shape for the fused mixer")
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         P = _lib.ptr
+        eta, delta = _planes(controls)
         if not save:
             _lib.check(lib.sparc_mixer_infer(
-                B, T, M, io, P(x), *[P(p) for p in params], P(eta), P(delta), P(y), P(last_re), P(last_im), P(ws),
-                ws.numel(), _lib.stream_of(dev)), "sparc_mixer_infer")
+                B, T, M, io, P(x), *[P(p) for p in params], eta, delta, P(y), P(last_re), P(last_im), P(ws),
+                ws_bytes, _lib.stream_of(dev)), "sparc_mixer_infer")
             return y, last_re, last_im
-        h_re = torch.empty(B, T, M, dtype=x.dtype, device=dev)
-        h_im = torch.empty_like(h_re)
+        h = torch.empty(2, B, T, M, dtype=x.dtype, device=dev)
         _lib.check(lib.sparc_mixer_forward(
-            B, T, M, io, P(x), *[P(p) for p in params], P(eta), P(delta), P(y), P(h_re), P(h_im),
-            P(last_re), P(last_im), P(ws), ws.numel(), _lib.stream_of(dev)), "sparc_mixer_forward")
-        ctx.save_for_backward(x, *params, eta, delta, h_re, h_im)
+            B, T, M, io, P(x), *[P(p) for p in params], eta, delta, P(y), *_planes(h), P(last_re), P(last_im), P(ws),
+            ws_bytes, _lib.stream_of(dev)), "sparc_mixer_forward")
+        ctx.save_for_backward(x, *params, controls, h)
         ctx.set_materialize_grads(False)  # unused last-state outputs: NULL, not zero tensors
         ctx.dtypes = [p.dtype for p in (phase_direction, radial_direction, nu_log, theta_log,
                                         write_log_gain, write_phase_response, write_radial_response)]
@@ -149,7 +156,7 @@ class _FusedMixer(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, dlast_re, dlast_im):
-        x, pd, rd, nu, th, wlg, wpr, wrr, eta, delta, h_re, h_im = ctx.saved_tensors
+        x, pd, rd, nu, th, wlg, wpr, wrr, controls, h = ctx.saved_tensors
         lib = _lib.load()
         dev = x.device
         B, T, W = x.shape
@@ -162,15 +169,16 @@ class _FusedMixer(torch.autograd.Function):
             dlast_re = z if dlast_re is None else dlast_re.float().contiguous()
             dlast_im = z.clone() if dlast_im is None else dlast_im.float().contiguous()
         dx = torch.empty_like(x)
-        grads = [torch.empty(W + 1, dtype=torch.float32, device=dev) for _ in range(2)]
-        grads += [torch.empty(M, dtype=torch.float32, device=dev) for _ in range(5)]
-        ws = torch.empty(lib.sparc_mixer_workspace_bytes(B, T, M, 1), dtype=torch.uint8, device=dev)
+        sizes = (W + 1, W + 1, M, M, M, M, M)
+        grads = torch.empty(2 * (W + 1) + 5 * M, dtype=torch.float32, device=dev).split(sizes)
+        ws_bytes = lib.sparc_mixer_workspace_bytes(B, T, M, 1)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         P = _lib.ptr
         _lib.check(lib.sparc_mixer_backward(
             B, T, M, _lib.io_code(x.dtype), P(x), P(pd), P(rd), P(nu), P(th), P(wlg), P(wpr), P(wrr),
-            P(eta), P(delta), P(h_re), P(h_im), P(dy), P(dlast_re), P(dlast_im), P(dx),
-            *[P(g) for g in grads], P(ws), ws.numel(), _lib.stream_of(dev)), "sparc_mixer_backward")
-        grads = [g.to(dt) for g, dt in zip(grads, ctx.dtypes)]
+            *_planes(controls), *_planes(h), P(dy), P(dlast_re), P(dlast_im), P(dx),
+            *[P(g) for g in grads], P(ws), ws_bytes, _lib.stream_of(dev)), "sparc_mixer_backward")
+        grads = [g if g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes)]
         shape, dt = ctx.energy
         # energy_response is an inactive parameter (0 * sum in make_controls): gradient 0
         return (dx, *grads, torch.zeros(shape, dtype=dt, device=dev), None)

@@ -231,7 +231,7 @@ def scan_step(transition, g0, g1, w_re, w_im, state, nu_log=None, theta_log=None
 # autograd
 # ---------------------------------------------------------------------------
 def _c(t):
-    return None if t is None else t.contiguous()
+    return t if t is None or t.is_contiguous() else t.contiguous()
 
 
 def _gate_dtype(g0, g1, io_dtype):
@@ -304,7 +304,8 @@ class _ChunkScan(torch.autograd.Function):
             else:
                 dlast_im = None
         g = scan_backward_raw(
-            transition, g0, g1, w_re, w_im, cs, _c(dy_re).to(w_re.dtype), _c(dy_im).to(w_re.dtype) if dy_im is not None else None,
+            transition, g0, g1, w_re, w_im, cs, _c(dy_re.to(w_re.dtype)),
+            None if dy_im is None else _c(dy_im.to(w_re.dtype)),
             nu_log, theta_log, h0_re, h0_im, segment_pos, reset_first, relu_output,
             dlast_re, dlast_im, want_dh0=h0_re is not None, y_re=ys_re, y_im=ys_im)
         return (None, None, None, g["dg0"], g["dg1"], g["dnu"], g["dth"],
