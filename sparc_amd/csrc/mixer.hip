@@ -2588,23 +2588,28 @@ int mixer_v(int64_t B, int64_t T, int64_t M, int direction, bool gw);
 // Time segments.  One wave per chain (batch row x 64 V modes) walks its
 // whole sequence, so with fewer chains than SIMDs most of the GPU idles.
 // Then the sequence is split into n_seg segments of t_seg steps (a multiple
-// of 8, at least kMinSegSteps) so that about two waves per SIMD run: a
-// summary pass gives each segment's map (P, Q), a carry kernel composes them
-// into the state entering every segment, and the full pass replays each
-// segment from its entering state.  This costs a second pass over the
-// transitions (and, forward, the writes), paid for by the occupancy.
+// of 8): a summary pass gives each segment's map (P, Q), a carry kernel
+// composes them into the state entering every segment, and the full pass
+// replays each segment from its entering state.  This costs a second pass
+// over the transitions (and, forward, the writes), paid for by the occupancy.
+// The waves fill whole rounds of the 1024 SIMDs, 4 of them (bf16) or 2
+// (fp32, whose kernels hold 2 to 3 waves per SIMD), or as many fewer (2, 1)
+// as leave segments of kAlignedSegSteps: a few waves past a round keep their
+// SIMDs busy for one more while the others idle.  Measured (training step,
+// us; segments of at least 128 steps before): P1 with resets, 72 chains,
+// T=4001, fp32 555 (2232 waves) -> 466 (2016; 4032 497), bf16 375 -> 319
+// (4032; 2016 347); module bf16, 72 chains, T=6000 829 (3312) -> 766, 64
+// chains, T=4096 510 (2048) -> 487 (4096), 16 chains, T=16384 467 -> 481.
 #ifndef SPARC_MIXER_SEG_CHAINS
 #define SPARC_MIXER_SEG_CHAINS 1024
 #endif
 constexpr int64_t kSegChains = SPARC_MIXER_SEG_CHAINS;  // segment below this many chains
-#ifndef SPARC_MIXER_SEG_TARGET
-#define SPARC_MIXER_SEG_TARGET 4096
-#endif
 #ifndef SPARC_MIXER_SEG_MIN
 #define SPARC_MIXER_SEG_MIN 128
 #endif
-constexpr int64_t kSegTarget = SPARC_MIXER_SEG_TARGET;  // waves to aim for
-constexpr int64_t kMinSegSteps = SPARC_MIXER_SEG_MIN;
+constexpr int64_t kSimds = 1024;
+constexpr int64_t kMinSegSteps = SPARC_MIXER_SEG_MIN;  // segments shorter than this only to fill rounds of the SIMDs
+constexpr int64_t kAlignedSegSteps = 64;
 int mixer_v(int64_t B, int64_t T, int64_t M, int direction, bool gw) {
   const int fixed = direction == 0 ? SPARC_MIXER_FWD_V : gw ? SPARC_P1_BWD_V : SPARC_MIXER_BWD_V;
   if (fixed == 1 || M % 2) return 1;
@@ -2614,12 +2619,19 @@ int mixer_v(int64_t B, int64_t T, int64_t M, int direction, bool gw) {
   if (direction == 1) return segmented ? 2 : 1;
   return chains2 >= 1280 || segmented ? 2 : 1;
 }
-void choose_segments(int64_t B, int64_t T, int n_mb, int& n_seg, int& t_seg) {
+void choose_segments(int64_t B, int64_t T, int n_mb, int32_t io, int& n_seg, int& t_seg) {
   n_seg = 1;
   t_seg = static_cast<int>(T > 0 ? T : 1);
   const int64_t chains = B * n_mb;
   if (chains >= kSegChains || T < 2 * kMinSegSteps) return;
-  int64_t n = std::min((kSegTarget + chains - 1) / chains, T / kMinSegSteps);
+  int64_t n = T / kMinSegSteps;
+  for (int64_t rounds = io == SPARC_F32 ? 2 : 4; rounds >= 1; rounds /= 2) {
+    const int64_t k = rounds * kSimds / chains;
+    if (k >= 2 && T / k >= kAlignedSegSteps) {
+      n = k;
+      break;
+    }
+  }
   if (n < 2) return;
   int64_t len = (T + n - 1) / n;
   len = (len + 7) / 8 * 8;
@@ -2758,15 +2770,15 @@ struct Layout {
 // gw: the P1 scan with the writes given (no controls, two per-mode gradients);
 // pieces: the module backward in time pieces where the shape allows; split:
 // waves per chain of the split-chain kernels, of split_v modes per lane
-Layout layout(int64_t B, int64_t T, int64_t M, int direction, bool gw = false, bool pieces = false, int split = 0,
-              int split_v = kSplitV) {
+Layout layout(int64_t B, int64_t T, int64_t M, int direction, int32_t io, bool gw = false, bool pieces = false,
+              int split = 0, int split_v = kSplitV) {
   Layout l;
   l.V = mixer_v(B, T, M, direction, gw);
   l.split = split;
   if (l.split) l.V = split_v;
   l.n_mb = static_cast<int>((M + 64 * l.V - 1) / (64 * l.V));
   if (l.split) l.t_seg = static_cast<int>(T);
-  else choose_segments(B, T, l.n_mb, l.n_seg, l.t_seg);
+  else choose_segments(B, T, l.n_mb, io, l.n_seg, l.t_seg);
   l.R = B * T;
   const ControlsLayout cl = controls_layout(l.R, 2 * M, 4);
   l.n_rb = cl.n_rb;
@@ -2934,18 +2946,18 @@ bool fwd_wide(const Layout& l, int64_t batch, int64_t modes, bool module = false
 // The forward's layout: split chains unless the wide kernel is the faster one
 // there (the P1 scan and the fp32 module with many chains, see split_waves).
 Layout forward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, bool gw) {
-  const Layout l = layout(batch, length, modes, 0, gw);
+  const Layout l = layout(batch, length, modes, 0, io_dtype, gw);
   if ((gw || io_dtype == SPARC_F32) && fwd_wide(l, batch, modes, !gw)) return l;
   const int nw = split_waves(batch, length, modes);
-  return nw ? layout(batch, length, modes, 0, gw, false, nw) : l;
+  return nw ? layout(batch, length, modes, 0, io_dtype, gw, false, nw) : l;
 }
 // The backward's, for chain mode cm (kRelu: split, or not there at all);
 // controls: the whole module backward (its time pieces, split_bwd).
 Layout backward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, int cm,
                        bool controls = false) {
   const SplitBwd sp = split_bwd(batch, length, modes, io_dtype, cm, controls);
-  if (!sp.waves) return layout(batch, length, modes, 1, cm != kModule, controls);
-  return layout(batch, length, modes, 1, cm != kModule, false, sp.waves, sp.V);
+  if (!sp.waves) return layout(batch, length, modes, 1, io_dtype, cm != kModule, controls);
+  return layout(batch, length, modes, 1, io_dtype, cm != kModule, false, sp.waves, sp.V);
 }
 
 // the split forward: l.split waves per chain
@@ -3545,7 +3557,7 @@ CoopLayout coop_layout(int64_t B, int64_t T, int64_t M, int kS) {
 // segments (the chains fill the GPU), and every chain resident at once.
 int coop_steps(int64_t B, int64_t T, int64_t M, int32_t io) {
   if (g_bwd_plan.load(std::memory_order_relaxed) != 0 || T <= 0) return 0;
-  const Layout l = layout(B, T, M, 1);
+  const Layout l = layout(B, T, M, 1, io);
   if (l.V != 1 || l.n_seg != 1) return 0;
   const int64_t grid = B * l.n_mb;
   const int64_t cap = io == SPARC_BF16 ? coop_capacity<sparc::bf16, kCoopS>() : coop_capacity<float, kCoopS>();
@@ -3639,7 +3651,7 @@ static sparc_status scan_forward_call(bool save, int64_t batch, int64_t length, 
   Layout l = forward_layout(batch, length, modes, io_dtype, false);
   const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
   // states aligned for one mode only: the forms that store one mode per lane
-  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 0);
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 0, io_dtype);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer scan forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
   if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(workspace, 256))
@@ -3666,7 +3678,7 @@ static sparc_status mixer_forward_call(bool save, int64_t batch, int64_t length,
   Layout l = forward_layout(batch, length, modes, io_dtype, false);
   const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
   // states aligned for one mode only: the forms that store one mode per lane
-  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 0);
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 0, io_dtype);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer forward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
   if (!al(x, 16) || !al(y, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(phase_direction, 16) ||
@@ -3691,12 +3703,13 @@ size_t sparc_mixer_workspace_bytes(int64_t batch, int64_t length, int64_t modes,
   if (batch <= 0 || length < 0 || modes <= 0 || modes % 4 || (direction != 0 && direction != 1)) return 0;
   // every form either I/O type may take: chains split or not, and the module
   // backward in time pieces or in one launch
-  size_t n = layout(batch, length, modes, direction).total;
-  for (const int32_t io : {SPARC_F32, SPARC_BF16})
+  size_t n = direction == 1 ? coop_layout(batch, length, modes, kCoopS).total : 0;
+  for (const int32_t io : {SPARC_F32, SPARC_BF16}) {
+    n = std::max(n, layout(batch, length, modes, direction, io).total);
     n = std::max(n, direction == 0 ? forward_layout(batch, length, modes, io, false).total
-                                   : backward_layout(batch, length, modes, io, kModule, true).total);
-  if (direction == 1)
-    n = std::max({n, layout(batch, length, modes, 1, false, true).total, coop_layout(batch, length, modes, kCoopS).total});
+                                   : std::max(backward_layout(batch, length, modes, io, kModule, true).total,
+                                              layout(batch, length, modes, 1, io, false, true).total));
+  }
   return n;
 }
 
@@ -3775,7 +3788,7 @@ sparc_status sparc_mixer_scan_backward(int64_t batch, int64_t length, int64_t mo
   if ((dlast_re == nullptr) != (dlast_im == nullptr)) return fail(SPARC_EINVAL, "mixer scan backward: dlast_re/dlast_im");
   Layout l = backward_layout(batch, length, modes, io_dtype, kModule);
   const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
-  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 1);
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 1, io_dtype);
   if (!workspace || workspace_bytes < l.total)
     return fail(SPARC_EWORKSPACE, "mixer scan backward: workspace too small (%zu < %zu)", workspace_bytes, l.total);
   if (!al(x, 16) || !al(dy, 16) || !al(dx, 16) || !al(h_re, esz * l.V) || !al(h_im, esz * l.V) || !al(workspace, 256))
@@ -3806,7 +3819,7 @@ sparc_status sparc_mixer_backward(int64_t batch, int64_t length, int64_t modes, 
   if ((dlast_re == nullptr) != (dlast_im == nullptr)) return fail(SPARC_EINVAL, "mixer backward: dlast_re/dlast_im");
   Layout l = backward_layout(batch, length, modes, io_dtype, kModule, true);
   const size_t esz = io_dtype == SPARC_BF16 ? 2 : 4;
-  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 1, false, true);
+  if (l.split && (!al(h_re, esz * l.V) || !al(h_im, esz * l.V))) l = layout(batch, length, modes, 1, io_dtype, false, true);
   const int cs = l.split ? 0 : coop_steps(batch, length, modes, io_dtype);
   const size_t need = cs ? coop_layout(batch, length, modes, cs).total : l.total;
   if (!workspace || workspace_bytes < need)

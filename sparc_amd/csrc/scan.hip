@@ -3671,7 +3671,10 @@ bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
 // Time segments of the serial kernels: below kSegChains chains (where the
 // look-back kernels would run), T splits into segments of a multiple of 64
-// steps, at least kSegMinSteps long, enough for about kSegTarget workgroups
+// steps, at least kSegMinSteps long, for at most kSegTarget workgroups, which
+// are whole workgroups per CU: a few past that keep their CUs busy for another
+// round (polar, 36 chains, T=8192: 590 us a training step with 540 and 1044
+// workgroups, 512 with 504 and 1008; 35 chains, T=10000: 667 -> 589)
 // (per direction: at B=1, T=65536, M=2048 the forward took 0.376 / 0.397 /
 // 0.426 ms with 512 / 1024 / 2048 workgroups, the backward 0.524 / 0.479 /
 // 0.489 ms).
@@ -3703,7 +3706,7 @@ void choose_serial_segments(int direction, int64_t below, int64_t chains, int64_
   t_seg = static_cast<int>(T);
   if (!want_segments(chains, T, below)) return;
   const int64_t target = kSegTarget[direction ? 1 : 0];
-  int64_t n = std::min((target + chains - 1) / chains, T / kSegMinSteps);
+  int64_t n = std::min(target / chains, T / kSegMinSteps);
   if (n < 2) return;
   int64_t len = (T + n - 1) / n;
   len = (len + kChunk - 1) / kChunk * kChunk;
