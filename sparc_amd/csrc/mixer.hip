@@ -2780,9 +2780,13 @@ Layout layout(int64_t B, int64_t T, int64_t M, int direction, int32_t io, bool g
   if (l.split) l.t_seg = static_cast<int>(T);
   else choose_segments(B, T, l.n_mb, io, l.n_seg, l.t_seg);
   l.R = B * T;
+  // the controls backward in row blocks of 128 where that leaves two
+  // workgroups per CU (fewer partial rows to sum: B=1, T=65536, width 2048
+  // 900 -> 893 us a training step against blocks of 64), else finer ones
   const ControlsLayout cl = controls_layout(l.R, 2 * M, 4);
-  l.n_rb = cl.n_rb;
-  l.rb_rows = cl.rows;
+  const int64_t blocks = (l.R + kCtrlBwdRows - 1) / kCtrlBwdRows;
+  l.rb_rows = blocks * cl.n_cb >= 512 ? kCtrlBwdRows : cl.rows;
+  l.n_rb = static_cast<int>(std::min<int64_t>((l.R + l.rb_rows - 1) / l.rb_rows, kMaxRowBlocks));
   int np = kPieces;
   while (np > 1 && T % (static_cast<int64_t>(np) * kCtrlBwdRows) != 0) np /= 2;
   if (pieces && !split && np > 1 && T > 0 && direction == 1 && !gw && l.n_seg == 1 && l.V == 1) {

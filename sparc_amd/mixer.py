@@ -126,8 +126,8 @@ class _FusedMixer(torch.autograd.Function):
         B, T, W = x.shape
         M = W // 2
         io = _lib.io_code(x.dtype)
-        # eta and delta, the states' planes, and (backward) the gradients share
-        # one allocation each: the library takes addresses, so no views either
+        # eta and delta, and (backward) the gradients share one allocation: the
+        # library takes addresses, so no views either
         controls = torch.empty(2, B, T, dtype=torch.float32, device=dev)
         y = torch.empty_like(x)
         last_re = torch.empty(B, M, dtype=torch.float32, device=dev)
@@ -143,11 +143,12 @@ class _FusedMixer(torch.autograd.Function):
                 B, T, M, io, P(x), *[P(p) for p in params], eta, delta, P(y), P(last_re), P(last_im), P(ws),
                 ws_bytes, _lib.stream_of(dev)), "sparc_mixer_infer")
             return y, last_re, last_im
-        h = torch.empty(2, B, T, M, dtype=x.dtype, device=dev)
+        h_re = torch.empty(B, T, M, dtype=x.dtype, device=dev)
+        h_im = torch.empty_like(h_re)
         _lib.check(lib.sparc_mixer_forward(
-            B, T, M, io, P(x), *[P(p) for p in params], eta, delta, P(y), *_planes(h), P(last_re), P(last_im), P(ws),
+            B, T, M, io, P(x), *[P(p) for p in params], eta, delta, P(y), P(h_re), P(h_im), P(last_re), P(last_im), P(ws),
             ws_bytes, _lib.stream_of(dev)), "sparc_mixer_forward")
-        ctx.save_for_backward(x, *params, controls, h)
+        ctx.save_for_backward(x, *params, controls, h_re, h_im)
         ctx.set_materialize_grads(False)  # unused last-state outputs: NULL, not zero tensors
         ctx.dtypes = [p.dtype for p in (phase_direction, radial_direction, nu_log, theta_log,
                                         write_log_gain, write_phase_response, write_radial_response)]
@@ -156,7 +157,7 @@ class _FusedMixer(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, dlast_re, dlast_im):
-        x, pd, rd, nu, th, wlg, wpr, wrr, controls, h = ctx.saved_tensors
+        x, pd, rd, nu, th, wlg, wpr, wrr, controls, h_re, h_im = ctx.saved_tensors
         lib = _lib.load()
         dev = x.device
         B, T, W = x.shape
@@ -176,7 +177,7 @@ class _FusedMixer(torch.autograd.Function):
         P = _lib.ptr
         _lib.check(lib.sparc_mixer_backward(
             B, T, M, _lib.io_code(x.dtype), P(x), P(pd), P(rd), P(nu), P(th), P(wlg), P(wpr), P(wrr),
-            *_planes(controls), *_planes(h), P(dy), P(dlast_re), P(dlast_im), P(dx),
+            *_planes(controls), P(h_re), P(h_im), P(dy), P(dlast_re), P(dlast_im), P(dx),
             *[P(g) for g in grads], P(ws), ws_bytes, _lib.stream_of(dev)), "sparc_mixer_backward")
         grads = [g if g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes)]
         shape, dt = ctx.energy
