@@ -310,24 +310,27 @@ struct TransitionLane {
     else return row * p.G + m0 / p.gs;
   }
 
-  __device__ __forceinline__ void load_gates(const ScanArgs& p, int64_t gi, float (&g0)[GV], float (&g1)[GV]) const {
-    if constexpr (GM == GATE_MODE) {
-      float tmp[V];
-      unpack<GT, V>(load_raw<GT, V>(p.g0, gi), tmp);
-#pragma unroll
-      for (int v = 0; v < V; ++v) g0[v] = tmp[v];
-      if constexpr (CPLX) {
-        unpack<GT, V>(load_raw<GT, V>(p.g1, gi), tmp);
-#pragma unroll
-        for (int v = 0; v < V; ++v) g1[v] = tmp[v];
-      } else {
-#pragma unroll
-        for (int v = 0; v < V; ++v) g1[v] = 0.0f;
-      }
+  // The gates of one step as they lie in memory, and their conversion apart: a
+  // conversion right after its load would make the wave wait for it before it
+  // issues the next step's loads.
+  using GRaw = typename Raw<GT, GV>::T;
+  __device__ __forceinline__ void load_gates_raw(const ScanArgs& p, int64_t gi, GRaw& r0, GRaw& r1) const {
+    r0 = load_raw<GT, GV>(p.g0, gi);
+    if constexpr (CPLX) r1 = load_raw<GT, GV>(p.g1, gi);
+  }
+  __device__ __forceinline__ void unpack_gates(const GRaw& r0, const GRaw& r1, float (&g0)[GV], float (&g1)[GV]) const {
+    unpack<GT, GV>(r0, g0);
+    if constexpr (CPLX) {
+      unpack<GT, GV>(r1, g1);
     } else {
-      g0[0] = load1<GT>(p.g0, gi);
-      g1[0] = CPLX ? load1<GT>(p.g1, gi) : 0.0f;
+#pragma unroll
+      for (int v = 0; v < GV; ++v) g1[v] = 0.0f;
     }
+  }
+  __device__ __forceinline__ void load_gates(const ScanArgs& p, int64_t gi, float (&g0)[GV], float (&g1)[GV]) const {
+    GRaw r0, r1;
+    load_gates_raw(p, gi, r0, r1);
+    unpack_gates(r0, r1, g0, g1);
   }
 
   // a = transition(g0, g1) for every distinct value
@@ -418,18 +421,28 @@ scan_fwd_kernel(ScanArgs p) {
   tl.init(p, m0, lane_ok);
 
   // ---- load the sub-chunk: inputs, gates, transitions --------------------
+  // Every load is issued before anything is made of one, without branches:
+  // steps past T read row T-1 and lanes past M their block's first element,
+  // and both are discarded below.  (With bf16 gates converted step by step the
+  // wave waited for each step's loads before the next one's: real scan, a gate
+  // per element, B=8, T=4096, M=4096 forward 204 us.)
   RawT wr_raw[S], wi_raw[S];
+  typename TL::GRaw g0_raw[S], g1_raw[S];
+  const uint32_t lane_ld = lane_ok ? lane_bytes : 0u;
+  const int mg = lane_ok ? m0 : mb0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int tc = min(t0 + s, p.T - 1);
+    const int64_t idx = (static_cast<int64_t>(b) * p.T + tc) * p.M + mb0;  // row of the block
+    wr_raw[s] = lb_load<IO, V>(p.w_re, idx, lane_ld);
+    if constexpr (CPLX) wi_raw[s] = lb_load<IO, V>(p.w_im, idx, lane_ld);
+    tl.load_gates_raw(p, tl.gate_index(p, b, tc, mg), g0_raw[s], g1_raw[s]);
+  }
   float g0[S][GV], g1[S][GV];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int t = t0 + s;
-    const bool ok = lane_ok && t < p.T;
-    const int64_t idx = (static_cast<int64_t>(b) * p.T + t) * p.M + mb0;  // row of the block
-    if (ok) {
-      wr_raw[s] = lb_load<IO, V>(p.w_re, idx, lane_bytes);
-      if constexpr (CPLX) wi_raw[s] = lb_load<IO, V>(p.w_im, idx, lane_bytes);
-      tl.load_gates(p, tl.gate_index(p, b, t, m0), g0[s], g1[s]);
-    } else {
+    tl.unpack_gates(g0_raw[s], g1_raw[s], g0[s], g1[s]);
+    if (!(lane_ok && t0 + s < p.T)) {
       float z[V] = {};
       wr_raw[s] = pack<IO, V>(z);
       if constexpr (CPLX) wi_raw[s] = wr_raw[s];
@@ -759,45 +772,53 @@ scan_bwd_kernel(ScanArgs p) {
   TL tl;
   tl.init(p, m0, lane_ok);
 
-  // ---- loads ----------------------------------------------------------------
+  // ---- loads (all issued first, without branches, as in the forward) --------
   RawT wr_raw[S], wi_raw[S], dr_raw[S], di_raw[S];
+  typename TL::GRaw g0_raw[S], g1_raw[S];
+  const uint32_t lane_ld = lane_ok ? lane_bytes : 0u;
+  const int mg = lane_ok ? m0 : mb0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int tc = min(t0 + s, p.T - 1);
+    const int64_t row = static_cast<int64_t>(b) * p.T + tc;
+    const int64_t idx = row * p.M + mb0;  // row of the block
+    if constexpr (SAVED) {
+      if constexpr (!SPARC_LB_SAVED_LATE) {  // y at t-1 (t = 0: own row, replaced by h0)
+        const int64_t pidx = tc > 0 ? idx - p.M : idx;
+        wr_raw[s] = lb_load<IO, V>(p.y_re, pidx, lane_ld);
+        if constexpr (CPLX) wi_raw[s] = lb_load<IO, V>(p.y_im, pidx, lane_ld);
+      }
+    } else {
+      wr_raw[s] = lb_load<IO, V>(p.w_re, idx, lane_ld);
+      if constexpr (CPLX) wi_raw[s] = lb_load<IO, V>(p.w_im, idx, lane_ld);
+    }
+    if (relu_out) {
+      dr_raw[s] = lb_load<IO, V>(p.dy_re, row * 2 * p.M + mb0, lane_ld);
+      di_raw[s] = lb_load<IO, V>(p.dy_re, row * 2 * p.M + p.M + mb0, lane_ld);
+    } else {
+      dr_raw[s] = lb_load<IO, V>(p.dy_re, idx, lane_ld);
+      if constexpr (CPLX) di_raw[s] = lb_load<IO, V>(p.dy_im, idx, lane_ld);
+    }
+    tl.load_gates_raw(p, tl.gate_index(p, b, tc, mg), g0_raw[s], g1_raw[s]);
+  }
   float g0[S][GV], g1[S][GV];
   bool rst[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int t = t0 + s;
-    const bool ok = lane_ok && t < p.T;
-    const int64_t row = static_cast<int64_t>(b) * p.T + t;
-    const int64_t idx = row * p.M + mb0;  // row of the block
-    if (ok) {
-      if constexpr (SAVED) {
-        if constexpr (!SPARC_LB_SAVED_LATE) {  // y at t-1 (t = 0: own row, replaced by h0)
-          const int64_t pidx = t > 0 ? idx - p.M : idx;
-          wr_raw[s] = lb_load<IO, V>(p.y_re, pidx, lane_bytes);
-          if constexpr (CPLX) wi_raw[s] = lb_load<IO, V>(p.y_im, pidx, lane_bytes);
-        }
-      } else {
-        wr_raw[s] = lb_load<IO, V>(p.w_re, idx, lane_bytes);
-        if constexpr (CPLX) wi_raw[s] = lb_load<IO, V>(p.w_im, idx, lane_bytes);
-      }
-      if (relu_out) {
-        dr_raw[s] = lb_load<IO, V>(p.dy_re, row * 2 * p.M + mb0, lane_bytes);
-        di_raw[s] = lb_load<IO, V>(p.dy_re, row * 2 * p.M + p.M + mb0, lane_bytes);
-      } else {
-        dr_raw[s] = lb_load<IO, V>(p.dy_re, idx, lane_bytes);
-        if constexpr (CPLX) di_raw[s] = lb_load<IO, V>(p.dy_im, idx, lane_bytes);
-      }
-      tl.load_gates(p, tl.gate_index(p, b, t, m0), g0[s], g1[s]);
-    } else {
+    tl.unpack_gates(g0_raw[s], g1_raw[s], g0[s], g1[s]);
+    if (!(lane_ok && t < p.T)) {
       float z[V] = {};
-      wr_raw[s] = pack<IO, V>(z);
-      wi_raw[s] = wr_raw[s];
-      dr_raw[s] = wr_raw[s];
-      di_raw[s] = wr_raw[s];
+      dr_raw[s] = pack<IO, V>(z);
+      di_raw[s] = dr_raw[s];
+      if constexpr (!SAVED || !SPARC_LB_SAVED_LATE) {
+        wr_raw[s] = dr_raw[s];
+        wi_raw[s] = dr_raw[s];
+      }
 #pragma unroll
       for (int v = 0; v < GV; ++v) { g0[s][v] = 0.0f; g1[s][v] = 0.0f; }
     }
-    if (p.segpos) rst[s] = (t < p.T) && p.segpos[row] == 0;
+    if (p.segpos) rst[s] = (t < p.T) && p.segpos[static_cast<int64_t>(b) * p.T + t] == 0;
     else rst[s] = reset_first && t == 0;
   }
   float a_r[S][AV], a_i[S][AV];
