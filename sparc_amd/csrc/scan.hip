@@ -1374,11 +1374,27 @@ struct SubChunk {
   using RawT = typename Raw<IO, V>::T;
   static constexpr bool CPLX = TL::CPLX;
   static constexpr int GV = TL::GV;
+  using GRaw = typename TL::GRaw;
   RawT wr[S], wi[S];
-  float g0[S][GV], g1[S][GV];
+  GRaw q0[S], q1[S];  // gates as loaded: converting them here would wait for them
 
-  // loads steps [t0, t0 + S) of row b for the lane's modes
-  __device__ __forceinline__ void load(const ScanArgs& p, const TL& tl, int b, int t0, int m0, bool lane_ok) {
+  // loads steps [t0, t0 + S) of row b for the lane's modes; `full`: every lane
+  // and every step is in range, so no load stands under a branch.  For bf16
+  // only (one mode per lane, elementwise gates, M = 4001, fwd+bwd: complex
+  // 1766 -> 1240 us, real 1416 -> 1069); fp32 measured the same either way
+  // and spills where it already fills the registers (P1 1840 -> 1867).
+  static constexpr bool kFull = sizeof(IO) == 2;
+  __device__ __forceinline__ void load(const ScanArgs& p, const TL& tl, int b, int t0, int m0, bool lane_ok, bool full) {
+    if (kFull && full) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const int64_t idx = (static_cast<int64_t>(b) * p.T + t0 + s) * p.M + m0;
+        wr[s] = load_raw<IO, V>(p.w_re, idx);
+        if constexpr (CPLX) wi[s] = load_raw<IO, V>(p.w_im, idx);
+        tl.load_gates_raw(p, tl.gate_index(p, b, t0 + s, m0), q0[s], q1[s]);
+      }
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int t = t0 + s;
@@ -1386,15 +1402,20 @@ struct SubChunk {
         const int64_t idx = (static_cast<int64_t>(b) * p.T + t) * p.M + m0;
         wr[s] = load_raw<IO, V>(p.w_re, idx);
         if constexpr (CPLX) wi[s] = load_raw<IO, V>(p.w_im, idx);
-        tl.load_gates(p, tl.gate_index(p, b, t, m0), g0[s], g1[s]);
+        tl.load_gates_raw(p, tl.gate_index(p, b, t, m0), q0[s], q1[s]);
       } else {
-        float z[V] = {};
+        float z[V] = {}, zg[GV] = {};
         wr[s] = pack<IO, V>(z);
         wi[s] = wr[s];
-#pragma unroll
-        for (int v = 0; v < GV; ++v) { g0[s][v] = 0.0f; g1[s][v] = 0.0f; }
+        q0[s] = pack<typename TL::GT, GV>(zg);
+        q1[s] = q0[s];
       }
     }
+  }
+
+  __device__ __forceinline__ void gates(const TL& tl, float (&g0)[S][GV], float (&g1)[S][GV]) const {
+#pragma unroll
+    for (int s = 0; s < S; ++s) tl.unpack_gates(q0[s], q1[s], g0[s], g1[s]);
   }
 };
 
@@ -1524,17 +1545,20 @@ chain_fwd_kernel(ScanArgs p) {
     ci[v] = (CPLX && p.h0_im && lane_ok) ? p.h0_im[hi] : 0.0f;
   }
   SC buf[2];
-  buf[0].load(p, tl, b, wave * S, m0, lane_ok);
+  const bool block_full = (mb + 1) * MB <= p.M;  // wave-uniform
+  buf[0].load(p, tl, b, wave * S, m0, lane_ok, block_full && wave * S + S <= p.T);
   for (int c0 = 0; c0 < p.n_chunks; c0 += 2) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int c = c0 + h;
       if (c >= p.n_chunks) break;
       const int t0 = c * C + wave * S;
-      if (c + 1 < p.n_chunks) buf[1 - h].load(p, tl, b, t0 + C, m0, lane_ok);
+      if (c + 1 < p.n_chunks) buf[1 - h].load(p, tl, b, t0 + C, m0, lane_ok, block_full && t0 + C + S <= p.T);
       float a_r[S][AV], a_i[S][AV];
       bool rst[S];
-      make_transitions<TL, S>(p, tl, b, t0, lane_ok, reset_first, buf[h].g0, buf[h].g1, a_r, a_i, rst);
+      float g0[S][TL::GV], g1[S][TL::GV];
+      buf[h].gates(tl, g0, g1);
+      make_transitions<TL, S>(p, tl, b, t0, lane_ok, reset_first, g0, g1, a_r, a_i, rst);
       local_maps<CPLX, IO, V, AV, S, NQ>(buf[h].wr, buf[h].wi, a_r, a_i, s_pq[h][wave], lane);
       __syncthreads();
       // start state of this wave, and the state after the chunk (same arithmetic in every wave)
@@ -1641,16 +1665,18 @@ chain_bwd_kernel(ScanArgs p) {
 #pragma unroll
   for (int v = 0; v < (P1 ? V : 1); ++v) { acc_nu[v] = 0.0f; acc_th[v] = 0.0f; }
 
+  const bool block_full = (mb + 1) * MB <= p.M;  // wave-uniform
   SC buf[2];
   RawT dr[2][S], di[2][S];
   float hs[2][V * NH];  // state entering the chunk (saved by the forward)
   auto load_all = [&](int hb, int c) {
     const int t0 = c * C + wave * S;
-    buf[hb].load(p, tl, b, t0, m0, lane_ok);
+    const bool full = SC::kFull && block_full && t0 + S <= p.T;
+    buf[hb].load(p, tl, b, t0, m0, lane_ok, full);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int t = t0 + s;
-      if (lane_ok && t < p.T) {
+      if (full || (lane_ok && t < p.T)) {
         const int64_t row = static_cast<int64_t>(b) * p.T + t;
         if (relu_out) {
           dr[hb][s] = load_raw<IO, V>(p.dy_re, row * 2 * p.M + m0);
@@ -1689,7 +1715,9 @@ chain_bwd_kernel(ScanArgs p) {
       if (c - 1 >= 0) load_all(1 - h, c - 1);
       float a_r[S][AV], a_i[S][AV];
       bool rst[S];
-      make_transitions<TL, S>(p, tl, b, t0, lane_ok, reset_first, buf[h].g0, buf[h].g1, a_r, a_i, rst);
+      float g0[S][TL::GV], g1[S][TL::GV];
+      buf[h].gates(tl, g0, g1);
+      make_transitions<TL, S>(p, tl, b, t0, lane_ok, reset_first, g0, g1, a_r, a_i, rst);
       local_maps<CPLX, IO, V, AV, S, NQ>(buf[h].wr, buf[h].wi, a_r, a_i, s_fq[wave], lane);
       __syncthreads();  // B1: forward maps visible
       float hr[V], hi[V];
@@ -1800,8 +1828,8 @@ chain_bwd_kernel(ScanArgs p) {
           }
           if (!live) { gar = 0.0f; gai = 0.0f; }
           if constexpr (P1) {
-            const float E = fast_exp(buf[h].g0[s][0]);
-            const float delta = buf[h].g1[s][0];
+            const float E = fast_exp(g0[s][0]);
+            const float delta = g1[s][0];
             const float lrad = -tl.nu[v] * E;
             const float em = expm1_nonpos(lrad);  // rho - 1 (as in the forward)
             const float rho = 1.0f + em;
@@ -1816,7 +1844,7 @@ chain_bwd_kernel(ScanArgs p) {
           } else if constexpr (tr_kind(TR) == TR_POLAR) {
             const float ar = a_r[s][av], ai = a_i[s][av];
             float cphi, sphi;
-            sincos_moderate(buf[h].g1[s][gv], sphi, cphi);
+            sincos_moderate(g1[s][gv], sphi, cphi);
             d0[gv] += gar * cphi + gai * sphi;
             d1[gv] += -gar * ai + gai * ar;
           } else if constexpr (tr_kind(TR) == TR_CART) {
@@ -2048,20 +2076,29 @@ chain_fwd_fast_kernel(ScanArgs p) {
     }
   }
 
+  const bool block_full = (mb + 1) * MB <= p.M;  // wave-uniform
   RawT wr[2][S], wi[2][S];
   GateBlock<S> gb[2];
   auto load_chunk = [&](int hb, int c) {
     const int t0 = c * C + wave * S;
     const int64_t off = wave_uniform(((row0 + t0) * p.M + mbase) * ESZ);
+    if (block_full && t0 + S <= p.T) {  // no load under a branch
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      if (t0 + s < p.T && lane_ok) {
+      for (int s = 0; s < S; ++s) {
         wr[hb][s] = ldb<RawT>(p.w_re, off + s * stride, lane_bytes);
         if constexpr (CPLX) wi[hb][s] = ldb<RawT>(p.w_im, off + s * stride, lane_bytes);
-      } else {
-        float z[V] = {};
-        wr[hb][s] = pack<IO, V>(z);
-        wi[hb][s] = wr[hb][s];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if (t0 + s < p.T && lane_ok) {
+          wr[hb][s] = ldb<RawT>(p.w_re, off + s * stride, lane_bytes);
+          if constexpr (CPLX) wi[hb][s] = ldb<RawT>(p.w_im, off + s * stride, lane_bytes);
+        } else {
+          float z[V] = {};
+          wr[hb][s] = pack<IO, V>(z);
+          wi[hb][s] = wr[hb][s];
+        }
       }
     }
     load_gate_pairs<TR, GateT<TR, IO>, S>(p, b, t0, g_base, gpw, lane, gb[hb]);
