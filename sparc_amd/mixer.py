@@ -126,8 +126,8 @@ class _FusedMixer(torch.autograd.Function):
         B, T, W = x.shape
         M = W // 2
         io = _lib.io_code(x.dtype)
-        # eta and delta, and (backward) the gradients share one allocation: the
-        # library takes addresses, so no views either
+        # eta and delta share one allocation: the library takes addresses, so no
+        # views either
         controls = torch.empty(2, B, T, dtype=torch.float32, device=dev)
         y = torch.empty_like(x)
         last_re = torch.empty(B, M, dtype=torch.float32, device=dev)
@@ -170,8 +170,9 @@ class _FusedMixer(torch.autograd.Function):
             dlast_re = z if dlast_re is None else dlast_re.float().contiguous()
             dlast_im = z.clone() if dlast_im is None else dlast_im.float().contiguous()
         dx = torch.empty_like(x)
-        sizes = (W + 1, W + 1, M, M, M, M, M)
-        grads = torch.empty(2 * (W + 1) + 5 * M, dtype=torch.float32, device=dev).split(sizes)
+        # a tensor of its own for each: views of one buffer would share a version
+        # counter, refuse detach_() and lie off 16 bytes (W + 1 is odd)
+        grads = [torch.empty(n, dtype=torch.float32, device=dev) for n in (W + 1, W + 1, M, M, M, M, M)]
         ws_bytes = lib.sparc_mixer_workspace_bytes(B, T, M, 1)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         P = _lib.ptr
