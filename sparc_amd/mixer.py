@@ -101,8 +101,9 @@ def _keeps_gradients(*tensors) -> bool:
 
 
 def _planes(t: torch.Tensor) -> tuple[int, int]:
-    """Addresses of the two halves of a [2, ...] tensor (NULL where empty)."""
-    base = t.data_ptr()
+    """Addresses of the two halves of a contiguous [2, ...] tensor (NULL where
+    empty; ValueError for another layout, which a saved-tensor hook may give)."""
+    base = _lib.ptr(t)
     return base, base + t.numel() // 2 * t.element_size()
 
 

@@ -306,3 +306,16 @@ def test_module_paths_reject_wrong_parameter_shapes():
         m.write_log_gain = torch.nn.Parameter(torch.zeros(6))
     with pytest.raises(ValueError, match="write_log_gain"):
         latest_sparc_decode(m, torch.zeros(2, 16), (torch.zeros(2, 8), torch.zeros(2, 8)))
+
+
+def test_control_planes_refuse_non_contiguous():
+    """The module's backward takes the two control planes of one saved tensor by
+    address: another layout (as a saved-tensor hook may give) is refused."""
+    from sparc_amd.mixer import _planes
+    t = torch.zeros(2, 3, 4)
+    a, b = _planes(t)
+    assert a == t.data_ptr() and b == t[1].data_ptr()
+    with pytest.raises(ValueError):
+        _planes(t.transpose(1, 2))
+    with pytest.raises(ValueError):
+        _planes(torch.zeros(2, 1, 1).expand(2, 3, 4))
