@@ -3483,6 +3483,7 @@ struct Plan {
   bool fast = false;  // chain kernels specialised for lane-shared gates
   bool serial = false;  // one wave per chain (lane-shared gates, many chains)
   bool g32 = false;  // fp32 gates beside bf16 I/O
+  bool recompute = false;  // backward: the states from w in fp32 although y was saved
   int n_chunks = 0, n_mblocks = 0, n_chains = 0;
   int n_seg = 1, t_seg = 0;  // time segments of the serial kernels (n_seg > 1: few chains)
   int64_t n_tiles = 0;
@@ -3846,6 +3847,16 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   const bool auto_plan = !force_l && !force_c && !force_s;
   const bool cplx_tr = d->transition != SPARC_TRANSITION_REAL;
   const bool bf16_io = d->io_dtype == SPARC_BF16;
+  // fp32 gates have fp32 gradients, and states read back in bf16 would leave
+  // them 8 bits (polar, B=8, T=70, 1024 groups of 16: d r 1.66e-3 off its 64-bit
+  // values, recomputed 1.4e-7).  So the chain kernels' backward recomputes the
+  // states in fp32 for such gates (polar, B=8, T=4096, 1024 groups of 16: 1641
+  // us, 1195 from the saved states); with fewer than kChainMin chains the
+  // automatic plan reads them back, as the look-back tiles do.
+  bool recompute = false;
+  if (g32 && direction == 1 && !force_l && (try_v(vmax) || try_v(1)))
+    recompute = force_c || force_s || d->batch * ((M + 64 * V - 1) / (64 * V)) >= kChainMin;
+  if (recompute) allow_wide = allow_seg = false;
   // Complex bf16 with lane-shared gates: the serial kernels stream 8 bytes
   // per lane and plane (4 modes) when that still leaves enough chains, or
   // over time segments when the chains are few.
@@ -3865,6 +3876,7 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   pl->V = V;
   pl->gm = gm;
   pl->g32 = g32;
+  pl->recompute = recompute;
   pl->n_chunks = static_cast<int>((d->length + kChunk - 1) / kChunk);
   pl->n_mblocks = static_cast<int>((M + 64 * V - 1) / (64 * V));
   pl->n_chains = static_cast<int>(d->batch * pl->n_mblocks);
@@ -4154,7 +4166,8 @@ sparc_status sparc_scan_backward(const sparc_scan_desc* d, const void* gate0, co
   if (cplx && ((dh0_re == nullptr) != (dh0_im == nullptr))) return fail(SPARC_EINVAL, "dh0_re/dh0_im must both be given");
   if (dh0_re && !h0_re) return fail(SPARC_EINVAL, "dh0 requested without h0");
   if (cplx && y_re && !y_im && !relu) return fail(SPARC_EINVAL, "y_im is required with y_re");
-  const bool saved = y_re && !relu;  // y = h (rounded to the I/O dtype) only without the relu epilogue
+  // y = h (rounded to the I/O dtype) only without the relu epilogue
+  const bool saved = y_re && !relu && !pl.recompute;
   const void* ptrs[] = {w_re, w_im, dy_re, relu ? nullptr : dy_im, dw_re, dw_im,
                         saved ? y_re : nullptr, saved ? y_im : nullptr};
   if (sparc_status s = check_io_ptrs(d, pl, ptrs, 8)) return s;

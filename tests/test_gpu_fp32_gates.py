@@ -58,3 +58,52 @@ def test_fp32_gates_lane_shared(transition, B, T, G, N, plan, reset):
             ops.set_algorithm("auto")
     for k, (a, b) in enumerate(zip(got["auto"], got["lookback"])):
         assert rel_err(a, b) <= 2.0 ** -7, f"tensor {k}: {rel_err(a, b):.3g}"
+
+
+def _gate_gradients_64(gates, w, dy, N):
+    """d gates of h_t = a_t h_{t-1} + w_t (polar, or real with one gate) in float64."""
+    gates = [t.double().requires_grad_() for t in gates]
+    w, dy = [t.double() for t in w], [t.double() for t in dy]
+    a = torch.polar(*gates) if len(gates) == 2 else gates[0]
+    a = a.repeat_interleave(N, dim=-1)
+    w, dy = (torch.complex(*t) if len(t) == 2 else t[0] for t in (w, dy))
+    h, hs = torch.zeros_like(w[:, 0]), []
+    for t in range(w.shape[1]):
+        h = a[:, t] * h + w[:, t]
+        hs.append(h)
+    loss = (torch.stack(hs, 1) * dy.conj()).real.sum()
+    return torch.autograd.grad(loss, gates)
+
+
+@pytest.mark.parametrize("transition,B,T,G,N,algo", [
+    ("polar", 8, 70, 1024, 16, "auto"),     # 1024 chains of 128 modes
+    ("polar", 8, 70, 512, 16, "auto"),      # 512 chains, the fewest whose states are recomputed
+    ("real", 8, 70, 1024, 16, "auto"),      # 512 chains of 256 modes
+    ("polar", 2, 130, 16, 16, "chain"),
+    ("real", 2, 130, 16, 16, "serial"),
+])
+def test_fp32_gate_gradients_from_fp32_states(transition, B, T, G, N, algo):
+    """fp32 gates get fp32 gradients: from states recomputed in fp32, not from
+    the saved bf16 output, which is 2^-9 off.  A state is a sum of products
+    that fades within some 20 steps, each rounded to 2^-24 of its value, as are
+    the adjoint and the transition: 2e-6 is some thirty such roundings, and a
+    thousandth of what one bf16 rounding of the states costs."""
+    print(f"[case] fp32 gate gradients {transition} B={B} T={T} G={G} N={N} {algo}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + G)
+    r = torch.sigmoid(2.0 + torch.randn(B, T, G, device="cuda", generator=g))
+    phi = (torch.rand(B, T, G, device="cuda", generator=g) * 2 - 1) * 3.14159
+    gates = [r, phi] if transition == "polar" else [r]
+    w, dy = ([torch.randn(B, T, G * N, device="cuda", generator=g).bfloat16() for _ in gates] for _ in range(2))
+    want = _gate_gradients_64(gates, w, dy, N)
+    ops.set_algorithm(algo)
+    try:
+        leaves = [t.clone().requires_grad_() for t in gates]
+        y, _ = ops.chunk_scan(transition, leaves[0], leaves[1] if len(leaves) == 2 else None, w[0],
+                              w[1] if len(leaves) == 2 else None)
+        got = torch.autograd.grad(list(y) if len(leaves) == 2 else [y], leaves, dy)
+    finally:
+        ops.set_algorithm("auto")
+    for a, b in zip(got, want):
+        err = ((a.double() - b).norm() / b.norm()).item()
+        print(f"[case] off by {err:.3g}", flush=True)
+        assert err <= 2e-6
