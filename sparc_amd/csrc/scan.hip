@@ -3804,6 +3804,20 @@ void plan_lane_shared(bool cplx, bool bf16, bool wide, bool recompute_bwd, int64
   }
 }
 
+// Whether the automatic plan takes time segments for fp32 gates beside bf16
+// I/O (chains of 256 modes).  Their gates are half the bytes of a tile or more
+// and the look-back reads them once, the summary and the replay twice.
+// Measured (us, look-back against segments): polar forward, 16 chains, T=1024
+// 33 and 94, T=4096 64 and 95, T=16384 179 and 197, 96 chains, T=4096 233 and
+// 296, but 4 chains, T=65536 230 and 193; its backward, 16 chains, T=4096 94 and
+// 115, T=8192 157 and 137, 64 chains, T=1024 90 and 121, T=4096 268 and 223;
+// real backward, 16 chains, T=8192 85 and 88, T=16384 146 and 121, 32 chains,
+// T=8192 131 and 118, 96 chains, T=4096 171 and 181.
+bool g32_segments(int direction, bool real, int64_t chains, int64_t T) {
+  if (chains <= 4 && T > 32768) return true;
+  return direction == 1 && (real ? chains <= 32 && chains * T >= (1 << 18) : chains * T >= (1 << 17));
+}
+
 // Chooses V and the gate mode; fills sizes.  Returns an error message or NULL.
 // allow_wide: the caller can use the 4-mode serial kernels (their pointers are
 // 8-byte aligned and, backward, the states come from the saved output).
@@ -3865,7 +3879,9 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
       gs % kWideV == 0 && (64 * kWideV) % gs == 0 && is_pow2(gs / kWideV) &&
       (64 * kWideV) / gs <= sparc::kFastMaxGpw && !force_l && !force_c && allow_wide) {
     const int64_t chains = d->batch * ((M + 64 * kWideV - 1) / (64 * kWideV));
-    wide = force_s || chains >= kSerialWideMin || (allow_seg && want_segments(chains, d->length, kSegBelowCplx));
+    wide = force_s || chains >= kSerialWideMin ||
+           (allow_seg && want_segments(chains, d->length, kSegBelowCplx) &&
+            (!g32 || g32_segments(direction, false, chains, d->length)));
   }
   if (wide) {
     V = kWideV;
@@ -3893,6 +3909,7 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
     seg_below = kSegChains;
   } else if (auto_plan && lane_shared) {
     plan_lane_shared(cplx_tr, bf16_io, wide, direction == 1 && !allow_seg, seg_below, serial_min, chain_min);
+    if (g32 && !g32_segments(direction, !cplx_tr, pl->n_chains, d->length)) seg_below = 0;
   }
   pl->n_seg = 1;
   pl->t_seg = static_cast<int>(d->length);

@@ -23,9 +23,12 @@ pytestmark = pytest.mark.gpu
     ("polar", 4, 130, 512, 16, "chain"),
     ("real", 4, 130, 2048, 8, "chain"),
     ("real", 16, 129, 2048, 8, "serial"),
-    ("polar", 1, 1100, 64, 16, "time segments"),
-    ("cartesian", 2, 640, 33, 8, "time segments, lanes past M"),
-    ("real", 1, 777, 48, 32, "time segments"),
+    ("polar", 1, 1100, 64, 16, "look-back"),
+    ("cartesian", 2, 640, 33, 8, "look-back, lanes past M"),
+    ("real", 1, 777, 48, 32, "look-back"),
+    ("polar", 8, 1100, 240, 16, "backward in time segments"),
+    ("cartesian", 1, 33000, 17, 16, "time segments, lanes past M"),
+    ("real", 1, 33000, 16, 16, "time segments"),
 ])
 @pytest.mark.parametrize("reset", [False, True])
 def test_fp32_gates_lane_shared(transition, B, T, G, N, plan, reset):
