@@ -3730,13 +3730,19 @@ bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
 // Time segments of the serial kernels: below kSegChains chains (where the
 // look-back kernels would run), T splits into segments of a multiple of 64
-// steps, at least kSegMinSteps long, for at most kSegTarget workgroups, which
-// are whole workgroups per CU: a few past that keep their CUs busy for another
-// round (polar, 36 chains, T=8192: 590 us a training step with 540 and 1044
-// workgroups, 512 with 504 and 1008; 35 chains, T=10000: 667 -> 589)
-// (per direction: at B=1, T=65536, M=2048 the forward took 0.376 / 0.397 /
-// 0.426 ms with 512 / 1024 / 2048 workgroups, the backward 0.524 / 0.479 /
-// 0.489 ms).
+// steps, at least kSegMinSteps long, for about kSegTarget workgroups (per
+// direction: at B=1, T=65536, M=2048 the forward took 0.376 / 0.397 / 0.426 ms
+// with 512 / 1024 / 2048 workgroups, the backward 0.524 / 0.479 / 0.489 ms).
+// Complex: at most kSegTarget, that is at most two (backward four) per CU: a
+// few past that keep their CUs busy for another round (polar, 36 chains,
+// T=8192: 590 us a training step with 540 and 1044 workgroups, 512 with 504
+// and 1008; 35 chains, T=10000: 667 -> 589).  The real forward, whose
+// workgroups are lighter, gains more from another segment than it loses to a
+// few past the target (171 chains, T=4096: 297 us with 513 workgroups, 377
+// with 342; 255 chains 349 and 395; 86 chains, T=16384: 548 with 516, 613 with
+// 430), while they still leave two segments; its backward measured the same
+// either way (171 chains 333 and 348, 127 chains, T=16384 871 and 835) up to
+// there and 6 to 12 % faster with the finer ones above (ALGO_SERIAL only).
 #ifndef SPARC_SERIAL_SEG_CHAINS
 #define SPARC_SERIAL_SEG_CHAINS 512
 #endif
@@ -3753,19 +3759,20 @@ constexpr int64_t kSegChains = SPARC_SERIAL_SEG_CHAINS;
 constexpr int64_t kSegTarget[2] = {SPARC_SERIAL_SEG_TARGET_FWD, SPARC_SERIAL_SEG_TARGET_BWD};
 constexpr int64_t kSegMinSteps = SPARC_SERIAL_SEG_MIN;
 static_assert(kSegMinSteps % 64 == 0 && kSegChains <= kSegTarget[0] && kSegChains <= kSegTarget[1],
-              "segments of whole chunks, at least two");
+              "segments of whole chunks");
 
 bool want_segments(int64_t chains, int64_t T, int64_t below = kSegChains) {
   return chains < below && T >= 2 * kSegMinSteps;
 }
 
 // n >= 2 segments of t_seg steps (a multiple of the saved-state chunk), or 1
-void choose_serial_segments(int direction, int64_t below, int64_t chains, int64_t T, int& n_seg, int& t_seg) {
+void choose_serial_segments(int direction, bool real, int64_t below, int64_t chains, int64_t T, int& n_seg, int& t_seg) {
   n_seg = 1;
   t_seg = static_cast<int>(T);
   if (!want_segments(chains, T, below)) return;
   const int64_t target = kSegTarget[direction ? 1 : 0];
-  int64_t n = std::min(target / chains, T / kSegMinSteps);
+  const bool past = real && (direction == 0) == (2 * chains <= kSegTarget[0]);  // may pass the target by a few
+  int64_t n = std::min((target + (past ? chains - 1 : 0)) / chains, T / kSegMinSteps);
   if (n < 2) return;
   int64_t len = (T + n - 1) / n;
   len = (len + kChunk - 1) / kChunk * kChunk;
@@ -3914,7 +3921,7 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   pl->n_seg = 1;
   pl->t_seg = static_cast<int>(d->length);
   if (allow_seg && lane_shared && seg_below > 0 && (wide || !cplx_tr || force_s))
-    choose_serial_segments(direction, seg_below, pl->n_chains, d->length, pl->n_seg, pl->t_seg);
+    choose_serial_segments(direction, !cplx_tr, seg_below, pl->n_chains, d->length, pl->n_seg, pl->t_seg);
   pl->serial = wide || pl->n_seg > 1 || (lane_shared && (force_s || (auto_plan && pl->n_chains >= serial_min)));
   pl->chain = pl->serial || force_c || force_s || (auto_plan && pl->n_chains >= chain_min);
   pl->fast = pl->chain && lane_shared;
