@@ -1545,7 +1545,9 @@ chain_fwd_kernel(ScanArgs p) {
     ci[v] = (CPLX && p.h0_im && lane_ok) ? p.h0_im[hi] : 0.0f;
   }
   SC buf[2];
-  const bool block_full = (mb + 1) * MB <= p.M;  // wave-uniform
+  // wave-uniform; the P1 forward keeps the guarded loads (its registers are
+  // full: B=8, T=2048, M=8192, 512 gate pairs a token 396 us, 417 without)
+  const bool block_full = tr_kind(TR) != TR_P1 && (mb + 1) * MB <= p.M;
   buf[0].load(p, tl, b, wave * S, m0, lane_ok, block_full && wave * S + S <= p.T);
   for (int c0 = 0; c0 < p.n_chunks; c0 += 2) {
 #pragma unroll
