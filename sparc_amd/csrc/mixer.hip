@@ -215,8 +215,10 @@ __device__ __forceinline__ int p1_keep(const Args& a, int b, int t) {
 struct ChainPos {
   int b, mb, seg, t_begin, t_end;
 };
-__device__ __forceinline__ ChainPos chain_pos(const Args& a) {
-  const int idx = xcd_swizzle(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+// chain `k` of the workgroup's NG
+template <int NG = 1>
+__device__ __forceinline__ ChainPos chain_pos(const Args& a, int k = 0) {
+  const int idx = xcd_swizzle(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * NG + k;
   const int n_chains = a.B * a.n_mb;
   const int sj = idx / n_chains, chain = idx - sj * n_chains;
   ChainPos c;
@@ -1277,8 +1279,16 @@ mixer_fwd_split_kernel(Args a) {
 // block's gradients are NaN.  Replaces the controls-backward launches and
 // the dx round trip between them (sparc-kernal/backward/control.py:10-89 for
 // the controls' chain rule).
-template <typename IO, int V, int kS, bool SUMMARY, int MODE>
-__global__ void __launch_bounds__(64, (MODE & 3) == kPlanes && kS >= 16 ? 1 : 2)
+//
+// NG chains per workgroup, one wave each (they share nothing).  Single-wave
+// workgroups spread evenly over the CUs but not over a CU's SIMDs: with 1024
+// of them, 4 per CU, between none and 107 SIMDs held two waves, depending on
+// what ran before, and the launch lasts as long as those (HW_ID of each
+// workgroup; module, 512 chains of 128 modes, T=512, bf16 276 against 378 us,
+// P1, 1024 chains, T=4096, bf16 1250 against 1640).  The waves of one
+// workgroup take a SIMD each, so grids of about a wave per SIMD group four.
+template <typename IO, int V, int kS, bool SUMMARY, int MODE, int NG = 1>
+__global__ void __launch_bounds__(64 * NG, (MODE & 3) == kPlanes && kS >= 16 ? 1 : 2)
 mixer_bwd_kernel(Args a) {
   using RawT = typename Raw<IO, V>::T;
   constexpr int ESZ = sizeof(IO);
@@ -1291,9 +1301,13 @@ mixer_bwd_kernel(Args a) {
   static_assert(GW || !RST, "resets in the P1 scan only");
   static_assert(!COOP || (CM == kModule && V == 1 && !SUMMARY), "one-launch form: the module, one mode per lane");
   constexpr int kSumLoad = SUMMARY ? CPOL_DEFAULT : CPOL_NT;  // as in mixer_fwd_kernel
-  __shared__ float4 tok[64];  // the block's per-step values (run_block)
-  const int lane = threadIdx.x;
-  const ChainPos cp = chain_pos(a);
+  static_assert(NG == 1 || !SUMMARY, "grouped chains without time segments only");
+  const int wave = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  __shared__ float4 toks[NG][64];
+  float4 (&tok)[64] = toks[wave];  // the block's per-step values (run_block)
+  const int lane = threadIdx.x & 63;
+  const ChainPos cp = chain_pos<NG>(a, wave);
+  if (NG > 1 && cp.seg > 0) return;  // the last workgroup's waves past the last chain (wave-uniform; no barriers below)
   const int b = cp.b, mb = cp.mb, t_begin = cp.t_begin, t_end = cp.t_end;
   const int m0 = mb * MB + lane * V;
   const bool lane_ok = m0 < a.M;
@@ -1323,7 +1337,8 @@ mixer_bwd_kernel(Args a) {
   // k % L), the next such gradient to use (loaded one block ahead) and the
   // block this chain is to reduce and has not yet (-1: none)
   constexpr int L = COOP ? kCoopLag<IO> : 1;
-  __shared__ typename CoopRing<IO>::T cring[L][COOP ? kS : 1][64];
+  __shared__ typename CoopRing<IO>::T crings[NG][L][COOP ? kS : 1][64];
+  auto& cring = crings[wave];
   float cu[4], ad[4], dpn[COOP ? 2 * kS : 1];
   int pend = -1;
   if constexpr (COOP) {
@@ -2616,6 +2631,15 @@ constexpr int64_t kSegChains = SPARC_MIXER_SEG_CHAINS;  // segment below this ma
 constexpr int64_t kSimds = 1024;
 constexpr int64_t kMinSegSteps = SPARC_MIXER_SEG_MIN;  // segments shorter than this only to fill rounds of the SIMDs
 constexpr int64_t kAlignedSegSteps = 64;
+// Grids that group four chains per workgroup (mixer_bwd_kernel, NG): about one
+// wave for each SIMD, above which some SIMDs hold two waves in any case.
+// light: the bf16 P1 scan without resets, from half of that on (T=255, 576
+// chains 107 us, grouped 89; 832 chains 111 and 91); the other kernels are
+// faster with a wave per workgroup on more CUs there (fp32 P1, 520 chains 105
+// and 122, module, 264 chains 142 and 156).
+bool bwd_grouped(int64_t waves, bool light = false) {
+  return waves > (light ? kSimds / 2 : kSimds - kSimds / 16) && waves <= kSimds;
+}
 int mixer_v(int64_t B, int64_t T, int64_t M, int direction, bool gw) {
   const int fixed = direction == 0 ? SPARC_MIXER_FWD_V : gw ? SPARC_P1_BWD_V : SPARC_MIXER_BWD_V;
   if (fixed == 1 || M % 2) return 1;
@@ -2625,11 +2649,12 @@ int mixer_v(int64_t B, int64_t T, int64_t M, int direction, bool gw) {
   if (direction == 1) return segmented ? 2 : 1;
   return chains2 >= 1280 || segmented ? 2 : 1;
 }
-void choose_segments(int64_t B, int64_t T, int n_mb, int32_t io, int& n_seg, int& t_seg) {
+void choose_segments(int64_t B, int64_t T, int n_mb, int direction, int32_t io, bool gw, int& n_seg, int& t_seg) {
   n_seg = 1;
   t_seg = static_cast<int>(T > 0 ? T : 1);
   const int64_t chains = B * n_mb;
   if (chains >= kSegChains || T < 2 * kMinSegSteps) return;
+  if (direction == 1 && gw && io == SPARC_BF16 && bwd_grouped(chains)) return;  // a wave for almost every SIMD as it is
   int64_t n = T / kMinSegSteps;
   for (int64_t rounds = io == SPARC_F32 ? 2 : 4; rounds >= 1; rounds /= 2) {
     const int64_t k = rounds * kSimds / chains;
@@ -2733,7 +2758,11 @@ int split_waves(int64_t B, int64_t T, int64_t M) {
 //     279 or less (the host's time), 128 421 -> 278, 384 1100 -> 556, 2048
 //     (T=1024) 4200 -> 1460; 16 chains, T=4096 185 -> 298
 // As in the forward, with few chains only short sequences are split, and with
-// many nothing below kSplitMinSteps is.
+// many nothing below kSplitMinSteps is.  P1 scan:
+//   bf16 at one wave per SIMD (bwd_grouped) keeps the one-wave kernel, without
+//     resets: 1024 chains, T=1024 330 against 374, T=2048 633 against 600-700
+//     (T=4096, M=16384 through the C entry point 1.26-1.34 ms against
+//     1.36-1.45); with resets T=1024 486 against 332
 struct SplitBwd {
   int waves = 0, V = 1;
 };
@@ -2742,7 +2771,10 @@ struct SplitBwd {
 // sparc_mixer_backward_form has always reported for such shapes.
 constexpr int64_t kCoopKeepSteps = 1024;
 constexpr int kReluBwdWaves = 8;  // 8 steps each: a round is a saved-state chunk
-SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int cm, bool controls = false) {
+// mode: the chain mode, with kReset where there are reset steps.
+SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int mode, bool controls = false) {
+  const int cm = mode & 3;
+  const bool reset = (mode & kReset) != 0;
   const int64_t n = B * ((M + 127) / 128);
   const bool bf = io == SPARC_BF16, few = T >= 16 && T <= kSplitFewSteps;
   SplitBwd r;
@@ -2760,7 +2792,7 @@ SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int cm, bool con
     if (n > (bf ? 768 : 511) || (controls && n >= 512 && T <= kCoopKeepSteps)) return r;
     if (bf && n > 256 && (n - 1) % 256 < 128) r.V = 1;
     r.waves = !bf || n <= 256 ? 8 : 4;
-  } else if (bf || n < 1024) {
+  } else if (bf ? reset || !bwd_grouped(n) : n < 1024) {
     r.waves = n >= 1024 ? 4 : 8;
   }
   return r;
@@ -2784,7 +2816,7 @@ Layout layout(int64_t B, int64_t T, int64_t M, int direction, int32_t io, bool g
   if (l.split) l.V = split_v;
   l.n_mb = static_cast<int>((M + 64 * l.V - 1) / (64 * l.V));
   if (l.split) l.t_seg = static_cast<int>(T);
-  else choose_segments(B, T, l.n_mb, io, l.n_seg, l.t_seg);
+  else choose_segments(B, T, l.n_mb, direction, io, gw, l.n_seg, l.t_seg);
   l.R = B * T;
   // the controls backward in row blocks of 128 where that leaves two
   // workgroups per CU (fewer partial rows to sum: B=1, T=65536, width 2048
@@ -2899,6 +2931,12 @@ void launch_bwd(const Args& a, int n_segs, hipStream_t st) {
   if constexpr ((MODE & 3) != kModule) {
     if (a.n_seg == 1) {  // no time segments; fp32 keeps 16-step blocks at one wave per SIMD (8 would spill)
       constexpr int S = sizeof(IO) == 2 ? SPARC_MIXER_BWD_P1_S : 16;
+      if constexpr (!SUMMARY) {
+        if (bwd_grouped(waves, sizeof(IO) == 2 && (MODE & kReset) == 0)) {
+          hipLaunchKernelGGL((mixer_bwd_kernel<IO, V, S, SUMMARY, MODE, 4>), dim3((waves + 3) / 4), dim3(256), 0, st, a);
+          return;
+        }
+      }
       hipLaunchKernelGGL((mixer_bwd_kernel<IO, V, S, SUMMARY, MODE>), g, dim3(64), 0, st, a);
       return;
     }
@@ -2961,13 +2999,14 @@ Layout forward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_d
   const int nw = split_waves(batch, length, modes);
   return nw ? layout(batch, length, modes, 0, io_dtype, gw, false, nw) : l;
 }
-// The backward's, for chain mode cm (kRelu: split, or not there at all);
+// The backward's, for a chain mode (kRelu: split, or not there at all; with
+// kReset where there are reset steps);
 // controls: the whole module backward (its time pieces, split_bwd).
-Layout backward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, int cm,
+Layout backward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, int mode,
                        bool controls = false) {
-  const SplitBwd sp = split_bwd(batch, length, modes, io_dtype, cm, controls);
-  if (!sp.waves) return layout(batch, length, modes, 1, io_dtype, cm != kModule, controls);
-  return layout(batch, length, modes, 1, io_dtype, cm != kModule, false, sp.waves, sp.V);
+  const SplitBwd sp = split_bwd(batch, length, modes, io_dtype, mode, controls);
+  if (!sp.waves) return layout(batch, length, modes, 1, io_dtype, mode != kModule, controls);
+  return layout(batch, length, modes, 1, io_dtype, mode != kModule, false, sp.waves, sp.V);
 }
 
 // the split forward: l.split waves per chain
@@ -3171,9 +3210,12 @@ bool p1_fused_relu_backward(const sparc_scan_desc* d) {
 
 size_t p1_fused_workspace_bytes(const sparc_scan_desc* d, int direction) {
   if (!p1_fused_shape(d)) return 0;
-  if (direction == 0) return forward_layout(d->batch, d->length, d->modes, d->io_dtype, true).total;
+  // enough for a call with reset steps and for one without
+  if (direction == 0)
+    return forward_layout(d->batch, d->length, d->modes, d->io_dtype, true).total;
+  size_t n = std::max(backward_layout(d->batch, d->length, d->modes, d->io_dtype, kPlanes).total,
+                      backward_layout(d->batch, d->length, d->modes, d->io_dtype, kPlanes | kReset).total);
   // the relu output's backward is the general kernels' where it is not split
-  size_t n = backward_layout(d->batch, d->length, d->modes, d->io_dtype, kPlanes).total;
   if (p1_fused_relu_backward(d))
     n = std::max(n, backward_layout(d->batch, d->length, d->modes, d->io_dtype, kRelu).total);
   return n;
@@ -3262,7 +3304,8 @@ sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const
   const bool relu = d && (d->flags & SPARC_FLAG_RELU_OUTPUT) != 0;
   if (!p1_fused_shape(d) || d->length <= 0 || (relu && !p1_fused_relu_backward(d)))
     return fail(SPARC_EINVAL, "p1 fused backward: shape");
-  const Layout l = backward_layout(d->batch, d->length, d->modes, d->io_dtype, relu ? kRelu : kPlanes);
+  const bool reset = segment_pos != nullptr || (d->flags & SPARC_FLAG_RESET_FIRST) != 0;
+  const Layout l = backward_layout(d->batch, d->length, d->modes, d->io_dtype, (relu ? kRelu : kPlanes) | (reset ? kReset : 0));
   if (workspace_bytes < l.total) return fail(SPARC_EWORKSPACE, "workspace too small: %zu < %zu", workspace_bytes, l.total);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
@@ -3293,7 +3336,6 @@ sparc_status p1_fused_backward(const sparc_scan_desc* d, const float* eta, const
   a.segpos = segment_pos;
   a.reset_first = (d->flags & SPARC_FLAG_RESET_FIRST) != 0;
   const bool bf = d->io_dtype == SPARC_BF16;
-  const bool reset = segment_pos || a.reset_first;
   if (relu && reset) run_bwd_split<kRelu | kReset>(a, l, bf, st);
   else if (relu) run_bwd_split<kRelu>(a, l, bf, st);
   else if (l.split && reset) run_bwd_split<kPlanes | kReset>(a, l, bf, st);
@@ -3506,13 +3548,13 @@ std::atomic<int> g_bwd_plan{0};
 // Steps per block of the one-launch form: 4 (with 8 the ring and the
 // reduction's registers spill under the two-waves-per-SIMD bound).
 constexpr int kCoopS = 4;
-template <typename IO, int kS>
+template <typename IO, int kS, int NG>
 const void* coop_kernel() {
-  return reinterpret_cast<const void*>(&mixer_bwd_kernel<IO, 1, kS, false, kModule | kCoop>);
+  return reinterpret_cast<const void*>(&mixer_bwd_kernel<IO, 1, kS, false, kModule | kCoop, NG>);
 }
-// Workgroups of the kernel that the current device holds at once (0 on any
+// Chains, NG per workgroup, that the current device holds at once (0 on any
 // failure), cached per device.
-template <typename IO, int kS>
+template <typename IO, int kS, int NG>
 int64_t coop_capacity() {
   static std::atomic<int64_t> cache[64];
   int dev = 0;
@@ -3523,12 +3565,12 @@ int64_t coop_capacity() {
   int64_t c = cache[dev].load(std::memory_order_relaxed);
   if (c > 0) return c;
   int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, coop_kernel<IO, kS>(), 64, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, coop_kernel<IO, kS, NG>(), 64 * NG, 0) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
-  c = static_cast<int64_t>(per_cu) * cus;
+  c = static_cast<int64_t>(per_cu) * NG * cus;
   cache[dev].store(c, std::memory_order_relaxed);
   return c;
 }
@@ -3570,8 +3612,21 @@ int coop_steps(int64_t B, int64_t T, int64_t M, int32_t io) {
   const Layout l = layout(B, T, M, 1, io);
   if (l.V != 1 || l.n_seg != 1) return 0;
   const int64_t grid = B * l.n_mb;
-  const int64_t cap = io == SPARC_BF16 ? coop_capacity<sparc::bf16, kCoopS>() : coop_capacity<float, kCoopS>();
+  const int64_t cap = io == SPARC_BF16 ? coop_capacity<sparc::bf16, kCoopS, 1>() : coop_capacity<float, kCoopS, 1>();
   return grid <= cap ? kCoopS : 0;
+}
+
+// one wave per chain, four per workgroup where bwd_grouped (all of them
+// resident either way: each chain takes the LDS of one ring)
+template <typename IO>
+void launch_coop(const Args& a, int64_t waves, hipStream_t st) {
+  constexpr int kC = kModule | kCoop;
+  static_assert(kCoopS == 4, "one instantiation per I/O type");
+  if (bwd_grouped(waves) && waves <= coop_capacity<IO, kCoopS, 4>())
+    hipLaunchKernelGGL((mixer_bwd_kernel<IO, 1, kCoopS, false, kC, 4>), dim3(static_cast<unsigned>((waves + 3) / 4)),
+                       dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((mixer_bwd_kernel<IO, 1, kCoopS, false, kC>), dim3(static_cast<unsigned>(waves)), dim3(64), 0, st, a);
 }
 
 sparc_status coop_backward(int kS, int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, const void* x,
@@ -3614,14 +3669,10 @@ sparc_status coop_backward(int kS, int64_t batch, int64_t length, int64_t modes,
   a.coop_nblk = c.nblk;
   a.coop_error = reinterpret_cast<uint32_t*>(ws) + 1;
   a.coop_spin = sparc::wait_limit();
-  const dim3 g(static_cast<unsigned>(batch * c.n_mb));
-  constexpr int kC = kModule | kCoop;
-  static_assert(kCoopS == 4, "one instantiation per I/O type");
+  const int64_t waves = batch * c.n_mb;
   if (kS != kCoopS) return fail(SPARC_EINVAL, "mixer backward: steps per block");
-  if (io_dtype == SPARC_BF16)
-    hipLaunchKernelGGL((mixer_bwd_kernel<sparc::bf16, 1, kCoopS, false, kC>), g, dim3(64), 0, st, a);
-  else
-    hipLaunchKernelGGL((mixer_bwd_kernel<float, 1, kCoopS, false, kC>), g, dim3(64), 0, st, a);
+  if (io_dtype == SPARC_BF16) launch_coop<sparc::bf16>(a, waves, st);
+  else launch_coop<float>(a, waves, st);
   if (hipError_t le = hipGetLastError()) return fail(SPARC_EHIP, "mixer backward: %s", hipGetErrorString(le));
   float* outs[5] = {dnu_log, dtheta_log, dwrite_log_gain, dwrite_phase_response, dwrite_radial_response};
   {
