@@ -332,16 +332,21 @@ void launch_ctrl_fwd_rows(hipStream_t st, int64_t R, int W, const void* x, const
     hipLaunchKernelGGL((ctrl_fwd_kernel<IO, 4, ROWS>), g, dim3(256), 0, st, R, W, x, pdir, rdir, eta, delta);
 }
 // 16 rows per workgroup where that leaves at least kCtrlFwdGroups workgroups
-// (four per CU, one wave per SIMD and workgroup), else 8 or 4: with few rows
+// (four per CU, one wave per SIMD and workgroup), else fewer: with few rows
 // 16 each left most CUs without work (232 workgroups at 3711 rows of 24576
 // bf16: 98 us, 1.9 TB/s; the no-gradient module forward there 372 -> 310 us
-// with 4 rows each).
+// with 4 rows each).  Between 8 and 16 thousand rows, us with 4, 8 and 16 rows
+// each: bf16 8192 rows of 32768 100, 96, 151, 12000 of 24576 106, 97, 128,
+// 8192 of 512 8, 9, 13; fp32, where 8 rows are the slowest everywhere, 8192
+// rows of 32768 252, 318, 185, 12000 of 8192 91, 115, 75, but 8192 of 1024 12,
+// 13, 22.
 constexpr int64_t kCtrlFwdGroups = 1024;
 template <typename IO>
 void launch_ctrl_fwd(hipStream_t st, int64_t R, int W, const void* x, const float* pdir, const float* rdir,
                      float* eta, float* delta) {
   if (R >= 16 * kCtrlFwdGroups) launch_ctrl_fwd_rows<IO, 16>(st, R, W, x, pdir, rdir, eta, delta);
-  else if (R >= 8 * kCtrlFwdGroups) launch_ctrl_fwd_rows<IO, 8>(st, R, W, x, pdir, rdir, eta, delta);
+  else if (R >= 8 * kCtrlFwdGroups && W >= 2048)
+    launch_ctrl_fwd_rows<IO, sizeof(IO) == 2 ? 8 : 16>(st, R, W, x, pdir, rdir, eta, delta);
   else launch_ctrl_fwd_rows<IO, 4>(st, R, W, x, pdir, rdir, eta, delta);
 }
 
