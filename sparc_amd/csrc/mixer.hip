@@ -2618,14 +2618,16 @@ int mixer_v(int64_t B, int64_t T, int64_t M, int direction, bool gw);
 // composes them into the state entering every segment, and the full pass
 // replays each segment from its entering state.  This costs a second pass
 // over the transitions (and, forward, the writes), paid for by the occupancy.
-// The waves fill whole rounds of the 1024 SIMDs, 4 of them (bf16) or 2
-// (fp32, whose kernels hold 2 to 3 waves per SIMD), or as many fewer (2, 1)
+// The waves fill whole rounds of the 1024 SIMDs, 4 of them (bf16, and the fp32
+// module forward) or 2 (fp32 else), or as many fewer (2, 1)
 // as leave segments of kAlignedSegSteps: a few waves past a round keep their
 // SIMDs busy for one more while the others idle.  Measured (training step,
 // us; segments of at least 128 steps before): P1 with resets, 72 chains,
 // T=4001, fp32 555 (2232 waves) -> 466 (2016; 4032 497), bf16 375 -> 319
 // (4032; 2016 347); module bf16, 72 chains, T=6000 829 (3312) -> 766, 64
-// chains, T=4096 510 (2048) -> 487 (4096), 16 chains, T=16384 467 -> 481.
+// chains, T=4096 510 (2048) -> 487 (4096), 16 chains, T=16384 467 -> 481.  The
+// fp32 module forward, 16 chains, T=65536, 2048 waves 1266 and 4096 waves
+// 1106, 96 chains, T=8192 0.88 of the time with 4032 against 2016.
 #ifndef SPARC_MIXER_SEG_CHAINS
 #define SPARC_MIXER_SEG_CHAINS 1024
 #endif
@@ -2661,7 +2663,7 @@ void choose_segments(int64_t B, int64_t T, int n_mb, int direction, int32_t io, 
   if (chains >= kSegChains || T < 2 * kMinSegSteps) return;
   if (direction == 1 && gw && io == SPARC_BF16 && bwd_grouped(chains)) return;  // a wave for almost every SIMD as it is
   int64_t n = T / kMinSegSteps;
-  for (int64_t rounds = io == SPARC_F32 ? 2 : 4; rounds >= 1; rounds /= 2) {
+  for (int64_t rounds = io == SPARC_F32 && (gw || direction == 1) ? 2 : 4; rounds >= 1; rounds /= 2) {
     const int64_t k = rounds * kSimds / chains;
     if (k >= 2 && T / k >= kAlignedSegSteps) {
       n = k;
