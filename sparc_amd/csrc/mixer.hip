@@ -2734,17 +2734,29 @@ constexpr int kPieces = SPARC_MIXER_BWD_PIECES;
 // The wide kernel stays ahead with many chains for the P1 scan (754 against
 // 822-918 at 1024 chains, T=4096) and the fp32 module (1475 against 1724,
 // T=2048), and below kSplitMinSteps with many chains nothing is split.
+// Two edges where segments or one wave per chain are the faster form:
+//   bf16, half the CUs or little more (kSplitHalfChains) and long sequences:
+//     128 chains, P1 with resets T=2048 split 0.80 of the time in segments,
+//     T=4096 1.08-1.11, T=8192 1.12-1.17 (324 and 381); module T=4096 1.05,
+//     T=8192 683 and 742; without resets T=4096 0.98; 136 chains 0.82-0.95
+//   fp32 P1 from 640 chains on: with resets 768 chains 1.05-1.09, 832 chains
+//     1.15-1.28, 896 chains 1.10-1.15; without 640 chains 1.05-1.16, 832
+//     chains 1.00-1.13, 704 and 768 chains 0.88-1.05
 constexpr int kSplitV = 2;
 template <typename IO> constexpr int kSplitFwdS = sizeof(IO) == 2 ? 8 : 4;
 constexpr int64_t kSplitChains = 128, kSplitMinSteps = 2 * kMinSegSteps, kSplitFewSteps = 768;
-// waves per chain of the split forward, 0: not split
-int split_waves(int64_t B, int64_t T, int64_t M) {
+constexpr int64_t kSplitHalfChains = 136, kSplitLongSteps = 3072, kSplitP1F32Chains = 640;
+// waves per chain of the split forward, 0: not split (gw: the P1 scan; reset:
+// with reset steps)
+int split_waves(int64_t B, int64_t T, int64_t M, int32_t io, bool gw, bool reset) {
   const int64_t chains = B * ((M + 64 * kSplitV - 1) / (64 * kSplitV));
   if (chains < kSplitChains) {
     if (T < 16 || T > kSplitFewSteps) return 0;
     return static_cast<int>(std::min<int64_t>(kSplitWaves, (T + 3) / 4));
   }
   if (T < kSplitMinSteps) return 0;
+  if (io == SPARC_F32 && gw && chains >= kSplitP1F32Chains) return 0;
+  if (io == SPARC_BF16 && (!gw || reset) && chains < kSplitHalfChains && T > kSplitLongSteps) return 0;
   return chains >= 512 ? 4 : chains >= 192 ? 8 : kSplitWaves;
 }
 // The split backward: waves per chain and modes per lane, or waves 0 (the
@@ -3000,10 +3012,10 @@ bool fwd_wide(const Layout& l, int64_t batch, int64_t modes, bool module = false
 }
 // The forward's layout: split chains unless the wide kernel is the faster one
 // there (the P1 scan and the fp32 module with many chains, see split_waves).
-Layout forward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, bool gw) {
+Layout forward_layout(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype, bool gw, bool reset = false) {
   const Layout l = layout(batch, length, modes, 0, io_dtype, gw);
   if ((gw || io_dtype == SPARC_F32) && fwd_wide(l, batch, modes, !gw)) return l;
-  const int nw = split_waves(batch, length, modes);
+  const int nw = split_waves(batch, length, modes, io_dtype, gw, reset);
   return nw ? layout(batch, length, modes, 0, io_dtype, gw, false, nw) : l;
 }
 // The backward's, for a chain mode (kRelu: split, or not there at all; with
@@ -3219,7 +3231,8 @@ size_t p1_fused_workspace_bytes(const sparc_scan_desc* d, int direction) {
   if (!p1_fused_shape(d)) return 0;
   // enough for a call with reset steps and for one without
   if (direction == 0)
-    return forward_layout(d->batch, d->length, d->modes, d->io_dtype, true).total;
+    return std::max(forward_layout(d->batch, d->length, d->modes, d->io_dtype, true, false).total,
+                    forward_layout(d->batch, d->length, d->modes, d->io_dtype, true, true).total);
   size_t n = std::max(backward_layout(d->batch, d->length, d->modes, d->io_dtype, kPlanes).total,
                       backward_layout(d->batch, d->length, d->modes, d->io_dtype, kPlanes | kReset).total);
   // the relu output's backward is the general kernels' where it is not split
@@ -3252,7 +3265,8 @@ sparc_status p1_fused_forward(const sparc_scan_desc* d, const float* eta, const 
                               void* y_im, float* chunk_state, void* workspace, size_t workspace_bytes,
                               sparc_stream_t stream) {
   if (!p1_fused_shape(d) || d->length <= 0) return fail(SPARC_EINVAL, "p1 fused forward: shape");
-  const Layout l = forward_layout(d->batch, d->length, d->modes, d->io_dtype, true);
+  const bool reset = segment_pos != nullptr || (d->flags & SPARC_FLAG_RESET_FIRST) != 0;
+  const Layout l = forward_layout(d->batch, d->length, d->modes, d->io_dtype, true, reset);
   if (workspace_bytes < l.total) return fail(SPARC_EWORKSPACE, "workspace too small: %zu < %zu", workspace_bytes, l.total);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
@@ -3270,7 +3284,6 @@ sparc_status p1_fused_forward(const sparc_scan_desc* d, const float* eta, const 
   a.w_re = w_re; a.w_im = w_im; a.h0_re = h0_re; a.h0_im = h0_im; a.chunk_state = chunk_state;
   a.segpos = segment_pos;
   a.reset_first = (d->flags & SPARC_FLAG_RESET_FIRST) != 0;
-  const bool reset = segment_pos != nullptr || a.reset_first;
   if (relu) {
     a.y = y_re;
   } else {
