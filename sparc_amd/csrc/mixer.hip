@@ -2778,10 +2778,20 @@ int split_waves(int64_t B, int64_t T, int64_t M, int32_t io, bool gw, bool reset
 //     (T=1024) 4200 -> 1460; 16 chains, T=4096 185 -> 298
 // As in the forward, with few chains only short sequences are split, and with
 // many nothing below kSplitMinSteps is.  P1 scan:
+//   where the second round has workgroups for few of the 256 CUs
+//     (kSplitSecondRound, with resets twice that) long sequences are not split
+//     (time against segments): bf16 272 chains, T=1024 0.89, T=2048 1.15, with
+//     resets 0.96 and 1.23, 320 chains, T=2048 1.01 and with resets 1.08, 352
+//     chains 0.91-0.98; fp32, two workgroups per 128 modes, 144 chains, T=2048
+//     0.94, T=4096 1.07, with resets 1.00 and 1.20, 176 chains, T=4096 0.93 and
+//     with resets 1.08
 //   bf16 at one wave per SIMD (bwd_grouped) keeps the one-wave kernel, without
 //     resets: 1024 chains, T=1024 330 against 374, T=2048 633 against 600-700
 //     (T=4096, M=16384 through the C entry point 1.26-1.34 ms against
 //     1.36-1.45); with resets T=1024 486 against 332
+//   bf16 with resets, more than 1536 chains, below kSplitManySteps as well:
+//     4096 chains, T=256 341 against 396, T=512 630 against 694, T=768 969
+//     against 925
 struct SplitBwd {
   int waves = 0, V = 1;
 };
@@ -2789,6 +2799,7 @@ struct SplitBwd {
 // one-launch form; up to this many steps it keeps that form there, as
 // sparc_mixer_backward_form has always reported for such shapes.
 constexpr int64_t kCoopKeepSteps = 1024;
+constexpr int64_t kSplitSecondRound = 48, kSplitManySteps = 768;
 constexpr int kReluBwdWaves = 8;  // 8 steps each: a round is a saved-state chunk
 // mode: the chain mode, with kReset where there are reset steps.
 SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int mode, bool controls = false) {
@@ -2811,7 +2822,11 @@ SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int mode, bool c
     if (n > (bf ? 768 : 511) || (controls && n >= 512 && T <= kCoopKeepSteps)) return r;
     if (bf && n > 256 && (n - 1) % 256 < 128) r.V = 1;
     r.waves = !bf || n <= 256 ? 8 : 4;
-  } else if (bf ? reset || !bwd_grouped(n) : n < 1024) {
+  } else if (bf ? (reset ? n <= 1536 || T >= kSplitManySteps : !bwd_grouped(n)) : n < 1024) {
+    const int64_t groups = B * ((M + 64 * r.V - 1) / (64 * r.V));
+    if (groups > 256 && groups < 256 + (reset ? 2 : 1) * kSplitSecondRound &&
+        T > (bf ? kSplitLongSteps / 2 : kSplitLongSteps))
+      return r;
     r.waves = n >= 1024 ? 4 : 8;
   }
   return r;

@@ -28,6 +28,10 @@ def _case(B, T, M, dtype, seg):
     (5, 256, 16384, F32, False),   # 640 chains: the forward not split
     (5, 256, 16260, F32, True),    # lanes past M
     (2, 3073, 8192, BF16, True),   # 128 chains: the forward in segments
+    (2, 1537, 17280, BF16, False),  # 270 chains: the backward in segments
+    (2, 1537, 21500, BF16, True),  # 336 chains, with resets only
+    (2, 3073, 8640, F32, False),   # 136 chains, fp32
+    (4, 257, 50000, BF16, True),   # 1564 chains with resets: one wave per chain
 ])
 def test_p1_split_edges(B, T, M, dtype, seg):
     print(f"[case] split edges B={B} T={T} M={M} {dtype} resets={seg}", flush=True)
