@@ -15,6 +15,7 @@ import torch
 
 import sparc_amd
 from sparc_amd import ops
+from test_gpu_module import _masked_dy, oracle_params
 from test_gpu_scan import BF16, F32, check_case, make_case, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -147,8 +148,10 @@ def test_forward_without_gradients_matches(B, L, width, dtype):
 ])
 def test_split_module_backward(B, L, width, dtype):
     """Every gradient of the module's split backward against the composed path
-    (separate operators on the general kernels), the incoming gradient masked
-    where the state is near the relu's edge."""
+    (separate operators on the general kernels).  The incoming gradient is
+    masked where the state before the relu is near its edge and nowhere else:
+    it reaches the kernel at clearly negative states, whose relu has to stop
+    it."""
     print(f"[case] split module backward B={B} L={L} width={width} {dtype}", flush=True)
     torch.manual_seed(L + B)
     m = sparc_amd.SPARCMixer(width).cuda()
@@ -162,18 +165,58 @@ def test_split_module_backward(B, L, width, dtype):
     dl = torch.randn(B, width // 2, device="cuda")
     params = [m.phase_direction, m.radial_direction, m.nu_log, m.theta_log, m.write_log_gain,
               m.write_phase_response, m.write_radial_response]
-    got, band = {}, None
+    p = oracle_params(m, requires_grad=False)
+    masked = _masked_dy(p, x.double().cpu(), dy.double().cpu(), band=1e-3 if dtype == torch.float32 else 2e-2)
+    dy = masked.to(dtype).cuda()
+    got = {}
     for path in ("composed", "fused"):
         sparc_amd.set_mixer_path(path)
         try:
             xx = x.clone().requires_grad_()
             y, last = m(xx, return_cache=True)
-            if band is None:  # positive outputs within the band and every zero next to one
-                edge = y.detach().float() < (1e-3 if dtype == torch.float32 else 5e-2)
-                band = (edge & (y.detach() > 0)) | (y.detach() == 0)
-            got[path] = torch.autograd.grad([y, last[0]], [xx, *params], [dy.masked_fill(band, 0.0), dl])
+            got[path] = torch.autograd.grad([y, last[0]], [xx, *params], [dy, dl])
+            assert (dy[y == 0] != 0).float().mean().item() > 0.5  # stopped states with a gradient coming in
         finally:
             sparc_amd.set_mixer_path("auto")
     tol = 1e-4 if dtype == torch.float32 else 2e-2
     for k, (a, b) in enumerate(zip(got["fused"], got["composed"])):
         assert rel_err(a, b) <= tol, f"gradient {k}: {rel_err(a, b):.3g}"
+
+
+@pytest.mark.parametrize("B,L,M,dtype", [(2, 100, 260, torch.bfloat16), (3, 77, 132, torch.float32)])
+def test_split_module_states_aligned_for_one_mode(B, L, M, dtype):
+    """Through the C entry points with h_re, h_im on odd elements: where the
+    split kernels hold two modes per lane the calls take the forms of one
+    mode, and give the results of aligned states up to the order of the sums."""
+    from sparc_amd import _lib
+    print(f"[case] states off alignment B={B} L={L} M={M} {dtype}", flush=True)
+    lib, P = _lib.load(), _lib.ptr
+    g = torch.Generator(device="cuda").manual_seed(L)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    x, dy = rn(B, L, 2 * M).to(dtype), rn(B, L, 2 * M).to(dtype)
+    dirs = [rn(2 * M + 1) * 0.5 / (2 * M) ** 0.5 for _ in range(2)]
+    modes = [torch.log(torch.rand(M, device="cuda", generator=g) + 0.01), rn(M), *(0.3 * rn(M) for _ in range(3))]
+    st, io = _lib.stream_of(x.device), _lib.io_code(dtype)
+    got = {}
+    for off in (0, 1):
+        controls = torch.empty(2, B * L, device="cuda")
+        y = torch.empty_like(x)
+        h = [torch.empty(B * L * M + 8, dtype=dtype, device="cuda")[off:off + B * L * M] for _ in range(2)]
+        last = [torch.empty(B, M, device="cuda") for _ in range(2)]
+        ws = torch.empty(lib.sparc_mixer_workspace_bytes(B, L, M, 0), dtype=torch.uint8, device="cuda")
+        _lib.check(lib.sparc_mixer_forward(B, L, M, io, P(x), *map(P, dirs), *map(P, modes), P(controls[0]), P(controls[1]),
+                                           P(y), *map(P, h), *map(P, last), P(ws), ws.numel(), st), "forward")
+        dx = torch.empty_like(x)
+        grads = [torch.empty(n, device="cuda") for n in (2 * M + 1, 2 * M + 1, M, M, M, M, M)]
+        ws = torch.empty(lib.sparc_mixer_workspace_bytes(B, L, M, 1), dtype=torch.uint8, device="cuda")
+        hs = h
+        if off:  # the backward from the same states, moved
+            hs = [torch.cat((t[:1], t))[1:] for t in got[0][1:3]]
+            assert all(t.data_ptr() % (2 * t.element_size()) for t in (*h, *hs))
+        _lib.check(lib.sparc_mixer_backward(B, L, M, io, P(x), *map(P, dirs), *map(P, modes), P(controls[0]), P(controls[1]),
+                                            *map(P, hs), P(dy), None, None, P(dx), *map(P, grads), P(ws), ws.numel(), st),
+                   "backward")
+        got[off] = [y, *h, *last, dx, *grads]
+    tol = 1e-5 if dtype == torch.float32 else 2.0 ** -7  # fp32 sums in another order, then one rounding
+    for k, (a, b) in enumerate(zip(got[1], got[0])):
+        assert rel_err(a, b) <= (tol if k < 6 else 5 * tol), f"tensor {k}: {rel_err(a, b):.3g}"
