@@ -432,22 +432,29 @@ sparc_status sparc_mixer_scan_backward(int64_t batch, int64_t length, int64_t mo
  * direction gradients [2M+1] and the parameter gradients [M] (fp32).
  * Deterministic (fixed-order reductions).
  *
- * Forms (sparc_mixer_backward_form): where no time segments are needed (at
- * least 1024 chains of 64 modes), T > 0 and every chain fits on the GPU at
- * once at the kernel's occupancy, the call runs in ONE launch that also
- * completes dx and the direction gradients: the chains of a batch row
+ * Forms (sparc_mixer_backward_form).  Split chains, one scan launch in which
+ * the waves of a workgroup share a chain's time and then the controls'
+ * backward: in bf16 from 192 to 511 chains of 128 modes with T >= 256, from
+ * 512 to 768 chains with T > 1024; in fp32 from 128 to 511 chains with T >=
+ * 256; in both below 128 chains with 16 <= T <= 768; the states h_re, h_im on
+ * addresses that hold as many modes per lane as the kernel takes (two in
+ * bf16).  Else, where no time segments are needed (at least 1024 chains of 64
+ * modes, or T < 256), T > 0 and every chain fits on the GPU at once at the
+ * kernel's occupancy, the call runs in ONE launch that also completes dx and
+ * the direction gradients: the chains of a batch row
  * exchange per-block sums through the workspace (no atomics: each block has
  * one owner chain, which sums the row's records in a fixed order once all
  * are stored) and each chain completes a block eight blocks (fp32: four)
  * after computing it.  Its waits are bounded (sparc_set_wait_limit): a wait
  * that reaches the bound sets the workspace error word
  * (sparc_scan_workspace_error) and leaves NaN gradients for that block, and
- * every workgroup still finishes.  Otherwise the time pieces below, else one
- * scan launch followed by the controls' backward.
+ * every workgroup still finishes.  Otherwise the time pieces below, else the
+ * scan (with few chains in time segments: a summary, a carry and a replay
+ * launch) followed by the controls' backward.
  *
- * Streams: when T splits into time pieces (T a multiple of 256, and at least
- * 1024 chains of 64 modes, so that no time segments are needed; the
- * workspace query covers both layouts), the call runs the
+ * Streams: when T splits into time pieces (T a multiple of 256, at least
+ * 1024 chains of 64 modes, so that no time segments are needed, and the chains
+ * not split; the workspace query covers every layout), the call runs the
  * pieces last first and launches each piece's controls backward on a second
  * stream, so that it overlaps the next piece's scan.  That stream is owned by
  * the library: one per device, non-blocking, default priority, created with
@@ -479,8 +486,9 @@ sparc_status sparc_mixer_backward(int64_t batch, int64_t length, int64_t modes, 
                                   sparc_stream_t stream);
 
 /* The form sparc_mixer_backward takes for this shape on the current device:
- * 2 (one launch), 1 (time pieces), 0 (one scan launch, then the controls'
- * backward), -1 (invalid shape).  No counterpart in the reference (one Triton
+ * 2 (one launch), 1 (time pieces), 0 (the scan, its chains split or in time
+ * segments or neither, then the controls' backward), -1 (invalid shape).  For
+ * h_re, h_im aligned for two values; see Forms above for others.  No counterpart in the reference (one Triton
  * launch sequence). */
 int sparc_mixer_backward_form(int64_t batch, int64_t length, int64_t modes, int32_t io_dtype);
 

@@ -377,8 +377,9 @@ struct ModeConsts {
 };
 
 // How the kernels of one I/O type and chain mode evaluate the P1 transition
-// (every kernel of the pair the same way, so that forward, backward and the
-// summary passes of time segments see the same a):
+// (the forward, the backward that reads its states and the summary passes of
+// time segments the same way, so that they see the same a; not the relu
+// output's backward in bf16, see below):
 //   HW   (bf16 I/O): the sine and cosine of the phase step from the hardware
 //        (sincos_rev_hw) instead of the degree-9/10 polynomials;
 //   FAST (bf16 I/O, writes given): rho = 2^{-nu log2(e) E} and em = rho - 1
@@ -390,7 +391,10 @@ struct ModeConsts {
 //        rounding of rho.  The module keeps the series: its write gain goes
 //        as sqrt(em) for slow modes.
 // fp32 I/O keeps the polynomials and the series, and so does the relu output's
-// split backward, which recomputes the states.
+// split backward, which recomputes the states: beside a bf16 forward its states
+// differ from that forward's in their last bits, and a state within them of
+// zero may be stopped by the relu in one and not in the other (as with the
+// general kernels' backward, which forms a the same way).
 template <typename IO, int MODE>
 struct P1Math {
   static constexpr bool HW = sizeof(IO) == 2;
@@ -2795,9 +2799,14 @@ int split_waves(int64_t B, int64_t T, int64_t M, int32_t io, bool gw, bool reset
 struct SplitBwd {
   int waves = 0, V = 1;
 };
-// controls: the whole module backward, which from 512 chains on has the
-// one-launch form; up to this many steps it keeps that form there, as
-// sparc_mixer_backward_form has always reported for such shapes.
+// controls: the whole module backward.  From 512 chains on it runs in one
+// launch, and up to kCoopKeepSteps it stays there: that form, and time pieces
+// for a caller that sets the one-launch form aside, is what the header has
+// promised for these shapes.  It costs time in bf16 (us, one launch against
+// split: 512 chains, T=512 276 and 242, T=1024 about 530 and 425; 640 chains
+// 370 and 301, 705 and 553; 768 chains 378 and 341, 717 and 624); fp32 is
+// faster in one launch (512 chains, T=1024 657 and 804, 768 chains 723 and
+// 1131).
 constexpr int64_t kCoopKeepSteps = 1024;
 constexpr int64_t kSplitSecondRound = 48, kSplitManySteps = 768;
 constexpr int kReluBwdWaves = 8;  // 8 steps each: a round is a saved-state chunk

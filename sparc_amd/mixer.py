@@ -39,8 +39,9 @@ _BWD_PLANS = ("auto", "pieces")
 def set_backward_plan(name: str) -> str:
     """Form of the fused module backward (sparc_mixer_backward_plan):
     "auto" runs it in one launch wherever every chain fits on the GPU at once
-    (the controls' backward inside), else in time pieces or as a scan launch
-    followed by the controls' backward; "pieces" never takes the one-launch
+    (the controls' backward inside) unless its chains are split over the waves
+    of a workgroup, else in time pieces or as a scan followed by the controls'
+    backward; "pieces" never takes the one-launch
     form.  Process-wide; returns the previous setting."""
     if name not in _BWD_PLANS:
         raise ValueError(f"unknown backward plan {name!r}")
