@@ -318,8 +318,9 @@ def bench_p1(args, dev):
     bf16 writes, fp32 eta/delta, fp32 state.  Forward and backward through the
     C ABI; at G = 1 they run the fused kernels with the writes given (the
     forward on chains of 256 modes with helper waves, mixer_fwd_wide_kernel;
-    the backward one wave per chain of 64 modes, mixer_bwd_kernel), the
-    backward reading the states from the forward's output.  Beside it the few-chain
+    the backward one wave per chain of 128 modes, four chains per workgroup,
+    mixer_bwd_kernel), the backward reading the states from the forward's
+    output.  Beside it the few-chain
     form, B=1, T=65536, M=2048 (32 chains of 64 modes, split into time
     segments: a summary pass, the carry, a replay)."""
     B, T, M = 8, 4096, 16384
@@ -415,7 +416,8 @@ def bench_module(args, dev):
     values so that every term is active).  On this shape the module runs the
     fused sequence path (controls, write, P1 scan, relu(cat) epilogue and their
     backward; the backward in one launch with the controls' backward inside,
-    `backward_form`).  Its kernels are VALU-bound (the counter summary's VALU
+    `backward_form`; the forward with its chains split over the waves of a
+    workgroup, mixer_fwd_split_kernel).  Its kernels are VALU-bound (the counter summary's VALU
     busy), so its roofline object reports the HBM rate of its algorithmic
     bytes beside the measured traffic and VALU-busy figures."""
     import sparc_amd
@@ -457,7 +459,7 @@ def bench_module(args, dev):
     M = W // 2
     algo_bytes = B * T * (M * 10 * 2 + 6 * 4)
     form = sparc_amd.backward_form(B, T, M, torch.bfloat16)
-    kernels = ("ctrl_fwd_kernel", "mixer_fwd_wide_kernel", "mixer_bwd_kernel")
+    kernels = ("ctrl_fwd_kernel", "mixer_fwd_split_kernel", "mixer_bwd_kernel")
     if form != "one_launch":
         kernels += ("ctrl_bwd_kernel",)
     traffic = measured_traffic(COUNTERS_FILE)
