@@ -1382,7 +1382,11 @@ struct SubChunk {
   // and every step is in range, so no load stands under a branch.  For bf16
   // only (one mode per lane, elementwise gates, M = 4001, fwd+bwd: complex
   // 1766 -> 1240 us, real 1416 -> 1069); fp32 measured the same either way
-  // and spills where it already fills the registers (P1 1840 -> 1867).
+  // and spills where it already fills the registers (P1 1840 -> 1867).  With
+  // two modes per lane it spills some registers more in bf16 as well (P1
+  // backward 177 -> 193) and is the faster one all the same (P1 backward, B=8,
+  // T=2048, M=8192, 512 gate pairs a token 2019 -> 1749; polar, B=16, T=1024,
+  // 1024 groups of 4, fwd+bwd 838 -> 662).
   static constexpr bool kFull = sizeof(IO) == 2;
   __device__ __forceinline__ void load(const ScanArgs& p, const TL& tl, int b, int t0, int m0, bool lane_ok, bool full) {
     if (kFull && full) {
@@ -2034,6 +2038,8 @@ __device__ __forceinline__ uint32_t fill_tab(const ScanArgs& p, int t0, int g_ba
   return rmask;
 }
 
+// (The bound of four waves per SIMD leaves 128 VGPRs: polar and cartesian bf16
+// at two modes per lane spill 20 of them, 60 bytes a lane.)
 template <int TR, typename IO, int V, int S, int NW, bool RELU>
 __global__ void __launch_bounds__(NW * 64, 4)
 chain_fwd_fast_kernel(ScanArgs p) {
@@ -3919,6 +3925,12 @@ const char* make_plan(const sparc_scan_desc* d, int direction, Plan* pl, bool al
   } else if (auto_plan && lane_shared) {
     plan_lane_shared(cplx_tr, bf16_io, wide, direction == 1 && !allow_seg, seg_below, serial_min, chain_min);
     if (g32 && !g32_segments(direction, !cplx_tr, pl->n_chains, d->length)) seg_below = 0;
+    // fp32 gates: the chain kernels' second round has workgroups for few of the
+    // 256 CUs, and the look-back is the faster one where T is not short (the
+    // chain kernels' time against its: polar, 256 chains, T=4096 0.75-0.93, 384
+    // chains 0.89-1.04, but 288 chains T=512 0.91, T=1024 1.02, T=4096 1.13;
+    // real, 288 chains, T=2048 1.12, 320 chains 1.08)
+    if (g32 && pl->n_chains > 256 && pl->n_chains < 352 && d->length >= 1024) chain_min = kChainMin;
   }
   pl->n_seg = 1;
   pl->t_seg = static_cast<int>(d->length);

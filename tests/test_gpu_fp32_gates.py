@@ -21,6 +21,8 @@ pytestmark = pytest.mark.gpu
     ("polar", 8, 70, 1024, 16, "serial, 4 modes per lane"),
     ("cartesian", 9, 65, 1022, 16, "serial, lanes past M"),
     ("polar", 4, 130, 512, 16, "chain"),
+    ("polar", 1, 1023, 2304, 16, "chain, 288 workgroups"),
+    ("real", 1, 1024, 4224, 16, "look-back, 264 chains"),
     ("real", 4, 130, 2048, 8, "chain"),
     ("real", 16, 129, 2048, 8, "serial"),
     ("polar", 1, 1100, 64, 16, "look-back"),
