@@ -2803,9 +2803,9 @@ struct SplitBwd {
 // launch, and up to kCoopKeepSteps it stays there: that form, and time pieces
 // for a caller that sets the one-launch form aside, is what the header has
 // promised for these shapes.  It costs time in bf16 (us, one launch against
-// split: 512 chains, T=512 276 and 242, T=1024 about 530 and 425; 640 chains
+// split: 512 chains, T=512 285 and 242, T=1024 556 and 425; 640 chains
 // 370 and 301, 705 and 553; 768 chains 378 and 341, 717 and 624); fp32 is
-// faster in one launch (512 chains, T=1024 657 and 804, 768 chains 723 and
+// faster in one launch (512 chains, T=1024 555 and 804, 768 chains 723 and
 // 1131).
 constexpr int64_t kCoopKeepSteps = 1024;
 constexpr int64_t kSplitSecondRound = 48, kSplitManySteps = 768;
