@@ -1,5 +1,5 @@
 """The backward with four chains per workgroup, which grids of about one wave
-per SIMD (961 to 1024 chains) take: the P1 scan and the module's one-launch
+per SIMD (961 to 1024 chains, the bf16 P1 scan without resets from 513) take: the P1 scan and the module's one-launch
 form, at a number of chains that leaves three waves of the last workgroup
 without one, with lanes past M."""
 import pytest
@@ -13,17 +13,18 @@ from test_gpu_split import _run
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T,dtype,extra", [
-    (70, BF16, dict(h0=True, dlast=True)),
-    (70, BF16, dict(h0=True, dlast=True, seg=True)),
-    (3, F32, dict(h0=True, dlast=True)),
-    (70, F32, dict(dlast=True, reset_first=True)),
-    (260, BF16, dict(dlast=True)),  # from 256 steps on fewer chains split their time
-], ids=["bf16", "resets_bf16", "short_f32", "reset_first_f32", "long_bf16"])
-def test_p1_backward_grouped(T, dtype, extra):
-    """969 = 17 x 57 chains of 128 modes against the general chain kernels
-    (tolerances as for the split chains)."""
-    B, M = 17, 57 * 128 - 4
+@pytest.mark.parametrize("B,T,dtype,extra", [
+    (17, 70, BF16, dict(h0=True, dlast=True)),
+    (17, 70, BF16, dict(h0=True, dlast=True, seg=True)),
+    (17, 3, F32, dict(h0=True, dlast=True)),
+    (17, 70, F32, dict(dlast=True, reset_first=True)),
+    (17, 260, BF16, dict(dlast=True)),  # from 256 steps on fewer chains split their time
+    (9, 70, BF16, dict(h0=True, dlast=True)),  # 513 chains: the fewest, without resets in bf16
+], ids=["bf16", "resets_bf16", "short_f32", "reset_first_f32", "long_bf16", "half_bf16"])
+def test_p1_backward_grouped(B, T, dtype, extra):
+    """969 = 17 x 57 and 513 = 9 x 57 chains of 128 modes against the general
+    chain kernels (tolerances as for the split chains)."""
+    M = 57 * 128 - 4
     print(f"[case] grouped P1 B={B} T={T} M={M} {dtype} {extra}", flush=True)
     case = make_case("p1", B, T, M, 1, dtype, seed=T, **extra)
     tol = 1e-5 if dtype == F32 else 2.0 ** -7
