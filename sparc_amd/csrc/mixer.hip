@@ -2779,7 +2779,10 @@ int split_waves(int64_t B, int64_t T, int64_t M, int32_t io, bool gw, bool reset
 //     316, 512 1150 -> 1016, 768 1736 -> 1520, 1024 2034 -> 2069
 //   relu output (recomputing, against the general kernels): T=2048: 96 345 ->
 //     279 or less (the host's time), 128 421 -> 278, 384 1100 -> 556, 2048
-//     (T=1024) 4200 -> 1460; 16 chains, T=4096 185 -> 298
+//     (T=1024) 4200 -> 1460; 16 chains, T=4096 185 -> 298; few chains (the
+//     look-back against split): 16 chains, T=256 32 -> 29, T=384 33 -> 37, T=768
+//     35 -> 58, 32 chains, T=384 38 -> 36, T=512 39 -> 44, 40 chains, T=768 56
+//     -> 59, 48 chains 70 -> 59
 // As in the forward, with few chains only short sequences are split, and with
 // many nothing below kSplitMinSteps is.  P1 scan:
 //   where the second round has workgroups for few of the 256 CUs
@@ -2810,6 +2813,7 @@ struct SplitBwd {
 constexpr int64_t kCoopKeepSteps = 1024;
 constexpr int64_t kSplitSecondRound = 48, kSplitManySteps = 768;
 constexpr int kReluBwdWaves = 8;  // 8 steps each: a round is a saved-state chunk
+constexpr int64_t kReluFewChains = 36, kReluFewSteps = 288;
 // mode: the chain mode, with kReset where there are reset steps.
 SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int mode, bool controls = false) {
   const int cm = mode & 3;
@@ -2818,7 +2822,7 @@ SplitBwd split_bwd(int64_t B, int64_t T, int64_t M, int32_t io, int mode, bool c
   const bool bf = io == SPARC_BF16, few = T >= 16 && T <= kSplitFewSteps;
   SplitBwd r;
   if (cm == kRelu) {
-    if (n >= 64 || few) r.waves = kReluBwdWaves;
+    if (n >= 64 || (few && (n >= kReluFewChains || T <= kReluFewSteps))) r.waves = kReluBwdWaves;
     return r;
   }
   r.V = bf ? 2 : 1;
