@@ -30,6 +30,9 @@ FEW = [  # few chains: T from 16 to 768 steps is split
     ("relu_f32", 2, 257, 132, F32, dict(relu=True, h0=True, dlast=True)),
     ("relu_resets_bf16", 2, 150, 256, BF16, dict(relu=True, seg=True)),
     ("longest_f32", 1, 768, 64, F32, dict(h0=True, dlast=True)),
+    ("relu_longest_f32", 2, 288, 132, F32, dict(relu=True, h0=True, dlast=True)),
+    ("relu_past_bf16", 2, 289, 132, BF16, dict(relu=True, dlast=True, seg=True)),  # the look-back's backward
+    ("relu_36_chains_f32", 3, 290, 1500, F32, dict(relu=True, dlast=True)),
 ]
 
 
